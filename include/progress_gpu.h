@@ -424,10 +424,9 @@ int prg_get_int8_moduli(void);
  * forced with the environment variable PRG_CRT_CONFIG.  0 before any int8
  * product.  Measurement support; no reference counterpart. */
 int prg_gpu_int8_waves(void);
-/* K slices of the FP64 SP2 step at size N: 1 for the fused one-kernel step
- * (sp2_step_kernel), s > 1 for the split product and its epilogue kernel
- * (fewer than 1024 upper-triangle 128 x 128 tiles).  Measurement support;
- * no reference counterpart. */
+/* K slices of the FP64 SP2 step at size N: 1, the step is one kernel
+ * (sp2_step_kernel) at every size.  Measurement support; no reference
+ * counterpart. */
 int prg_gpu_sp2_split_slices(int N);
 /* Forces the int8 CRT product kernel configuration (one of the codes above;
  * 0 returns to timing them per size).  Returns a status (1 for an unknown
@@ -448,8 +447,8 @@ int prg_gpu_sp2_alg2_device(int N, const double *dH, double *dRho, double bndfil
 /* prg_gpu_sp2_alg2_device in FP64 without any allocation: no counterpart in
  * the reference.  For callers that cannot allocate (code under HIP graph
  * capture, tight serving or MD loops, harnesses that forbid hipMalloc).  The
- * ping-pong X, partial sums, state and K-split accumulators live in a static
- * device array of 52.3 MiB held by every device the library runs on until
+ * ping-pong X, partial sums and state live in a static
+ * device array of 16.5 MiB held by every device the library runs on until
  * the process ends; N is limited to 1024 (larger N returns status 1, bad
  * argument).  prg_progress_init must have been called on the device (it
  * resolves the array's address; otherwise status 6, no device).  The array

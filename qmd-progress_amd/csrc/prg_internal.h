@@ -153,30 +153,26 @@ int reduce_partials(const double* d_part, int nblocks, int nq, double* d_out);
 // GEMM family (FP64 MFMA 16x16x4).
 // C = alpha * sum_p A_p B_p + beta * Cin + gamma * I ; npair in {1, 2}.
 // sym != 0: the product is symmetric; only upper-triangle tiles are computed
-// and mirrored (Cin must then be symmetric too).  d_part (optional) receives
-// per-tile [Tr(C), ||C||^2, <C, dotE>, 0].  C must not alias A_p or B_p.
+// and mirrored (Cin must then be symmetric too).  b_symmetric: every B_p is
+// symmetric (it is then read along its columns, as A is).  d_part (optional)
+// receives per-tile [Tr(C), ||C||^2, <C, dotE>, 0].  C must not alias A_p or
+// B_p.  Operands are zero outside their n x n blocks (C.n).
 int gemm(int npair, const DMat* A, const DMat* B, double alpha, double beta, const DMat* Cin,
-         double gamma, DMat C, int sym, double* d_part, int* ntiles,
-         const DMat* dotE = nullptr);
+         double gamma, DMat C, int sym, double* d_part, int* ntiles, const DMat* dotE,
+         bool b_symmetric);
+int gemm_tiles(int ld, int sym);  // records of partial sums it writes
 
-// Fused SP2 step: Y = X*X, then per the device state's planned branch
-// Xn = Y or 2X - Y; epilogue partials [||Xn||^2, Tr Xn, idem, Tr Y].  Below
-// 1024 upper-triangle tiles the product is split along K
-// (sp2_split_count(ld) slices) into split_acc (sp2_split_bytes(ld) bytes; the
-// library workspace when null) and summed in slice order by a second kernel.
-// thresholded: the sparse formats' thresholding of the state's threshold
-// (product and update in two kernels; split_acc then holds one slice per
-// tile at least).
-int sp2_step(const DMat& x0, const DMat& x1, Sp2State* d_state, double* d_part, int* ntiles,
-             double* split_acc = nullptr, bool thresholded = false);
-int sp2_split_count(int ld);
-// Workgroups per tile of the split product's epilogue (4, or 8 at small ld);
-// each writes one record of partial sums.
-int sp2_epilogue_parts(int ld);
-size_t sp2_split_bytes(int ld);
-// Fused response step: Y = X D + D X with the same branch: Dn = Y or 2D - Y.
-int sp2_response_step(const DMat& x0, const DMat& x1, const DMat& d0, const DMat& d1,
-                      Sp2State* d_state, double* d_part, int* ntiles);
+// Fused SP2 step in one launch: the previous step's sums are absorbed and the
+// next step planned (link; see prg_plan.h), Y = X*X, then per the planned
+// branch Xn = Y or 2X - Y; epilogue partials [||Xn||^2, Tr Xn, idem, Tr Y],
+// sp2_step_tiles(ld) records.  d0, d1 (or null): the response's ping-pong
+// pair, Y = X D + D X with the same branch: Dn = Y or 2D - Y.  thresholded:
+// the sparse formats' thresholding of the state's threshold.  cur: the buffer
+// that holds X (0: x0).
+struct Sp2Link;
+int sp2_step(const DMat& x0, const DMat& x1, const DMat* d0, const DMat* d1, const Sp2Link& link,
+             double* d_part, int* ntiles, bool thresholded, int cur);
+int sp2_step_tiles(int ld);
 // Device-side SP2 bookkeeping kernels.
 int sp2_init_state(Sp2State* d_state, const double* d_part, int nblocks);
 int sp2_absorb_plan(Sp2State* d_state, const double* d_part, int ntiles);

@@ -1,6 +1,7 @@
 // Host-side wrappers of the device matrix operations (see prg_ops.h).
 #include "prg_ops.h"
 
+#include <algorithm>
 #include <cstring>
 #include <string>
 
@@ -93,11 +94,13 @@ int fetch(const double* d_part, int nb, int nq, double* host) {
   return OK;
 }
 
-// Partials of one launch: 128 x 128 tiles of the FP64 kernels, 64 x 64
-// blocks of the int8 CRT epilogue, or the elementwise kernels' blocks.
+// Partials of one launch: tiles of the FP64 or split kernels, 64 x 64 blocks
+// of the int8 CRT epilogue, or the elementwise kernels' blocks.
 static double* part_buf(int ld, int* st) {
-  const int nb = ld / 64;
-  return (double*)workspace("ops_part", sizeof(double) * 4 * (size_t)(nb * nb + 2048), st);
+  const size_t nb = ld / 64;
+  const size_t records =
+      std::max({nb * nb, (size_t)gemm_tiles(ld, 0), (size_t)gemm_tiles(ld, 1)}) + 2048;
+  return (double*)workspace("ops_part", sizeof(double) * 4 * records, st);
 }
 
 int mm(const DMat& A, const DMat& B, DMat C, bool sym, double alpha, double beta,
@@ -115,7 +118,7 @@ int mm(const DMat& A, const DMat& B, DMat C, bool sym, double alpha, double beta
     g_products += 1;
     g_alg_flops += 2.0 * C.n * (double)C.n * C.n;
   } else {
-    if ((st = gemm(1, &A, &B, alpha, beta, Cin, gamma, C, sym ? 1 : 0, part, &nt, dotE)))
+    if ((st = gemm(1, &A, &B, alpha, beta, Cin, gamma, C, sym ? 1 : 0, part, &nt, dotE, sym)))
       return st;
     count_products(1, C, sym);
   }
@@ -131,7 +134,7 @@ int mm(const DMat& A, const DMat& B, DMat C, bool sym, double alpha, double beta
 
 int mm_symmetric_result(const DMat& A, const DMat& B, DMat C) {
   int nt = 0;
-  const int st = gemm(1, &A, &B, 1.0, 0.0, nullptr, 0.0, C, 1, nullptr, &nt, nullptr);
+  const int st = gemm(1, &A, &B, 1.0, 0.0, nullptr, 0.0, C, 1, nullptr, &nt, nullptr, false);
   if (!st) count_products(1, C, true);
   return st;
 }
@@ -143,7 +146,8 @@ int mm2(const DMat& A0, const DMat& B0, const DMat& A1, const DMat& B1, DMat C, 
   if (st) return st;
   const DMat A[2] = {A0, A1}, B[2] = {B0, B1};
   int nt = 0;
-  if ((st = gemm(2, A, B, alpha, beta, Cin, gamma, C, sym ? 1 : 0, part, &nt))) return st;
+  if ((st = gemm(2, A, B, alpha, beta, Cin, gamma, C, sym ? 1 : 0, part, &nt, nullptr, sym)))
+    return st;
   count_products(2, C, sym);
   if (sums) {
     double h[4];

@@ -1,13 +1,18 @@
 // Device-side FP64 bookkeeping of the SP2 loop: the branch decision for the
-// next step and the absorption of a step's partial sums, for the one-block
-// kernels that run them.  (A last-workgroup absorb inside the split epilogue
-// was slower: the device-scope fences it needs write back and invalidate the
-// per-XCD L2s, 10.8 us per step at N = 1024 against 4.6 us for this launch.)
+// next step and the absorption of a step's partial sums.  The mixed-precision
+// loops run them in a one-block kernel after each step.  The FP64 loop runs
+// them at the start of the next step's launch, in every workgroup, on an LDS
+// copy of the state header: the launch and its gap (4.5 + 1 us per step) give
+// way to about 2 us of reads that a workgroup needs anyway.  (A last-workgroup
+// absorb at the end of the step was slower than a launch of its own: the
+// device-scope fences it needs write back and invalidate the per-XCD L2s.)
 #pragma once
 
 #include "prg_internal.h"
+#include "prg_tile.h"
 
 #include <cmath>
+#include <cstddef>
 
 namespace prg {
 
@@ -16,7 +21,9 @@ namespace prg {
 // :469-513, alg1 :801-849, alg1_genseq :941-982, basic :89-119, replay
 // variants :581-600 / :1060-1072 / :1288-1300, and the response loop of
 // src/prg_response_mod.F90:730-770.
-__device__ inline void sp2_plan(Sp2State* s) {
+// pp: the branch log (pp[] of the state, or of the state the header was
+// copied from).
+__device__ inline void sp2_plan(Sp2State* s, const int* pp) {
   s->planned = 0;
   s->apply = 0;
   s->last = 0;
@@ -42,7 +49,7 @@ __device__ inline void sp2_plan(Sp2State* s) {
         // falling quadratically (numerical noise floor)
         const double e = trx - trx2;
         const int it0 = s->iter;  // 0-based index of the step being planned
-        const bool alt = it0 > 2 && s->pp[it0 - 1] != s->pp[it0 - 2];
+        const bool alt = it0 > 2 && pp[it0 - 1] != pp[it0 - 2];
         s->ie2 = s->ie1;
         s->ie1 = s->ie0;
         s->ie0 = e;
@@ -152,7 +159,7 @@ __device__ inline void sp2_plan(Sp2State* s) {
     case V_SEQ_ALG1:
     case V_SUBMATRIX: {
       if (s->iter >= s->icount) { s->done = 1; return; }
-      s->sigma = s->pp[s->iter] != 0;
+      s->sigma = pp[s->iter] != 0;
       s->trx_next = s->sigma ? s->fro2 : 2.0 * s->trx_fresh - s->fro2;
       s->apply = 1;
       s->planned = 1;
@@ -199,29 +206,27 @@ __device__ inline void block_sum4(const double* part, int nb, double* out /*shar
   __syncthreads();
 }
 
-// Absorb the partials of the product just computed (ntiles records of 4),
-// then plan the next step.  Called by every thread of one BT-thread block of
-// a launch whose step was planned.
-template <int BT>
-__device__ inline void sp2_absorb_plan_block(Sp2State* s, const double* part, int ntiles) {
-  __shared__ double sums[4];
-  block_sum4<BT>(part, ntiles, sums);
-  if (threadIdx.x != 0) return;
+// Absorb the sums of the product just computed, then plan the next step (one
+// thread).  pp, vv: the logs; written only if `log` (one workgroup of a
+// launch that plans in all of them).
+__device__ inline void sp2_absorb_sums(Sp2State* s, const double* sums, int* pp, double* vv,
+                                       bool log) {
   const double fro2 = sums[0], trf = sums[1], idem = sums[2];
   s->x2_trace = sums[3];
   const int v = s->variant;
   const int k = s->iter + 1;
   const int idx = k - 1;
-  if (v == V_ALG2_GENSEQ || v == V_ALG1_GENSEQ || v == V_SEQ_ALG2 || v == V_SEQ_ALG1) {
-    if (idx < kMaxIter) s->vv[idx] = sqrt(idem);
-  } else if (v == V_SUBMATRIX) {
-    if (idx < kMaxIter) s->vv[idx] += idem;
+  if (log && idx < kMaxIter) {
+    if (v == V_ALG2_GENSEQ || v == V_ALG1_GENSEQ || v == V_SEQ_ALG2 || v == V_SEQ_ALG1)
+      vv[idx] = sqrt(idem);
+    else if (v == V_SUBMATRIX)
+      vv[idx] += idem;
   }
   double trx_old = (v == V_ALG2_GENSEQ) ? s->trx_fresh : s->trx;
   if (v == V_BASIC || v == V_BASIC_FIXED) trx_old = s->trx_fresh;
   if (s->apply) {
-    if (v != V_SEQ_ALG2 && v != V_SEQ_ALG1 && v != V_SUBMATRIX && idx < kMaxIter)
-      s->pp[idx] = s->sigma;
+    if (log && v != V_SEQ_ALG2 && v != V_SEQ_ALG1 && v != V_SUBMATRIX && idx < kMaxIter)
+      pp[idx] = s->sigma;
     s->iter = k;
     s->cur ^= 1;
     s->fro2 = fro2;
@@ -239,7 +244,88 @@ __device__ inline void sp2_absorb_plan_block(Sp2State* s, const double* part, in
   s->e0 = e_new;
   if (s->refine_phase && s->apply) s->refine_steps += 1;
   if (s->last) s->done = 1;
-  sp2_plan(s);
+  sp2_plan(s, pp);
+}
+
+// The same from ntiles records of 4 partials.  Called by every thread of one
+// BT-thread block of a launch whose step was planned.
+template <int BT>
+__device__ inline void sp2_absorb_plan_block(Sp2State* s, const double* part, int ntiles) {
+  __shared__ double sums[4];
+  block_sum4<BT>(part, ntiles, sums);
+  if (threadIdx.x == 0) sp2_absorb_sums(s, sums, s->pp, s->vv, true);
+}
+
+// What an FP64 step launch reads first: the state header as the previous
+// launch left it and the partial sums of the step that launch ran.  Every
+// workgroup absorbs them into its own copy (the same operations in the same
+// order everywhere) and workgroup 0 stores that copy as the next header, in
+// the other slot, so that no workgroup reads what another writes.
+struct Sp2Link {
+  const Sp2State* in;
+  Sp2State* out;       // null: the header is already planned and stays as it is
+  int* pp;             // logs, in the first slot
+  double* vv;
+  const double* part;  // null: nothing to absorb (first step)
+  int nparts;
+};
+
+constexpr int kSp2HeadBytes = (int)offsetof(Sp2State, pp);
+
+// The reads of a link, issued before anything waits for them (wave 0 of the
+// workgroup; every thread learns `planned`, the header's flag before the
+// absorption: 0 when the loop had ended).
+struct Sp2LinkReads {
+  static constexpr int kRecords = 4;  // per lane: 256 workgroups' sums
+  uint32_t word;
+  double2 lo[kRecords], hi[kRecords];
+  int planned;
+};
+
+__device__ __forceinline__ void sp2_link_read(const Sp2Link& l, Sp2LinkReads& r) {
+  static_assert(kSp2HeadBytes % 4 == 0 && kSp2HeadBytes / 4 <= 64, "one header word per lane");
+  r.planned = l.in->planned;
+  if (threadIdx.x >= 64) return;
+  if (threadIdx.x < kSp2HeadBytes / 4) r.word = ((const uint32_t*)l.in)[threadIdx.x];
+#pragma unroll
+  for (int i = 0; i < Sp2LinkReads::kRecords; ++i) {
+    const int b = threadIdx.x + 64 * i;
+    r.lo[i] = r.hi[i] = double2{0.0, 0.0};
+    if (l.part && b < l.nparts) {
+      r.lo[i] = *(const double2*)(l.part + 4 * (size_t)b);
+      r.hi[i] = *(const double2*)(l.part + 4 * (size_t)b + 2);
+    }
+  }
+}
+
+// Wave 0 leaves the planned header in `head` (LDS, kSp2HeadBytes; the other
+// waves see it after the next barrier), workgroup 0's also in the other slot.
+__device__ __forceinline__ void sp2_link(const Sp2Link& l, Sp2LinkReads& r, char* head) {
+  if (threadIdx.x >= 64) return;
+  constexpr int words = kSp2HeadBytes / 4;
+  if (threadIdx.x < words) ((uint32_t*)head)[threadIdx.x] = r.word;
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  if (l.part && r.planned) {
+    double a[4] = {0.0, 0.0, 0.0, 0.0};
+    auto add = [&](double2 lo, double2 hi) {
+      a[0] += lo.x;
+      a[1] += lo.y;
+      a[2] += hi.x;
+      a[3] += hi.y;
+    };
+#pragma unroll
+    for (int i = 0; i < Sp2LinkReads::kRecords; ++i) add(r.lo[i], r.hi[i]);
+#pragma unroll 4
+    for (int b = threadIdx.x + 64 * Sp2LinkReads::kRecords; b < l.nparts; b += 64)
+      add(*(const double2*)(l.part + 4 * (size_t)b), *(const double2*)(l.part + 4 * (size_t)b + 2));
+    tile::wave_sum4(a);
+    if (threadIdx.x == 0) sp2_absorb_sums((Sp2State*)head, a, l.pp, l.vv, blockIdx.x == 0);
+  }
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  if (l.out && blockIdx.x == 0 && threadIdx.x < words)
+    ((uint32_t*)l.out)[threadIdx.x] = ((const volatile uint32_t*)head)[threadIdx.x];
 }
 
 }  // namespace prg

@@ -1,14 +1,16 @@
 // SP2 purification drivers (src/prg_sp2_mod.F90) on one GPU.
 //
-// The whole iteration runs on the device: one fused product-and-update launch
-// (two for the K-split product of small matrices) and one single-workgroup
-// bookkeeping launch per step, enqueued in chunks.  The host reads the state
+// The whole iteration runs on the device: in FP64 one launch per step (the
+// bookkeeping of the step before, the product and the update), in the
+// mixed-precision modes a product, an update and a single-workgroup
+// bookkeeping launch, enqueued in chunks.  The host reads the state
 // header of a chunk (an asynchronous copy into pinned memory) only after the
 // next chunk is enqueued, so no scalar crosses PCIe per iteration and the
 // device does not wait for the host.  Once the loop has stopped, the
-// launches still queued exit at their first instruction.
+// launches still queued exit after reading the state.
 #include "prg_sp2.h"
 #include "prg_ops.h"
+#include "prg_plan.h"
 
 #include <algorithm>
 #include <cmath>
@@ -24,29 +26,24 @@ namespace prg {
 namespace {
 // Static device scratch of the no-allocation SP2 entry point
 // (prg_gpu_sp2_alg2_device_noalloc, FP64, N <= 1024): the ping-pong X, the
-// K-split accumulators, the partial sums, the bounds, the state and the
-// Gershgorin scratch, each at a 256-byte aligned offset.  Every device the
+// partial sums, the bounds, the two state slots and the Gershgorin scratch, each at a 256-byte aligned offset.  Every device the
 // library runs on holds its own copy for the life of the process; calls that
 // overlap on one device share it and race.
 constexpr int kNoallocMaxLd = 1024;
 constexpr size_t kMatBytes = sizeof(double) * (size_t)kNoallocMaxLd * kNoallocMaxLd;
-// K-split accumulators: room for 288 partial 128 x 128 tiles (36 MiB), at
-// least what the split rule asks for with ld <= 1024; checked per call
-constexpr size_t kSplitBytes = sizeof(double) * 36 * 8 * 128 * 128;
-constexpr size_t kPartBytes = 128 * 1024;
+constexpr size_t kPartBytes = 160 * 1024;
 constexpr size_t kBoundsBytes = 256;
 constexpr size_t kStateBytes = 16 * 1024;
 constexpr size_t kGershBytes = 160 * 1024;
 constexpr size_t kOffX0 = 0;
 constexpr size_t kOffX1 = kOffX0 + kMatBytes;
-constexpr size_t kOffSplit = kOffX1 + kMatBytes;
-constexpr size_t kOffPart = kOffSplit + kSplitBytes;
+constexpr size_t kOffPart = kOffX1 + kMatBytes;
 constexpr size_t kOffBounds = kOffPart + kPartBytes;
 constexpr size_t kOffState = kOffBounds + kBoundsBytes;
 constexpr size_t kOffGersh = kOffState + kStateBytes;
-constexpr size_t kScratchBytes = kOffGersh + kGershBytes;  // 52.3 MiB
-static_assert(sizeof(Sp2State) <= kStateBytes, "state slot too small");
-static_assert(kOffSplit % 256 == 0 && kOffPart % 256 == 0 && kOffState % 256 == 0 &&
+constexpr size_t kScratchBytes = kOffGersh + kGershBytes;  // 16.5 MiB
+static_assert(2 * sizeof(Sp2State) <= kStateBytes, "state slot too small");
+static_assert(kOffPart % 256 == 0 && kOffState % 256 == 0 &&
                   kOffGersh % 256 == 0,
               "scratch offsets must stay 256-byte aligned");
 
@@ -56,7 +53,7 @@ __device__ __align__(256) char scratch[kScratchBytes];
 // array's name), and the host state images of the no-allocation loop.
 constexpr int kMaxDevices = 64;
 char* g_scratch_ptr[kMaxDevices] = {};
-Sp2State g_noalloc_host[3];
+Sp2State g_noalloc_host[5];
 
 int g_precision = PRG_PREC_FP64;
 
@@ -115,6 +112,18 @@ int noalloc_setup() {
   return OK;
 }
 
+namespace {
+// Doubles of one set of partial sums: a record per product tile (the int8 CRT
+// update writes one per 64 x 64 block) or the normalisation's.  The FP64 loop
+// alternates between two sets: a step's workgroups read the last step's while
+// others already write theirs.
+size_t part_doubles(int ld) {
+  const int nt = ld / kTile;
+  const int nslots = std::max({nt * (nt + 1) / 2, sp2_step_tiles(ld), crt_update_blocks(ld)});
+  return 4 * (size_t)(nslots + 2048);
+}
+}  // namespace
+
 int precision_mode() { return g_precision; }
 void set_precision_mode(int m) { g_precision = m; }
 
@@ -130,8 +139,6 @@ int run_sp2(const DMat& H, const Sp2Params& p_in, DMat out, Sp2Result* res, cons
     set_error(ERR_ARG, "run_sp2: bad matrix layout");
     return ERR_ARG;
   }
-  const int nt = ld / kTile;
-  const int ntiles = nt * (nt + 1) / 2;
   const size_t mat_bytes = sizeof(double) * (size_t)ld * ld;
   if (bufs && (H1 || p.variant == V_RESPONSE || p.precision != PRG_PREC_FP64)) {
     set_error(ERR_ARG, "run_sp2: caller buffers serve FP64 solves without response only");
@@ -149,18 +156,15 @@ int run_sp2(const DMat& H, const Sp2Params& p_in, DMat out, Sp2Result* res, cons
   } else {
     x0 = (double*)workspace("sp2_x0", mat_bytes, &st);
     x1 = (double*)workspace("sp2_x1", mat_bytes, &st);
-    // partial sums: one slot per product tile (the int8 CRT update writes one
-    // per 64 x 64 block) plus the normalisation's
-    // (the K-split epilogue writes four or eight per tile)
-    const int nslots = std::max(8 * ntiles, crt_update_blocks(ld));
-    part = (double*)workspace("sp2_part", sizeof(double) * 4 * (size_t)(nslots + 2048), &st);
+    part = (double*)workspace("sp2_part", sizeof(double) * 2 * part_doubles(ld), &st);
     bounds = (double*)workspace("sp2_bounds", sizeof(double) * 4, &st);
-    dst = (Sp2State*)workspace("sp2_state", sizeof(Sp2State), &st);
-    // pinned host memory: the state image, then two header slots that the
-    // pipelined loop below reads back alternately
-    hst = (Sp2State*)host_staging(3 * sizeof(Sp2State), &st);
+    dst = (Sp2State*)workspace("sp2_state", 2 * sizeof(Sp2State), &st);
+    // pinned host memory: the state image, two header slots that the
+    // pipelined loop below reads back alternately, and the final state slots
+    hst = (Sp2State*)host_staging(5 * sizeof(Sp2State), &st);
   }
   if (st) return st;
+  double* part2[2] = {part, part + part_doubles(ld)};
   DMat X0{n, ld, x0}, X1{n, ld, x1};
   const bool response = (p.variant == V_RESPONSE);
   DMat D0{n, ld, nullptr}, D1{n, ld, nullptr};
@@ -240,9 +244,9 @@ int run_sp2(const DMat& H, const Sp2Params& p_in, DMat out, Sp2Result* res, cons
   int prec = p.precision;
   const bool timing = g_timing && !bufs;
   if (timing) crt_timing_begin();
-  if (timing && (int)g_events.size() < 2 * (maxsteps + 1)) {
+  if (timing && (int)g_events.size() < 2 * (maxsteps + 2)) {
     const size_t old = g_events.size();
-    g_events.resize(2 * (maxsteps + 1));
+    g_events.resize(2 * (maxsteps + 2));
     for (size_t e = old; e < g_events.size(); ++e) PRG_HIP_CHECK(hipEventCreate(&g_events[e]));
   }
   if (!bufs && !g_head_ev[0]) {
@@ -255,18 +259,31 @@ int run_sp2(const DMat& H, const Sp2Params& p_in, DMat out, Sp2Result* res, cons
   // launches still queued exit at their first instruction.  Chunk lengths
   // follow the iteration count of the last solve of the same shape (one long
   // chunk, then short ones), otherwise 16 steps (8 from n = 4096).
+  //
+  // FP64 (link) steps: launch L reads state slot L & 1 and the sums of launch
+  // L - 1, and leaves the planned state in the other slot, so a solve of k
+  // products takes k + 1 launches (the last one only absorbs) and the final
+  // state is in slot L & 1.
   const ShapeKey key{n, p.variant, p.precision};
   const int expect = (replay || bufs) ? 0 : expected_iterations(key);
+  // (Above 1280 tiles a step is long and every workgroup would read every
+  // record: a bookkeeping launch per step instead, as in the other modes.)
+  const bool fp64 = (p.precision == PRG_PREC_FP64) || response;
+  const bool linked = fp64 && sp2_step_tiles(ld) <= 1280;
+  int launches = 0;
+  const Sp2State* last_head = hst;  // the last header read back
+  int polish_cur = 0;               // the buffer that holds X when polishing begins
   Sp2State* slot[2] = {hst + 1, hst + 2};
   int phase0_steps = 0;
   for (int phase = 0; phase < 2; ++phase) {
     int steps = 0;
-    int phase_steps = maxsteps;
+    int phase_steps = maxsteps + (linked ? 1 : 0);
     if (phase == 1) {
       // FP64 polishing steps after a low-precision loop
       if (!hst->noise_stop || hst->refine_max <= 0) break;
       prec = PRG_PREC_FP64;
       if ((st = sp2_begin_refine(dst))) return st;
+      polish_cur = last_head->cur;
       phase_steps = hst->refine_max + 1;
     }
     int chunk_no = 0;
@@ -275,21 +292,31 @@ int run_sp2(const DMat& H, const Sp2Params& p_in, DMat out, Sp2Result* res, cons
     while (steps < phase_steps && !done) {
       int len;
       if (phase == 0 && replay)
-        len = maxsteps;
+        len = phase_steps;
       else if (phase == 0 && expect > 0)
-        len = (chunk_no == 0) ? std::max(1, expect - 2) : 4;
+        len = (chunk_no == 0) ? std::max(1, linked ? expect + 1 : expect - 2) : 4;
       else
         len = n >= 4096 ? 8 : 16;
       for (int c = 0; c < len && steps < phase_steps; ++c, ++steps) {
         int nt_used = 0;
         const bool timed = timing && phase == 0;
         if (timed) PRG_HIP_CHECK(hipEventRecord(g_events[2 * steps], stream()));
-        if (response) {
-          if ((st = sp2_response_step(X0, X1, D0, D1, dst, part, &nt_used))) return st;
-        }
-        if (prec == PRG_PREC_FP64 || response) {
-          st = sp2_step(X0, X1, dst, part, &nt_used, bufs ? bufs->split_acc : nullptr,
-                        p.threshold > 0.0);
+        if (linked) {
+          Sp2Link link;
+          link.in = dst + (launches & 1);
+          link.out = dst + (~launches & 1);
+          link.pp = dst->pp;
+          link.vv = dst->vv;
+          link.part = launches ? part2[~launches & 1] : nullptr;
+          link.nparts = sp2_step_tiles(ld);
+          st = sp2_step(X0, X1, response ? &D0 : nullptr, response ? &D1 : nullptr, link,
+                        part2[launches & 1], &nt_used, p.threshold > 0.0, launches & 1);
+          ++launches;
+        } else if (prec == PRG_PREC_FP64) {
+          // planned by the bookkeeping launch below
+          st = sp2_step(X0, X1, response ? &D0 : nullptr, response ? &D1 : nullptr,
+                        Sp2Link{dst, nullptr, dst->pp, dst->vv, nullptr, 0}, part, &nt_used,
+                        p.threshold > 0.0, (polish_cur + steps) & 1);
         } else if (prec == PRG_PREC_F16SPLIT || prec == PRG_PREC_BF16SPLIT ||
                    prec == PRG_PREC_INT8CRT) {
           st = sp2_step_mixed(X0, X1, dst, part, &nt_used, prec);
@@ -299,21 +326,33 @@ int run_sp2(const DMat& H, const Sp2Params& p_in, DMat out, Sp2Result* res, cons
         }
         if (st) return st;
         if (timed) PRG_HIP_CHECK(hipEventRecord(g_events[2 * steps + 1], stream()));
-        if ((st = sp2_absorb_plan(dst, part, nt_used))) return st;
+        if (!linked && (st = sp2_absorb_plan(dst, part, nt_used))) return st;
       }
+      Sp2State* cur_state = dst + (linked ? (launches & 1) : 0);
       const int sl = chunk_no & 1;
-      PRG_HIP_CHECK(hipMemcpyAsync(slot[sl], dst, head, hipMemcpyDeviceToHost, stream()));
+      PRG_HIP_CHECK(hipMemcpyAsync(slot[sl], cur_state, head, hipMemcpyDeviceToHost, stream()));
       if (bufs) {
         // caller buffers: a plain synchronous read-back, no events
         PRG_HIP_CHECK(hipStreamSynchronize(stream()));
         done = slot[sl]->done != 0;
+        last_head = slot[sl];
         ++chunk_no;
         continue;
       }
       PRG_HIP_CHECK(hipEventRecord(g_head_ev[sl], stream()));
+      if (linked && phase == 0 && expect > 0 && chunk_no == 0) {
+        // as many launches as the last solve of this shape took: most likely
+        // all of them, so the next chunk waits for the answer
+        PRG_HIP_CHECK(hipEventSynchronize(g_head_ev[sl]));
+        done = slot[sl]->done != 0;
+        last_head = slot[sl];
+        ++chunk_no;
+        continue;
+      }
       if (waiting) {
         PRG_HIP_CHECK(hipEventSynchronize(g_head_ev[sl ^ 1]));
         done = slot[sl ^ 1]->done != 0;
+        last_head = slot[sl ^ 1];
       }
       waiting = true;
       ++chunk_no;
@@ -322,22 +361,29 @@ int run_sp2(const DMat& H, const Sp2Params& p_in, DMat out, Sp2Result* res, cons
       // the last chunk's header
       PRG_HIP_CHECK(hipEventSynchronize(g_head_ev[(chunk_no - 1) & 1]));
       done = slot[(chunk_no - 1) & 1]->done != 0;
+      last_head = slot[(chunk_no - 1) & 1];
     }
     if (phase == 0) phase0_steps = steps;
   }
   // the int8 CRT update keeps X in its residue planes (or the lower
   // triangle of an FP64 master at 12 or more moduli) between steps
+  const int final_slot = linked ? (launches & 1) : 0;
+  const Sp2State* fin = dst + final_slot;
   if (p.precision == PRG_PREC_INT8CRT && !response) {
-    if ((st = crt_finish(X0, X1, dst, 2.0, out, crt_moduli()))) return st;
-  } else if ((st = sp2_finish(X0, X1, dst, 2.0, out))) {
+    if ((st = crt_finish(X0, X1, fin, 2.0, out, crt_moduli()))) return st;
+  } else if ((st = sp2_finish(X0, X1, fin, 2.0, out))) {
     return st;
   }
   if (response && out1) {
     // rho1 = 2 Delta, Delta in the ping-pong slot named by the state
-    if ((st = sp2_finish(D0, D1, dst, 2.0, *out1))) return st;
+    if ((st = sp2_finish(D0, D1, fin, 2.0, *out1))) return st;
   }
-  PRG_HIP_CHECK(hipMemcpyAsync(hst, dst, sizeof(Sp2State), hipMemcpyDeviceToHost, stream()));
+  // the header of the final slot, the logs of the first
+  PRG_HIP_CHECK(hipMemcpyAsync(hst + 3, dst, (1 + final_slot) * sizeof(Sp2State),
+                               hipMemcpyDeviceToHost, stream()));
   PRG_HIP_CHECK(hipStreamSynchronize(stream()));
+  std::memcpy(hst, hst + 3, sizeof(Sp2State));
+  std::memcpy(hst, hst + 3 + final_slot, head);
   if (!replay && !bufs) record_iterations(key, hst->iter);
   if (!hst->done) {
     set_error(ERR_NOT_CONVERGED, "SP2 loop did not finish within the step budget");
@@ -497,7 +543,7 @@ int prg_set_int8_moduli(int count) {
 }
 int prg_get_int8_moduli(void) { return crt_moduli(); }
 int prg_gpu_int8_waves(void) { return crt_last_waves(); }
-int prg_gpu_sp2_split_slices(int N) { return N > 0 ? sp2_split_count(padded(N)) : 0; }
+int prg_gpu_sp2_split_slices(int N) { return N > 0 ? 1 : 0; }
 int prg_gpu_set_int8_config(int config) {
   clear_error();
   return set_crt_config(config);
@@ -730,14 +776,14 @@ int prg_gpu_sp2_alg2_device_noalloc(int N, const double* dH, double* dRho, doubl
   int dev = 0;
   PRG_HIP_CHECK(hipGetDevice(&dev));
   char* base = g_scratch_ptr[dev];
-  if (sp2_split_bytes(ld) > kSplitBytes || gershgorin_scratch_doubles(N) * 8 > kGershBytes) {
+  if (2 * sizeof(double) * part_doubles(ld) > kPartBytes ||
+      gershgorin_scratch_doubles(N) * 8 > kGershBytes) {
     set_error(ERR_ARG, "prg_gpu_sp2_alg2_device_noalloc: scratch layout too small");
     return ERR_ARG;
   }
   Sp2Buffers b;
   b.x0 = (double*)(base + kOffX0);
   b.x1 = (double*)(base + kOffX1);
-  b.split_acc = (double*)(base + kOffSplit);
   b.part = (double*)(base + kOffPart);
   b.bounds = (double*)(base + kOffBounds);
   b.state = (Sp2State*)(base + kOffState);

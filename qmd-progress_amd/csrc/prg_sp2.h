@@ -40,8 +40,8 @@ struct Sp2Result {
 
 // Buffers a caller hands to run_sp2 instead of the library workspace (the
 // no-allocation entry point): device memory for the ping-pong X, the partial
-// sums, the bounds, the state, the K-split accumulators and the Gershgorin
-// scratch, and three host state images.  With them the loop reads the state
+// sums (two sets), the bounds, the state (two slots) and the Gershgorin
+// scratch, and five host state images.  With them the loop reads the state
 // header back synchronously (no events) and keeps no per-shape history.
 struct Sp2Buffers {
   double* x0;
@@ -49,7 +49,6 @@ struct Sp2Buffers {
   double* part;
   double* bounds;
   Sp2State* state;
-  double* split_acc;
   double* gersh;
   Sp2State* host;
 };

@@ -1,0 +1,106 @@
+"""The FP64 MFMA tiles (products and SP2 steps) at the sizes where their edges
+and dispatch can go wrong: single chunks of K, sizes that are not multiples of
+the tile, the last row pairs, and both sides of each change of the tile edge
+(16, 32, 48) and of the bookkeeping (inside the step or in its own launch).
+
+Products against numpy in float64: each entry is a sum of n terms in another
+order, so it may differ by n eps sum_k |a_ik b_kj| (twice that is allowed)."""
+import numpy as np
+import pytest
+
+import progress_oracle as O
+
+pytestmark = pytest.mark.gpu
+
+SIZES = [1, 2, 15, 17, 33, 47, 100, 129, 352, 385, 500, 640, 701, 1000, 1153, 1500, 2305]
+
+
+@pytest.fixture(scope="module")
+def P():
+    import progress_amd
+    progress_amd.set_precision(progress_amd.PREC_FP64)
+    return progress_amd
+
+
+@pytest.mark.parametrize("n", SIZES)
+def test_symmetric_product(P, n):
+    """A B for commuting symmetric A, B (polynomials of one matrix)."""
+    import torch
+    rng = np.random.default_rng(n)
+    x = rng.standard_normal((n, n)) / np.sqrt(n)
+    a = 0.5 * (x + x.T)
+    b = a @ a + 0.3 * a
+    b = 0.5 * (b + b.T)
+    ld = P.padded_ld(n)
+    pad = torch.zeros((3, ld, ld), dtype=torch.float64, device="cuda")
+    pad[0, :n, :n] = torch.from_numpy(a)
+    pad[1, :n, :n] = torch.from_numpy(b)
+    pad[2] = 7.0  # the product overwrites all of it
+    torch.cuda.synchronize()
+    P.symmetric_product_device(pad[0], pad[1], pad[2], n)
+    c = pad[2].cpu().numpy()
+    bound = 2 * n * np.finfo(float).eps * (np.abs(a) @ np.abs(b)) + 1e-300
+    # the lower triangle is the upper one mirrored: it may differ by the
+    # asymmetry that b's own rounding leaves in the exact product
+    exact = a @ b
+    skew = np.abs(exact - exact.T)
+    assert np.all(np.abs(c[:n, :n] - exact) <= bound + bound.T + skew)
+    assert np.array_equal(c, c.T)
+    assert not c[n:].any() and not c[:, n:].any()
+
+
+@pytest.mark.parametrize("n", [17, 130, 500, 900, 1400])
+def test_general_products(P, n):
+    """Z^T A Z: products of operands that are not symmetric."""
+    rng = np.random.default_rng(n)
+    a, z = rng.standard_normal((n, n)), rng.standard_normal((n, n))
+    out = P.orthogonalize(a, z)
+    ref = z.T @ a @ z
+    absref = np.abs(z.T) @ (np.abs(a) @ np.abs(z))
+    assert np.all(np.abs(out - ref) <= 4 * n * np.finfo(float).eps * absref)
+
+
+@pytest.mark.parametrize("n", [1, 2, 17, 48, 129, 352, 385, 639, 700, 1153, 1409, 2320])
+def test_replayed_steps(P, n):
+    """A replayed branch sequence equals the same steps in numpy: x <- x^2 or
+    2x - x^2 keeps [0, 1], so each step adds at most n eps to an entry and at
+    most doubles what the steps before left."""
+    import torch
+    rng = np.random.default_rng(n)
+    x = rng.standard_normal((n, n)) / np.sqrt(n)
+    h = 0.5 * (x + x.T)
+    lo, hi = -3.0, 3.0
+    pp = [1, 0, 0, 1, 1]
+    ld = P.padded_ld(n)
+    dh = torch.zeros((ld, ld), dtype=torch.float64, device="cuda")
+    dh[:n, :n] = torch.from_numpy(h)
+    rho = torch.zeros_like(dh)
+    P.sp2_seq_device(dh, rho, n, pp, lo, hi)
+    x = (hi * np.eye(n) - h) / (hi - lo)
+    for s in pp:
+        x = x @ x if s else 2 * x - x @ x
+    r = rho[:n, :n].cpu().numpy()
+    assert np.max(np.abs(r - 2 * x)) <= 2 * 2 ** len(pp) * n * np.finfo(float).eps
+    assert np.array_equal(r, r.T)
+
+
+@pytest.mark.parametrize("n", [30, 400, 1201])
+def test_response_steps(P, n):
+    """Density and response of a gapped Hamiltonian against the oracle's
+    recursion (the same branches; the response is of order 1 / gap)."""
+    rng = np.random.default_rng(n)
+    q = np.linalg.qr(rng.standard_normal((n, n)))[0]
+    e = np.concatenate([rng.uniform(-3, -1, n // 2), rng.uniform(1, 3, n - n // 2)])
+    h = (q * e) @ q.T
+    h = 0.5 * (h + h.T)
+    h1 = rng.standard_normal((n, n)) / np.sqrt(n)
+    h1 = 0.5 * (h1 + h1.T)
+    rho, rsp = P.compute_response_sp2(h, h1, (n // 2) / n, 1, 100, "Abs", 1e-10)
+    c, v = q[:, :n // 2], q[:, n // 2:]
+    # Rayleigh-Schroedinger: sum over occupied-virtual pairs
+    u = (c.T @ h1 @ v) / (e[:n // 2, None] - e[None, n // 2:])
+    ref = 2 * (c @ u @ v.T)
+    ref = ref + ref.T
+    assert np.linalg.norm(rho - 2 * c @ c.T) < 1e-9
+    assert np.linalg.norm(rsp - ref) < 1e-7 * np.linalg.norm(ref)
+    assert np.array_equal(rsp, rsp.T)
