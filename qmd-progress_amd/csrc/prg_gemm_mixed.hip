@@ -15,16 +15,17 @@
 // v_mfma_f32_16x16x32_bf16.
 //
 // Because the planes are symmetric, the A operand (rows of the I panel) and
-// the B operand (columns of the J panel) are both read as contiguous column
-// chunks of a plane.
+// the B operand (columns of the J panel) are both read as contiguous slabs of
+// a plane.
 #include "prg_sp2.h"
+#include "prg_lds_dma.h"
 #include "prg_tile.h"
 
 namespace prg {
 namespace {
 
-using tile::block_store_partials;
-using tile::sym_tile;
+using tile::block_store4;
+using tile::sym_tile_banded;
 using tile::xcd_remap;
 
 typedef float f4 __attribute__((ext_vector_type(4)));
@@ -51,162 +52,281 @@ struct Split<__bf16> {
   }
 };
 
-constexpr int BM = 128, BK = 64, NT = 256;
-constexpr int HROW = BK + 8;  // padded LDS row (halves): 144 bytes
+constexpr int BM = 128, NT = 256;
+constexpr int KB = 32;                 // halves of K per slab and per plane block
+constexpr int kPanel = BM * KB * 2;    // bytes of one operand plane's slab
+constexpr int kSlab = 4 * kPanel;      // A hi, A lo, B hi, B lo
+constexpr int kRing = 2 * kSlab;       // two slabs: 64 KB, two workgroups per CU
 
-struct F16Args {
-  const double* buf[2];         // FP64 master ping-pong
-  const void* hi[2];            // hi planes ping-pong (T)
-  const void* lo[2];            // lo planes ping-pong (T)
-  int ld;
-  Sp2State* st;
-  double* part;
-};
+// Planes are stored in blocks of 32 columns, element (r, k) at
+// (k / 32) 32 ld + 32 r + k % 32: the 128 rows of a slab are 8 KB in one piece.
+__device__ __forceinline__ size_t plane_at(int r, int k, int ld) {
+  return (size_t)(k >> 5) * KB * ld + (size_t)r * KB + (k & 31);
+}
 
+// One 128 x 128 tile of A B (both symmetric, by their planes) over the whole
+// K: four waves in a 2 x 2 grid of 64 x 64.  The slabs are copied global ->
+// LDS directly (dma16), the next one while this one is multiplied; a slab is
+// 32 chunks of 16 rows x 64 bytes, wave w copies chunks w + 4 q.  Within a
+// row the 16-byte chunk g sits in slot g ^ ((row >> 1) & 3), which keeps the
+// fragment reads of 8 consecutive rows on distinct banks.  Two workgroups
+// share a CU: one multiplies while the other waits for its slab and reads its
+// fragments.
+//
+// Bound: the operand stream from L2, 32 KB per slab of 3 x 128 x 128 x 32
+// products (42 B/clk per CU at the 16-bit peak).  Registers: 128 for the two
+// accumulator sets, 64 for a slab's fragments.
 template <typename T>
-__global__ __launch_bounds__(NT, 1) void sp2_f16split_kernel(F16Args g) {
+__device__ __forceinline__ void split_tile(const T* ahi, const T* alo, const T* bhi, const T* blo,
+                                           int ld, int I, int J, int8_t* ring, f4 (&hh)[4][4],
+                                           f4 (&xx)[4][4]) {
   typedef typename Split<T>::v8 h8;
-  constexpr double kScale = Split<T>::kScale;
-  __shared__ T As[BM][HROW];
-  __shared__ T Bs[BM][HROW];
-  __shared__ int s_flags[4];
-  if (threadIdx.x == 0) {
-    s_flags[0] = g.st->planned;
-    s_flags[1] = g.st->apply;
-    s_flags[2] = g.st->sigma;
-    s_flags[3] = g.st->cur;
-  }
-  __syncthreads();
-  if (!s_flags[0]) return;
-  const int apply = s_flags[1], sigma = s_flags[2], cur = s_flags[3];
-  const int ld = g.ld;
-  const double* X = g.buf[cur];
-  double* Xn = const_cast<double*>(g.buf[cur ^ 1]);
-  const T* hi = (const T*)g.hi[cur];
-  const T* lo = (const T*)g.lo[cur];
-  T* hin = (T*)const_cast<void*>(g.hi[cur ^ 1]);
-  T* lon = (T*)const_cast<void*>(g.lo[cur ^ 1]);
-
-  const int t = xcd_remap(blockIdx.x, gridDim.x);
-  int I, J;
-  sym_tile(t, I, J);
   const int tid = threadIdx.x, lane = tid & 63;
-  const int w = tid >> 6, wm = w & 1, wn = w >> 1;
-
-  f4 acc_hh[4][4], acc_x[4][4];
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6), wm = w & 1, wn = w >> 1;
+  const int lrow = lane >> 2;
+  const uint32_t voff = (uint32_t)(lrow * 64 + 16 * ((lane & 3) ^ ((lrow >> 1) & 3)));
+  const uint32_t ring0 = __builtin_amdgcn_readfirstlane(lds_dma::lds_addr(ring));
+  // chunk w + 4 q (q < 8) is rows 16 ((w + 4 q) % 8) of panel q / 2
+  const size_t kblock = (size_t)KB * ld * sizeof(T);
+  const uint64_t panel[4] = {
+      lds_dma::uniform64((uint64_t)(uintptr_t)(ahi + (size_t)I * BM * KB)),
+      lds_dma::uniform64((uint64_t)(uintptr_t)(alo + (size_t)I * BM * KB)),
+      lds_dma::uniform64((uint64_t)(uintptr_t)(bhi + (size_t)J * BM * KB)),
+      lds_dma::uniform64((uint64_t)(uintptr_t)(blo + (size_t)J * BM * KB))};
+  auto issue = [&](int s) {
+    const size_t off = (size_t)s * kblock;
+    const uint32_t slot = ring0 + kSlab * (s & 1);
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      const int c = w + 4 * (q & 1);  // chunk of its panel
+      lds_dma::dma16(panel[q >> 1] + off + 1024 * c, voff,
+                     __builtin_amdgcn_readfirstlane(slot + kPanel * (q >> 1) + 1024 * c));
+    }
+  };
+  const int fo = (lane & 15) * 64 + 16 * ((lane >> 4) ^ (((lane & 15) >> 1) & 3));
+  const int8_t* fa = ring + wm * 64 * 64 + fo;
+  const int8_t* fb = ring + 2 * kPanel + wn * 64 * 64 + fo;
 #pragma unroll
   for (int m = 0; m < 4; ++m)
 #pragma unroll
     for (int n = 0; n < 4; ++n) {
-      acc_hh[m][n] = f4{0.f, 0.f, 0.f, 0.f};
-      acc_x[m][n] = f4{0.f, 0.f, 0.f, 0.f};
+      hh[m][n] = f4{0.f, 0.f, 0.f, 0.f};
+      xx[m][n] = f4{0.f, 0.f, 0.f, 0.f};
     }
-
-  // three segments over K: (hi,hi) -> acc_hh ; (hi,lo), (lo,hi) -> acc_x
-  const int ksteps = ld / BK;
-  const int total = 3 * ksteps;
-  const int c = tid >> 1, kh = (tid & 1) * 32;
-  i4 ra[4], rb[4];
-  auto load = [&](int s) {
-    const int seg = s / ksteps;
-    const int k0 = (s - seg * ksteps) * BK;
-    const T* Ap = (seg == 2) ? lo : hi;
-    const T* Bp = (seg == 1) ? lo : hi;
-    const T* pa = Ap + (size_t)(I * BM + c) * ld + k0 + kh;
-    const T* pb = Bp + (size_t)(J * BM + c) * ld + k0 + kh;
+  const int slabs = ld / KB;
+  issue(0);
+  for (int s = 0; s < slabs; ++s) {
+    // slab s has landed in every wave, and every wave has read slab s - 1
+    lds_dma::wait_vm_barrier<0>();
+    if (s + 1 < slabs) issue(s + 1);
+    const int o = kSlab * (s & 1);
+    h8 ah[4], al[4], bh[4], bl[4];
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      ra[q] = *(const i4*)(pa + 8 * q);
-      rb[q] = *(const i4*)(pb + 8 * q);
-    }
-  };
-  load(0);
-  for (int s = 0; s < total; ++s) {
-    __syncthreads();
+    for (int m = 0; m < 4; ++m) ah[m] = *(const h8*)(fa + o + 1024 * m);
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      *(i4*)(&As[c][kh + 8 * q]) = ra[q];
-      *(i4*)(&Bs[c][kh + 8 * q]) = rb[q];
-    }
-    __syncthreads();
-    if (s + 1 < total) load(s + 1);
-    const bool cross = s >= ksteps;
+    for (int n = 0; n < 4; ++n) bh[n] = *(const h8*)(fb + o + 1024 * n);
 #pragma unroll
-    for (int kk = 0; kk < BK / 32; ++kk) {
-      const int kc = kk * 32 + 8 * (lane >> 4);
-      h8 a[4], b[4];
+    for (int n = 0; n < 4; ++n) bl[n] = *(const h8*)(fb + o + kPanel + 1024 * n);
 #pragma unroll
-      for (int m = 0; m < 4; ++m) a[m] = *(const h8*)(&As[wm * 64 + m * 16 + (lane & 15)][kc]);
+    for (int m = 0; m < 4; ++m) al[m] = *(const h8*)(fa + o + kPanel + 1024 * m);
 #pragma unroll
-      for (int n = 0; n < 4; ++n) b[n] = *(const h8*)(&Bs[wn * 64 + n * 16 + (lane & 15)][kc]);
-      if (cross) {
+    for (int m = 0; m < 4; ++m)
 #pragma unroll
-        for (int m = 0; m < 4; ++m)
+      for (int n = 0; n < 4; ++n) hh[m][n] = Split<T>::mfma(bh[n], ah[m], hh[m][n]);
 #pragma unroll
-          for (int n = 0; n < 4; ++n)
-            acc_x[m][n] = Split<T>::mfma(b[n], a[m], acc_x[m][n]);
-      } else {
+    for (int m = 0; m < 4; ++m)
 #pragma unroll
-        for (int m = 0; m < 4; ++m)
+      for (int n = 0; n < 4; ++n) xx[m][n] = Split<T>::mfma(bl[n], ah[m], xx[m][n]);
 #pragma unroll
-          for (int n = 0; n < 4; ++n)
-            acc_hh[m][n] = Split<T>::mfma(b[n], a[m], acc_hh[m][n]);
-      }
-    }
+    for (int m = 0; m < 4; ++m)
+#pragma unroll
+      for (int n = 0; n < 4; ++n) xx[m][n] = Split<T>::mfma(bh[n], al[m], xx[m][n]);
   }
+}
 
-  // Epilogue.  Operands were swapped, so this lane holds (X^2)[row][col]
-  // with row = lane%16 and col = 4*(lane/16) + r within each 16 x 16 block.
-  // Off-diagonal tiles are mirrored; inside a diagonal tile the upper half is
-  // mirrored onto the lower one (the hi.lo and lo.hi terms of (r, c) and
-  // (c, r) accumulate in different orders), so X_next is exactly symmetric.
-  const double ca = apply ? (sigma ? 1.0 : -1.0) : 0.0;
-  const double cb = apply ? (sigma ? 0.0 : 2.0) : 1.0;
+// Operands were swapped, so a lane holds (A B)[row][col] with
+// row = lane % 16 and col = 4 (lane / 16) + r inside each 16 x 16 block.
+struct SplitAt {
+  int lane, row0, col0;  // the lane's first row and column
+  int w;
+  __device__ SplitAt(int I, int J) {
+    lane = threadIdx.x & 63;
+    w = threadIdx.x >> 6;
+    row0 = I * BM + (w & 1) * 64 + (lane & 15);
+    col0 = J * BM + (w >> 1) * 64 + 4 * (lane >> 4);
+  }
+};
+
+struct F16Args {
+  const double* buf[2];         // FP64 master ping-pong (lower triangle)
+  const void* hi[2];            // hi planes ping-pong (T)
+  const void* lo[2];            // lo planes ping-pong (T)
+  int ld, nt;
+  Sp2State* st;
+  double* part;
+};
+
+constexpr int kBand = 8;  // tile columns of a band: an XCD's 64 workgroups cover 8 x 8 tiles
+constexpr int kPitch = 64 + 4;  // halves per row of a wave's 64 x 64 block in LDS
+
+// The upper-triangle tile (I, J) of X^2 and the SP2 update.  The FP64 master
+// lives in the lower triangle (and the whole of each diagonal 128 x 128
+// block), where a lane's four columns are 32 contiguous bytes; the loop's end
+// restores the upper one.  Both positions of the planes are written: (row,
+// col) by the lane's four columns at a time, (col, row) after a transposition
+// of each wave's block through LDS, 8 bytes per lane each.
+template <typename T>
+__global__ __launch_bounds__(NT, 2) void sp2_f16split_kernel(F16Args g) {
+  constexpr double kScale = Split<T>::kScale;
+  __shared__ __attribute__((aligned(1024))) int8_t ring[kRing];
+  const volatile Sp2State* stv = g.st;
+  if (!stv->planned) return;
+  const int apply = stv->apply, sigma = stv->sigma, cur = stv->cur;
   // prg_sp2_submatrix: the idempotency sum runs over the first `core` rows
   // (and, by symmetry, the mirrored columns) only
-  const int core_lim = (g.st->variant == V_SUBMATRIX) ? g.st->core : 0x7fffffff;
+  const int core_lim = (stv->variant == V_SUBMATRIX) ? stv->core : 0x7fffffff;
+  const int ld = g.ld;
+  const int t = xcd_remap(blockIdx.x, gridDim.x);
+  int I, J;
+  sym_tile_banded<kBand>(t, g.nt, I, J);
+  f4 hh[4][4], xx[4][4];
+  split_tile<T>((const T*)g.hi[cur], (const T*)g.lo[cur], (const T*)g.hi[cur], (const T*)g.lo[cur],
+                ld, I, J, ring, hh, xx);
+  const double* X = g.buf[cur];
+  double* Xn = const_cast<double*>(g.buf[cur ^ 1]);
+  T* hin = (T*)const_cast<void*>(g.hi[cur ^ 1]);
+  T* lon = (T*)const_cast<void*>(g.lo[cur ^ 1]);
+  const double ca = apply ? (sigma ? 1.0 : -1.0) : 0.0;
+  const double cb = apply ? (sigma ? 0.0 : 2.0) : 1.0;
+  const SplitAt at(I, J);
   double sums[4] = {0.0, 0.0, 0.0, 0.0};
+  typedef T t4 __attribute__((ext_vector_type(4)));
+  // every wave is done with the ring: its LDS takes the waves' blocks
+  lds_dma::wait_vm_barrier<0>();
+  T* block = (T*)ring + (size_t)at.w * 64 * kPitch;
+  if (I != J) {
 #pragma unroll
-  for (int m = 0; m < 4; ++m) {
+    for (int m = 0; m < 4; ++m) {
+      const int row = at.row0 + 16 * m;
+      const double wrow = row < core_lim ? 1.0 : 0.0;
+      t4 lov[4];
 #pragma unroll
-    for (int n = 0; n < 4; ++n) {
-      const int row = I * BM + wm * 64 + m * 16 + (lane & 15);
-      double q0 = 0.0, q1 = 0.0, q2 = 0.0, q3 = 0.0;
+      for (int n = 0; n < 4; ++n) {
+        const int col = at.col0 + 16 * n;
+        const double2* xp = (const double2*)(X + col + (size_t)row * ld);
+        const double2 u = xp[0], v = xp[1];
+        const double xs[4] = {u.x, u.y, v.x, v.y};
+        double z[4];
+        t4 h, l;
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int col = J * BM + wn * 64 + n * 16 + 4 * (lane >> 4) + r;
-        if (row > col) continue;  // lower half of a diagonal tile
-        const bool mirror = (row != col);
-        const double we = mirror ? 2.0 : 1.0;
-        const size_t idx = row + (size_t)col * ld;
-        const size_t tdx = mirror ? col + (size_t)row * ld : idx;
-        const double y = (double)acc_hh[m][n][r] + (1.0 / kScale) * (double)acc_x[m][n][r];
-        const double x = X[idx];
-        const double z = fma(cb, x, ca * y);
-        const double dxy = x - y;
-        const bool diag = (row == col);
-        const double wc = (row < core_lim ? 1.0 : 0.0) + ((mirror && col < core_lim) ? 1.0 : 0.0);
-        q0 += we * z * z;
-        q2 += wc * dxy * dxy;
-        q1 += diag ? z : 0.0;
-        q3 += diag ? y : 0.0;
-        const T h = (T)z;
-        const T l = (T)((z - (double)h) * kScale);
-        Xn[idx] = z;
-        Xn[tdx] = z;
-        hin[idx] = h;
-        hin[tdx] = h;
-        lon[idx] = l;
-        lon[tdx] = l;
+        for (int r = 0; r < 4; ++r) {
+          const double y = (double)hh[m][n][r] + (1.0 / kScale) * (double)xx[m][n][r];
+          z[r] = fma(cb, xs[r], ca * y);
+          const double d = xs[r] - y;
+          sums[0] += 2.0 * z[r] * z[r];
+          sums[2] += (wrow + (col + r < core_lim ? 1.0 : 0.0)) * d * d;
+          h[r] = (T)z[r];
+          l[r] = (T)((z[r] - (double)h[r]) * kScale);
+        }
+        double2* zp = (double2*)(Xn + col + (size_t)row * ld);
+        zp[0] = double2{z[0], z[1]};
+        zp[1] = double2{z[2], z[3]};
+        const size_t pi = plane_at(row, col, ld);
+        *(t4*)(hin + pi) = h;
+        *(t4*)(lon + pi) = l;
+        *(t4*)(block + (16 * m + (at.lane & 15)) * kPitch + 16 * n + 4 * (at.lane >> 4)) = h;
+        lov[n] = l;
+        __builtin_amdgcn_sched_barrier(0);
       }
-      sums[0] += q0;
-      sums[1] += q1;
-      sums[2] += q2;
-      sums[3] += q3;
-      __builtin_amdgcn_sched_barrier(0);
+      // the lo halves wait in the accumulators' place for the second pass
+#pragma unroll
+      for (int n = 0; n < 4; ++n) {
+        const uint2 b = __builtin_bit_cast(uint2, lov[n]);
+        hh[m][n][0] = __uint_as_float(b.x);
+        hh[m][n][1] = __uint_as_float(b.y);
+      }
+    }
+    // Transposed store of the wave's block: lane b handles the 4 x 4 blocks
+    // (row block b % 16, column blocks b / 16 + 4 q), 16 lanes covering the
+    // 64 rows, i.e. two runs of 64 bytes per column.
+    auto mirror = [&](T* plane) {
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      const int rb = 4 * (at.lane & 15), cb0 = 4 * (at.lane >> 4);
+      const int rowb = I * BM + (at.w & 1) * 64 + rb, colb = J * BM + (at.w >> 1) * 64 + cb0;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        t4 e[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) e[i] = *(const t4*)(block + (rb + i) * kPitch + cb0 + 16 * q);
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          *(t4*)(plane + plane_at(colb + 16 * q + j, rowb, ld)) =
+              t4{e[0][j], e[1][j], e[2][j], e[3][j]};
+      }
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+    };
+    mirror(hin);
+#pragma unroll
+    for (int m = 0; m < 4; ++m)
+#pragma unroll
+      for (int n = 0; n < 4; ++n)
+        *(uint2*)(block + (16 * m + (at.lane & 15)) * kPitch + 16 * n + 4 * (at.lane >> 4)) =
+            uint2{__float_as_uint(hh[m][n][0]), __float_as_uint(hh[m][n][1])};
+    mirror(lon);
+  } else {
+    // inside a diagonal tile the upper half is written to both places (the
+    // hi.lo and lo.hi terms of (r, c) and (c, r) accumulate in different
+    // orders), so X_next is exactly symmetric
+#pragma unroll
+    for (int m = 0; m < 4; ++m) {
+      const int row = at.row0 + 16 * m;
+#pragma unroll
+      for (int n = 0; n < 4; ++n) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int col = at.col0 + 16 * n + r;
+          if (row > col) continue;
+          const bool diag = (row == col);
+          const double y = (double)hh[m][n][r] + (1.0 / kScale) * (double)xx[m][n][r];
+          const size_t idx = row + (size_t)col * ld, tdx = col + (size_t)row * ld;
+          const double x = X[tdx];
+          const double z = fma(cb, x, ca * y);
+          const double d = x - y;
+          const double wc =
+              (row < core_lim ? 1.0 : 0.0) + ((!diag && col < core_lim) ? 1.0 : 0.0);
+          sums[0] += (diag ? 1.0 : 2.0) * z * z;
+          sums[2] += wc * d * d;
+          sums[1] += diag ? z : 0.0;
+          sums[3] += diag ? y : 0.0;
+          const T h = (T)z;
+          const T l = (T)((z - (double)h) * kScale);
+          Xn[idx] = z;
+          Xn[tdx] = z;
+          hin[plane_at(row, col, ld)] = h;
+          hin[plane_at(col, row, ld)] = h;
+          lon[plane_at(row, col, ld)] = l;
+          lon[plane_at(col, row, ld)] = l;
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
     }
   }
-  block_store_partials<4>(sums, g.part + 4 * (size_t)t);
+  block_store4<NT>(sums, g.part + 4 * (size_t)t);
+}
+
+// X (current buffer) from its lower triangle: the upper 64 x 64 blocks are
+// the transposes of their mirror blocks, through LDS.
+__global__ void sp2_mirror_kernel(double* x0, double* x1, const Sp2State* __restrict__ s, int ld) {
+  __shared__ double t[64][65];
+  double* x = s->cur ? x1 : x0;
+  const int br = blockIdx.x * 64, bc = blockIdx.y * 64;
+  if (br <= bc) return;  // blocks below the diagonal, whose transposes are written
+  const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
+  for (int j = ty; j < 64; j += 4) t[j][tx] = x[(br + tx) + (size_t)(bc + j) * ld];
+  __syncthreads();
+  for (int j = ty; j < 64; j += 4) x[(bc + tx) + (size_t)(br + j) * ld] = t[tx][j];
 }
 
 struct SplitGemmArgs {
@@ -219,142 +339,128 @@ struct SplitGemmArgs {
   double* C;
   double* part;       // per tile [Tr C, ||C||_F^2, <C, E>, 0], or null
   double alpha, beta, gamma;
-  int ld, n;
+  int ld, n, nt;
 };
 
 // C = alpha A B + beta Cin + gamma I (gamma on the n x n diagonal) for
 // symmetric, commuting A and B from their hi/lo planes: one workgroup per
 // upper-triangle 128 x 128 tile, the tile mirrored; inside a diagonal tile
 // the upper half is mirrored onto the lower one, so C is exactly symmetric.
-template <typename T>
-__global__ __launch_bounds__(NT, 1) void split_gemm_kernel(SplitGemmArgs g) {
+// FUSE bit 0: with Cin, bit 1: with <C, E>.
+template <typename T, int FUSE>
+__global__ __launch_bounds__(NT, 2) void split_gemm_kernel(SplitGemmArgs g) {
   constexpr double kScale = Split<T>::kScale;
-  __shared__ T As[BM][HROW];
-  __shared__ T Bs[BM][HROW];
+  __shared__ __attribute__((aligned(1024))) int8_t ring[kRing];
   const int ld = g.ld;
   const int t = xcd_remap(blockIdx.x, gridDim.x);
   int I, J;
-  sym_tile(t, I, J);
-  const T* ahi = (const T*)g.ahi;
-  const T* alo = (const T*)g.alo;
-  const T* bhi = (const T*)g.bhi;
-  const T* blo = (const T*)g.blo;
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int w = tid >> 6, wm = w & 1, wn = w >> 1;
-  // the main loop of sp2_f16split_kernel on the operand planes, three
-  // segments over K: (hi, hi) -> acc_hh; (hi, lo), (lo, hi) -> acc_x.  (An
-  // inline copy: behind a shared function the compiler moved the
-  // accumulators between AGPRs and VGPRs inside the loop, a third slower.)
-  typedef typename Split<T>::v8 h8;
-  f4 acc_hh[4][4], acc_x[4][4];
-#pragma unroll
-  for (int m = 0; m < 4; ++m)
-#pragma unroll
-    for (int n = 0; n < 4; ++n) {
-      acc_hh[m][n] = f4{0.f, 0.f, 0.f, 0.f};
-      acc_x[m][n] = f4{0.f, 0.f, 0.f, 0.f};
-    }
-  const int ksteps = ld / BK;
-  const int total = 3 * ksteps;
-  const int c = tid >> 1, kh = (tid & 1) * 32;
-  i4 ra[4], rb[4];
-  auto load = [&](int s) {
-    const int seg = s / ksteps;
-    const int k0 = (s - seg * ksteps) * BK;
-    const T* Ap = (seg == 2) ? alo : ahi;
-    const T* Bp = (seg == 1) ? blo : bhi;
-    const T* pa = Ap + (size_t)(I * BM + c) * ld + k0 + kh;
-    const T* pb = Bp + (size_t)(J * BM + c) * ld + k0 + kh;
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      ra[q] = *(const i4*)(pa + 8 * q);
-      rb[q] = *(const i4*)(pb + 8 * q);
-    }
-  };
-  load(0);
-  for (int s = 0; s < total; ++s) {
-    __syncthreads();
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      *(i4*)(&As[c][kh + 8 * q]) = ra[q];
-      *(i4*)(&Bs[c][kh + 8 * q]) = rb[q];
-    }
-    __syncthreads();
-    if (s + 1 < total) load(s + 1);
-    const bool cross = s >= ksteps;
-#pragma unroll
-    for (int kk = 0; kk < BK / 32; ++kk) {
-      const int kc = kk * 32 + 8 * (lane >> 4);
-      h8 a[4], b[4];
-#pragma unroll
-      for (int m = 0; m < 4; ++m) a[m] = *(const h8*)(&As[wm * 64 + m * 16 + (lane & 15)][kc]);
-#pragma unroll
-      for (int n = 0; n < 4; ++n) b[n] = *(const h8*)(&Bs[wn * 64 + n * 16 + (lane & 15)][kc]);
-      if (cross) {
-#pragma unroll
-        for (int m = 0; m < 4; ++m)
-#pragma unroll
-          for (int n = 0; n < 4; ++n)
-            acc_x[m][n] = Split<T>::mfma(b[n], a[m], acc_x[m][n]);
-      } else {
-#pragma unroll
-        for (int m = 0; m < 4; ++m)
-#pragma unroll
-          for (int n = 0; n < 4; ++n)
-            acc_hh[m][n] = Split<T>::mfma(b[n], a[m], acc_hh[m][n]);
-      }
-    }
-  }
+  sym_tile_banded<kBand>(t, g.nt, I, J);
+  f4 hh[4][4], xx[4][4];
+  split_tile<T>((const T*)g.ahi, (const T*)g.alo, (const T*)g.bhi, (const T*)g.blo, ld, I, J, ring,
+                hh, xx);
+  const SplitAt at(I, J);
   double sums[4] = {0.0, 0.0, 0.0, 0.0};
+  if (I != J) {
+    // the (col, row) position is 32 contiguous bytes per lane
 #pragma unroll
-  for (int m = 0; m < 4; ++m) {
+    for (int m = 0; m < 4; ++m) {
+      const int row = at.row0 + 16 * m;
 #pragma unroll
-    for (int n = 0; n < 4; ++n) {
-      const int row = I * BM + wm * 64 + m * 16 + (lane & 15);
+      for (int n = 0; n < 4; ++n) {
+        const int col = at.col0 + 16 * n;
+        const size_t tdx = col + (size_t)row * ld;
+        double v[4];
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int col = J * BM + wn * 64 + n * 16 + 4 * (lane >> 4) + r;
-        if (row > col) continue;  // lower half of a diagonal tile
-        const bool mirror = (row != col), diag = !mirror;
-        const size_t idx = row + (size_t)col * ld;
-        double v = g.alpha * ((double)acc_hh[m][n][r] + (1.0 / kScale) * (double)acc_x[m][n][r]);
-        if (g.Cin) v += g.beta * g.Cin[idx];
-        v += (diag && row < g.n) ? g.gamma : 0.0;
-        const double we = mirror ? 2.0 : 1.0;
-        sums[0] += diag ? v : 0.0;
-        sums[1] += we * v * v;
-        if (g.E) sums[2] += we * v * g.E[idx];
-        g.C[idx] = v;
-        if (mirror) g.C[col + (size_t)row * ld] = v;
+        for (int r = 0; r < 4; ++r)
+          v[r] = g.alpha * ((double)hh[m][n][r] + (1.0 / kScale) * (double)xx[m][n][r]);
+        if (FUSE & 1) {
+          const double2* cp = (const double2*)(g.Cin + tdx);
+          const double2 a = cp[0], b = cp[1];
+          v[0] += g.beta * a.x;
+          v[1] += g.beta * a.y;
+          v[2] += g.beta * b.x;
+          v[3] += g.beta * b.y;
+        }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) sums[1] += 2.0 * v[r] * v[r];
+        if (FUSE & 2) {
+          const double2* ep = (const double2*)(g.E + tdx);
+          const double2 a = ep[0], b = ep[1];
+          sums[2] += 2.0 * (v[0] * a.x + v[1] * a.y + v[2] * b.x + v[3] * b.y);
+        }
+        double2* tp = (double2*)(g.C + tdx);
+        tp[0] = double2{v[0], v[1]};
+        tp[1] = double2{v[2], v[3]};
+#pragma unroll
+        for (int r = 0; r < 4; ++r) g.C[row + (size_t)(col + r) * ld] = v[r];
+        __builtin_amdgcn_sched_barrier(0);
       }
-      __builtin_amdgcn_sched_barrier(0);
+    }
+  } else {
+#pragma unroll
+    for (int m = 0; m < 4; ++m) {
+      const int row = at.row0 + 16 * m;
+#pragma unroll
+      for (int n = 0; n < 4; ++n) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int col = at.col0 + 16 * n + r;
+          if (row > col) continue;  // lower half of a diagonal tile
+          const bool diag = (row == col);
+          const size_t idx = row + (size_t)col * ld;
+          double v = g.alpha * ((double)hh[m][n][r] + (1.0 / kScale) * (double)xx[m][n][r]);
+          if (FUSE & 1) v += g.beta * g.Cin[idx];
+          v += (diag && row < g.n) ? g.gamma : 0.0;
+          const double we = diag ? 1.0 : 2.0;
+          sums[0] += diag ? v : 0.0;
+          sums[1] += we * v * v;
+          if (FUSE & 2) sums[2] += we * v * g.E[idx];
+          g.C[idx] = v;
+          g.C[col + (size_t)row * ld] = v;
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
     }
   }
-  if (g.part) block_store_partials<4>(sums, g.part + 4 * (size_t)t);
+  if (g.part) block_store4<NT>(sums, g.part + 4 * (size_t)t);
 }
 
-// hi/lo planes of an FP64 matrix (whole ld x ld buffer, padding stays zero).
+// hi/lo planes of a symmetric FP64 matrix (whole ld x ld buffer, padding stays
+// zero) in the blocked layout: a thread converts 4 consecutive k's of a row r,
+// read as (k, r), 32 contiguous bytes.
 template <typename T>
 __global__ void split_f16_kernel(const double* __restrict__ x, T* __restrict__ hi,
-                                 T* __restrict__ lo, size_t count) {
+                                 T* __restrict__ lo, int ld) {
+  typedef T t4 __attribute__((ext_vector_type(4)));
+  const size_t count = (size_t)ld * ld / 4;
   for (size_t i = (size_t)blockIdx.x * NT + threadIdx.x; i < count; i += (size_t)gridDim.x * NT) {
-    const double z = x[i];
-    const T h = (T)z;
-    hi[i] = h;
-    lo[i] = (T)((z - (double)h) * Split<T>::kScale);
+    // i-th group of 4 in plane order: 8 groups per row of a 32-column block
+    const int kq = (int)(i & 7);
+    const size_t q = i >> 3;
+    const int r = (int)(q % ld), k = (int)(q / ld) * KB + 4 * kq;
+    const double2* xp = (const double2*)(x + k + (size_t)r * ld);
+    const double2 a = xp[0], b = xp[1];
+    const double z[4] = {a.x, a.y, b.x, b.y};
+    t4 h, l;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      h[j] = (T)z[j];
+      l[j] = (T)((z[j] - (double)h[j]) * Split<T>::kScale);
+    }
+    *(t4*)(hi + 4 * i) = h;
+    *(t4*)(lo + 4 * i) = l;
   }
 }
 
 }  // namespace
 
 int split_f16(const DMat& x, void* hi, void* lo, bool bf16) {
-  const size_t count = (size_t)x.ld * x.ld;
   if (bf16)
     hipLaunchKernelGGL(split_f16_kernel<__bf16>, dim3(2048), dim3(NT), 0, stream(), x.p,
-                       (__bf16*)hi, (__bf16*)lo, count);
+                       (__bf16*)hi, (__bf16*)lo, x.ld);
   else
     hipLaunchKernelGGL(split_f16_kernel<_Float16>, dim3(2048), dim3(NT), 0, stream(), x.p,
-                       (_Float16*)hi, (_Float16*)lo, count);
+                       (_Float16*)hi, (_Float16*)lo, x.ld);
   PRG_HIP_CHECK(hipGetLastError());
   return OK;
 }
@@ -380,15 +486,23 @@ int sp2_step_mixed(const DMat& x0, const DMat& x1, Sp2State* d_state, double* d_
   g.hi[1] = planes + 2 * plane;
   g.lo[1] = planes + 3 * plane;
   g.ld = ld;
+  g.nt = ld / BM;
   g.st = d_state;
   g.part = d_part;
-  const int nt = ld / BM;
-  const int nb = nt * (nt + 1) / 2;
+  const int nb = g.nt * (g.nt + 1) / 2;
   if (ntiles) *ntiles = nb;
   if (bf16)
     hipLaunchKernelGGL(sp2_f16split_kernel<__bf16>, dim3(nb), dim3(NT), 0, stream(), g);
   else
     hipLaunchKernelGGL(sp2_f16split_kernel<_Float16>, dim3(nb), dim3(NT), 0, stream(), g);
+  PRG_HIP_CHECK(hipGetLastError());
+  return OK;
+}
+
+int sp2_mirror(const DMat& x0, const DMat& x1, const Sp2State* d_state) {
+  const int nb = x0.ld / 64;
+  hipLaunchKernelGGL(sp2_mirror_kernel, dim3(nb, nb), dim3(NT), 0, stream(), x0.p, x1.p, d_state,
+                     x0.ld);
   PRG_HIP_CHECK(hipGetLastError());
   return OK;
 }
@@ -474,10 +588,15 @@ int split_gemm(const DMat& A, const DMat& B, DMat C, double alpha, double beta, 
   g.gamma = gamma;
   g.ld = ld;
   g.n = C.n;
-  const int nt = ld / BM;
-  const int nb = nt * (nt + 1) / 2;
+  g.nt = ld / BM;
+  const int nb = g.nt * (g.nt + 1) / 2;
   if (nparts) *nparts = nb;
-  hipLaunchKernelGGL(split_gemm_kernel<__bf16>, dim3(nb), dim3(NT), 0, stream(), g);
+  const int fuse = (g.Cin ? 1 : 0) | (g.E ? 2 : 0);
+  void (*k)(SplitGemmArgs) = fuse == 0   ? split_gemm_kernel<__bf16, 0>
+                             : fuse == 1 ? split_gemm_kernel<__bf16, 1>
+                             : fuse == 2 ? split_gemm_kernel<__bf16, 2>
+                                         : split_gemm_kernel<__bf16, 3>;
+  hipLaunchKernelGGL(k, dim3(nb), dim3(NT), 0, stream(), g);
   PRG_HIP_CHECK(hipGetLastError());
   return OK;
 }

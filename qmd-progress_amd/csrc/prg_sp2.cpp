@@ -363,7 +363,12 @@ int run_sp2(const DMat& H, const Sp2Params& p_in, DMat out, Sp2Result* res, cons
       done = slot[(chunk_no - 1) & 1]->done != 0;
       last_head = slot[(chunk_no - 1) & 1];
     }
-    if (phase == 0) phase0_steps = steps;
+    if (phase == 0) {
+      phase0_steps = steps;
+      if ((prec == PRG_PREC_F16SPLIT || prec == PRG_PREC_BF16SPLIT) && !response &&
+          (st = sp2_mirror(X0, X1, dst)))
+        return st;
+    }
   }
   // the int8 CRT update keeps X in its residue planes (or the lower
   // triangle of an FP64 master at 12 or more moduli) between steps

@@ -64,6 +64,9 @@ int sp2_step_mixed(const DMat& x0, const DMat& x1, Sp2State* d_state, double* d_
                    int* ntiles, int prec);
 // Builds the low-precision representation of X0 (after normalisation).
 int sp2_mixed_prepare(const DMat& x0, int prec);
+// The 16-bit split steps keep the FP64 master's lower triangle; this fills the
+// upper one of the current buffer.
+int sp2_mirror(const DMat& x0, const DMat& x1, const Sp2State* d_state);
 
 // int8 Chinese-remainder products (prg_gemm_crt.hip)
 int crt_prepare(const DMat& x0, int np);

@@ -21,7 +21,8 @@ ROOT = Path(__file__).resolve().parent.parent
 CSRC = ROOT / "qmd-progress_amd" / "csrc"
 # (source file, mangled-name pattern of its LDS-ring kernels)
 RING_KERNELS = [("prg_gemm_crt.hip", r"_Z\S*crt_product\S*kernel\S*"),
-                ("prg_batched.hip", r"_Z\S*batched_split_ring_kernel\S*")]
+                ("prg_batched.hip", r"_Z\S*batched_split_ring_kernel\S*"),
+                ("prg_gemm_mixed.hip", r"_Z\S*(?:sp2_f16split|split_gemm)_kernel\S*")]
 HIPCC = Path("/opt/rocm/bin/hipcc")
 
 
