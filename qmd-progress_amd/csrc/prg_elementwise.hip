@@ -301,6 +301,40 @@ __global__ void transpose_kernel(const double* __restrict__ a, double* __restric
   for (int j = ty; j < 64; j += 4) out[(by + tx) + (size_t)(bx + j) * ld] = t[tx][j];
 }
 
+// U = ((W - 2 F) + (W - 2 F)^T) / 2 and S = F + F^T, one 64 x 64 block of the
+// upper triangle and its mirror per workgroup: both matrices are read once and
+// both results written once (HBM bound, 32 bytes per entry; as transposes and
+// sums of whole matrices it was 9 passes).
+__global__ void symmetrize_pair_kernel(const double* __restrict__ w, const double* __restrict__ f,
+                                       double* __restrict__ u, double* __restrict__ s, int ld) {
+  __shared__ double tu[64][65], ts[64][65];
+  const int bx = blockIdx.x * 64, by = blockIdx.y * 64;
+  if (bx > by) return;
+  const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;  // 64 x 4 threads
+  for (int j = ty; j < 64; j += 4) {
+    const size_t i = (by + tx) + (size_t)(bx + j) * ld;  // the mirror block
+    tu[j][tx] = w[i] - 2.0 * f[i];
+    ts[j][tx] = f[i];
+  }
+  __syncthreads();
+  // this block, and in LDS (each thread its own entries) what the mirror gets
+  for (int j = ty; j < 64; j += 4) {
+    const size_t i = (bx + tx) + (size_t)(by + j) * ld;
+    const double fv = f[i], us = 0.5 * ((w[i] - 2.0 * fv) + tu[tx][j]), ss = fv + ts[tx][j];
+    u[i] = us;
+    s[i] = ss;
+    tu[tx][j] = us;
+    ts[tx][j] = ss;
+  }
+  if (bx == by) return;  // its own mirror
+  __syncthreads();
+  for (int j = ty; j < 64; j += 4) {
+    const size_t i = (by + tx) + (size_t)(bx + j) * ld;
+    u[i] = tu[j][tx];
+    s[i] = ts[j][tx];
+  }
+}
+
 __global__ void scale_cols_kernel(const double* __restrict__ a, const double* __restrict__ f,
                                   double* __restrict__ out, int n, int ld) {
   for (int col = blockIdx.x; col < ld; col += gridDim.x) {
@@ -374,6 +408,19 @@ int transpose_kernel_launch(const DMat& A, DMat out) {
   }
   const int nb = A.ld / 64;
   hipLaunchKernelGGL(transpose_kernel, dim3(nb, nb), dim3(NT), 0, stream(), A.p, out.p, A.ld);
+  PRG_HIP_CHECK(hipGetLastError());
+  return OK;
+}
+
+int symmetrize_pair_launch(const DMat& W, const DMat& F, DMat U, DMat S) {
+  if (W.ld != F.ld || W.ld != U.ld || W.ld != S.ld || U.p == W.p || U.p == F.p || S.p == W.p ||
+      S.p == F.p || U.p == S.p) {
+    set_error(ERR_ARG, "symmetrize_pair: layout mismatch or aliasing");
+    return ERR_ARG;
+  }
+  const int nb = W.ld / 64;
+  hipLaunchKernelGGL(symmetrize_pair_kernel, dim3(nb, nb), dim3(NT), 0, stream(), W.p, F.p, U.p,
+                     S.p, W.ld);
   PRG_HIP_CHECK(hipGetLastError());
   return OK;
 }

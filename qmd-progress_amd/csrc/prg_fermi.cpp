@@ -10,6 +10,7 @@
 #include <cmath>
 #include <cstdio>
 #include <string>
+#include <utility>
 #include <vector>
 
 #include "prg_bml.h"
@@ -66,30 +67,44 @@ int conjgrad(const DMat& A, DMat X, const DMat& B, double tol, bool commuting, i
 // `commuting`: Ai is a polynomial of A (true of every inverse the implicit
 // Fermi recursion refines: A and the initial Ai are functions of H), so both
 // products are symmetric and only their upper-triangle tiles are computed.
-int newtonschulz(const DMat& A, DMat Ai, double tol, int* iters, bool commuting) {
-  DMat R, T, I;
+// The iterates alternate between the buffers `out` and `scratch` (no copy
+// passes); on return `out` names the one that holds the result.  `start` (the
+// initial Ai) may be `out`, otherwise it is not changed.
+int newtonschulz_into(const DMat& A, const DMat& start, DMat& out, DMat& scratch, double tol,
+                      int* iters, bool commuting) {
+  DMat R, I;
   int st;
   ops::HoldOperand hold(A);  // A is not changed here
-  if ((st = ops::temp("ns_r", A.n, &R)) || (st = ops::temp("ns_t", A.n, &T)) ||
-      (st = ops::temp("ns_i", A.n, &I)))
-    return st;
+  if ((st = ops::temp("ns_r", A.n, &R)) || (st = ops::temp("ns_i", A.n, &I))) return st;
   double err = 100000.0;
   int i = 0;
   Sums s;
+  DMat cur = start;  // the current iterate, in start, out or scratch
   while (err > tol) {
-    if ((st = ops::mm(A, Ai, R, commuting, -1.0, 0.0, nullptr, 1.0, &s))) return st;
-    const double prev = err;
-    err = std::sqrt(s.fro2);
-    if (!std::isfinite(err)) {
-      set_error(ERR_NUMERIC, "Newton-Schulz: non-finite residual");
-      return ERR_NUMERIC;
+    bool grew = false;
+    {
+      ops::HoldOperand hold_cur(cur);  // an operand of both products
+      if ((st = ops::mm(A, cur, R, commuting, -1.0, 0.0, nullptr, 1.0, &s))) return st;
+      const double prev = err;
+      err = std::sqrt(s.fro2);
+      if (!std::isfinite(err)) {
+        set_error(ERR_NUMERIC, "Newton-Schulz: non-finite residual");
+        return ERR_NUMERIC;
+      }
+      grew = prev + 0.01 < err;
+      if (!grew) {
+        const DMat next = (cur.p == out.p) ? scratch : out;
+        if ((st = ops::mm(cur, R, next, commuting, 1.0, 1.0, &cur))) return st;
+        cur = next;
+      }
     }
-    if (prev + 0.01 < err) {
+    if (grew) {
+      if (cur.p != out.p && cur.p != scratch.p) {
+        if ((st = ops::copy(cur, out))) return st;
+        cur = out;
+      }
       if ((st = ops::identity(I))) return st;
-      if ((st = conjgrad(A, Ai, I, 0.00001, commuting, nullptr))) return st;
-    } else {
-      if ((st = ops::mm(Ai, R, T, commuting, 1.0, 1.0, &Ai))) return st;
-      if ((st = ops::copy(T, Ai))) return st;
+      if ((st = conjgrad(A, cur, I, 0.00001, commuting, nullptr))) return st;
     }
     ++i;
     if (i > 200) {
@@ -97,8 +112,22 @@ int newtonschulz(const DMat& A, DMat Ai, double tol, int* iters, bool commuting)
       return ERR_NOT_CONVERGED;
     }
   }
+  if (cur.p == scratch.p) {
+    std::swap(out, scratch);
+  } else if (cur.p != out.p) {
+    if ((st = ops::copy(cur, out))) return st;  // tol above the first residual
+  }
   if (iters) *iters = i;
   return OK;
+}
+
+// The same in place.
+int newtonschulz(const DMat& A, DMat Ai, double tol, int* iters, bool commuting) {
+  DMat out = Ai, scratch;
+  int st;
+  if ((st = ops::temp("ns_t", A.n, &scratch))) return st;
+  if ((st = newtonschulz_into(A, Ai, out, scratch, tol, iters, commuting))) return st;
+  return out.p == Ai.p ? OK : ops::copy(out, Ai);
 }
 
 // prg_pcg (src/prg_implicit_fermi_mod.F90:934-996): conjugate gradient for
@@ -197,10 +226,11 @@ int implicit_fermi(const DMat& H, DMat P, int nsteps, int k, double nocc, double
     set_error(ERR_ARG, "prg_implicit_fermi: nsteps out of range");
     return ERR_ARG;
   }
-  DMat P2, Y, AI, I;
+  DMat P2, Y, AI, I, scratch;
   int st;
   if ((st = ops::temp("if_p2", H.n, &P2)) || (st = ops::temp("if_y", H.n, &Y)) ||
-      (st = ops::temp("if_ai", H.n, &AI)) || (st = ops::temp("if_i", H.n, &I)))
+      (st = ops::temp("if_ai", H.n, &AI)) || (st = ops::temp("if_i", H.n, &I)) ||
+      (st = ops::temp("ns_t", H.n, &scratch)))
     return st;
   if (method == 1) {
     if ((st = ops::identity(AI)) || (st = ops::identity(I))) return st;
@@ -221,7 +251,7 @@ int implicit_fermi(const DMat& H, DMat P, int nsteps, int k, double nocc, double
         // level-1 CG inverse (tol 0.9) refined by Newton-Schulz at every level;
         // the reference comments the refinement out and then diverges
         if (i == 0 && (st = conjgrad(Y, AI, I, 0.9, true, nullptr))) return st;
-        if ((st = newtonschulz(Y, AI, tol, nullptr, true))) return st;
+        if ((st = newtonschulz_into(Y, AI, AI, scratch, tol, nullptr, true))) return st;
         if ((st = ops::mm(AI, P2, P, true))) return st;
       }
     }
@@ -472,9 +502,10 @@ int implicit_fermi_levels(const DMat& H, int nsteps, double mu, double beta, dou
     if ((st = ops::temp(("ifa_x" + std::to_string(i)).c_str(), H.n, &X[i]))) return st;
   for (int i = 0; i < nsteps; ++i)
     if ((st = ops::temp(("ifa_inv" + std::to_string(i)).c_str(), H.n, &Inv[i]))) return st;
-  DMat P2, Y, AI, I;
+  DMat P2, Y, AI, I, scratch;
   if ((st = ops::temp("if_p2", H.n, &P2)) || (st = ops::temp("if_y", H.n, &Y)) ||
-      (st = ops::temp("if_ai", H.n, &AI)) || (st = ops::temp("if_i", H.n, &I)))
+      (st = ops::temp("if_ai", H.n, &AI)) || (st = ops::temp("if_i", H.n, &I)) ||
+      (st = ops::temp("ns_t", H.n, &scratch)))
     return st;
   if ((st = ops::identity(AI)) || (st = ops::identity(I))) return st;
   const double cnst = beta / (4.0 * std::pow(2.0, nsteps));
@@ -483,9 +514,10 @@ int implicit_fermi_levels(const DMat& H, int nsteps, double mu, double beta, dou
     if ((st = ops::mm(X[i], X[i], P2, true))) return st;
     if ((st = ops::lin(P2, 2.0, &X[i], -2.0, 1.0, Y))) return st;
     if (i == 0 && (st = conjgrad(Y, AI, I, 0.9, true, nullptr))) return st;
-    if ((st = newtonschulz(Y, AI, tol, nullptr, true))) return st;
-    if ((st = ops::copy(AI, Inv[i]))) return st;
-    if ((st = ops::mm(AI, P2, X[i + 1], true))) return st;
+    // from the last level's inverse, which stays, into this level's
+    if ((st = newtonschulz_into(Y, i ? Inv[i - 1] : AI, Inv[i], scratch, tol, nullptr, true)))
+      return st;
+    if ((st = ops::mm(Inv[i], P2, X[i + 1], true))) return st;
   }
   return OK;
 }
@@ -505,10 +537,9 @@ int implicit_fermi_adjoint(const DMat& H, const DMat& A, DMat G, int nsteps, dou
   std::vector<DMat> X, Inv;
   int st;
   if ((st = implicit_fermi_levels(H, nsteps, mu, beta, tol, X, Inv))) return st;
-  DMat Gb, W, WF, U, Ut, V, T1, T2;
+  DMat Gb, W, WF, U, T1, T2;
   if ((st = ops::temp("ifa_gb", H.n, &Gb)) || (st = ops::temp("ifa_w", H.n, &W)) ||
       (st = ops::temp("ifa_wf", H.n, &WF)) || (st = ops::temp("ifa_u", H.n, &U)) ||
-      (st = ops::temp("ifa_ut", H.n, &Ut)) || (st = ops::temp("ifa_v", H.n, &V)) ||
       (st = ops::temp("ifa_t1", H.n, &T1)) || (st = ops::temp("ifa_t2", H.n, &T2)))
     return st;
   if ((st = ops::copy(A, Gb))) return st;
@@ -527,15 +558,10 @@ int implicit_fermi_adjoint(const DMat& H, const DMat& A, DMat G, int nsteps, dou
   for (int i = nsteps - 1; i >= 0; --i) {
     if ((st = ops::mm(Inv[i], Gb, W, false))) return st;          // W = Y^-1 Gb
     if ((st = ops::mm(W, X[i + 1], WF, false))) return st;        // W F
-    if ((st = ops::lin(W, 1.0, &WF, -2.0, 0.0, U))) return st;    // U = W - 2 W F
-    if ((st = ops::transpose(U, Ut))) return st;
-    if ((st = ops::lin(U, 0.5, &Ut, 0.5, 0.0, U))) return st;     // Us
-    if ((st = ops::mm(X[i], U, V, false))) return st;             // X Us
-    if ((st = ops::transpose(V, Ut))) return st;
-    if ((st = ops::lin(V, 1.0, &Ut, 1.0, 0.0, T1))) return st;    // X Us + Us X
-    if ((st = ops::transpose(WF, Ut))) return st;
-    if ((st = ops::lin(WF, 1.0, &Ut, 1.0, 0.0, T2))) return st;   // W F + (W F)^T
-    if ((st = ops::lin(T1, 1.0, &T2, 1.0, 0.0, Gb))) return st;
+    // Us = sym(W - 2 W F) and W F + (W F)^T in one pass
+    if ((st = ops::symmetrize_pair(W, WF, U, T2))) return st;
+    // Gb = X Us + Us X + W F + (W F)^T
+    if ((st = ops::mm2(X[i], U, U, X[i], Gb, true, 1.0, 1.0, &T2))) return st;
   }
   const double cnst = beta / (4.0 * std::pow(2.0, nsteps));
   if ((st = ops::lin(Gb, -cnst, nullptr, 0.0, 0.0, G))) return st;

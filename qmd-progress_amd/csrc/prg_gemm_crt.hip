@@ -1392,9 +1392,10 @@ int set_crt_config(int config) {
   return ERR_ARG;
 }
 
-// One operand that a caller promises not to change while held (the matrix of
-// a Newton-Schulz or CG solve): its residue planes and scale are formed once
-// and reused by every product that names it until the hold ends.
+// Operands that a caller promises not to change while held (the matrix and the
+// current iterate of a Newton-Schulz or CG solve): their residue planes and
+// scales are formed once and reused by every product that names them until
+// the hold ends.
 namespace {
 struct HeldOperand {
   const double* key = nullptr;
@@ -1402,21 +1403,32 @@ struct HeldOperand {
   bool valid = false;
   int np = 0, ld = 0;
 };
-HeldOperand g_held;
+HeldOperand g_held[2];
+const char* const kHeldPlanes[2] = {"crtg_planes_held", "crtg_planes_held2"};
+
+int held_slot(const double* p) {
+  for (int i = 0; i < 2; ++i)
+    if (g_held[i].depth > 0 && g_held[i].key == p) return i;
+  return -1;
+}
 }  // namespace
 
 void crt_hold_operand(const double* p) {
-  if (g_held.depth == 0) {
-    g_held.key = p;
-    g_held.valid = false;
-  }
-  if (g_held.key == p) ++g_held.depth;
+  int i = held_slot(p);
+  for (int j = 0; i < 0 && j < 2; ++j)
+    if (g_held[j].depth == 0) {
+      g_held[j].key = p;
+      g_held[j].valid = false;
+      i = j;
+    }
+  if (i >= 0) ++g_held[i].depth;
 }
 
 void crt_release_operand(const double* p) {
-  if (g_held.depth > 0 && g_held.key == p && --g_held.depth == 0) {
-    g_held.key = nullptr;
-    g_held.valid = false;
+  const int i = held_slot(p);
+  if (i >= 0 && --g_held[i].depth == 0) {
+    g_held[i].key = nullptr;
+    g_held[i].valid = false;
   }
 }
 
@@ -1439,19 +1451,19 @@ int crt_gemm(const DMat& A, const DMat& B, DMat C, double alpha, double beta, co
   const int nt = pld / TM;
   const int nb = nt * (nt + 1) / 2;
   const bool same = (A.p == B.p);
-  const bool held_a = g_held.depth > 0 && A.p == g_held.key;
-  const bool held_b = g_held.depth > 0 && B.p == g_held.key && !same;
+  const int ha = held_slot(A.p), hb = same ? -1 : held_slot(B.p);
   int st = OK;
-  int8_t* pa_planes = (int8_t*)workspace(held_a ? "crtg_planes_held" : "crtg_planes_a",
+  int8_t* pa_planes = (int8_t*)workspace(ha >= 0 ? kHeldPlanes[ha] : "crtg_planes_a",
                                          (size_t)np * plane, &st);
   int8_t* pb_planes = same ? nullptr
-                           : (int8_t*)workspace(held_b ? "crtg_planes_held" : "crtg_planes_b",
+                           : (int8_t*)workspace(hb >= 0 ? kHeldPlanes[hb] : "crtg_planes_b",
                                                 (size_t)np * plane, &st);
   int8_t* res = (int8_t*)workspace("crt_residues", (size_t)nb * np * kItemBytes, &st);
-  double* sc = (double*)workspace("crtg_scales", sizeof(double) * 6, &st);
+  double* sc = (double*)workspace("crtg_scales", sizeof(double) * 8, &st);
   double* npart = (double*)workspace("crtg_norm_part", sizeof(double) * 1024, &st);
   if (st) return st;
-  if ((held_a || held_b) && (g_held.np != np || g_held.ld != ld)) g_held.valid = false;
+  for (int h : {ha, hb})
+    if (h >= 0 && (g_held[h].np != np || g_held[h].ld != ld)) g_held[h].valid = false;
   const double* fold = fold_constants(np, &st);
   if (st) return st;
   const int4* items = item_list(nt, np, &st);
@@ -1467,16 +1479,21 @@ int crt_gemm(const DMat& A, const DMat& B, DMat C, double alpha, double beta, co
     PRG_HIP_CHECK(hipGetLastError());
     return OK;
   };
-  // scale slots: A at sc, B at sc + 2, the held operand at sc + 4
-  double* sa = held_a ? sc + 4 : sc;
-  double* sb = same ? sa : (held_b ? sc + 4 : sc + 2);
-  if (!(held_a && g_held.valid) && (st = scale_split(A, pa_planes, sa))) return st;
-  if (!same && !(held_b && g_held.valid) && (st = scale_split(B, pb_planes, sb))) return st;
-  if (held_a || held_b) {
-    g_held.valid = true;
-    g_held.np = np;
-    g_held.ld = ld;
-  }
+  // scale slots: A at sc, B at sc + 2, the held operands at sc + 4 and sc + 6
+  double* sa = ha >= 0 ? sc + 4 + 2 * ha : sc;
+  double* sb = same ? sa : (hb >= 0 ? sc + 4 + 2 * hb : sc + 2);
+  auto form = [&](const DMat& X, int8_t* planes, double* s, int h) -> int {
+    if (h >= 0 && g_held[h].valid) return OK;
+    const int e = scale_split(X, planes, s);
+    if (!e && h >= 0) {
+      g_held[h].valid = true;
+      g_held[h].np = np;
+      g_held[h].ld = ld;
+    }
+    return e;
+  };
+  if ((st = form(A, pa_planes, sa, ha))) return st;
+  if (!same && (st = form(B, pb_planes, sb, hb))) return st;
   ProductArgs pa;
   pa.planes[0] = pa_planes;
   pa.planes[1] = pa_planes;

@@ -519,9 +519,9 @@ int sp2_mixed_prepare(const DMat& x0, int prec) {
   return split_f16(x0, planes, planes + plane, bf16);
 }
 
-// One operand that a caller promises not to change while held (the matrix of
-// a Newton-Schulz or CG solve): its planes are formed once and reused by
-// every split product that names it until the hold ends.
+// Operands that a caller promises not to change while held (the matrix and the
+// current iterate of a Newton-Schulz or CG solve): their planes are formed
+// once and reused by every split product that names them until the hold ends.
 namespace {
 struct SplitHeld {
   const double* key = nullptr;
@@ -529,21 +529,32 @@ struct SplitHeld {
   bool valid = false;
   int ld = 0;
 };
-SplitHeld g_split_held;
+SplitHeld g_split_held[2];
+const char* const kSplitHeldPlanes[2] = {"splitg_planes_held", "splitg_planes_held2"};
+
+int split_held_slot(const double* p) {
+  for (int i = 0; i < 2; ++i)
+    if (g_split_held[i].depth > 0 && g_split_held[i].key == p) return i;
+  return -1;
+}
 }  // namespace
 
 void split_hold_operand(const double* p) {
-  if (g_split_held.depth == 0) {
-    g_split_held.key = p;
-    g_split_held.valid = false;
-  }
-  if (g_split_held.key == p) ++g_split_held.depth;
+  int i = split_held_slot(p);
+  for (int j = 0; i < 0 && j < 2; ++j)
+    if (g_split_held[j].depth == 0) {
+      g_split_held[j].key = p;
+      g_split_held[j].valid = false;
+      i = j;
+    }
+  if (i >= 0) ++g_split_held[i].depth;
 }
 
 void split_release_operand(const double* p) {
-  if (g_split_held.depth > 0 && g_split_held.key == p && --g_split_held.depth == 0) {
-    g_split_held.key = nullptr;
-    g_split_held.valid = false;
+  const int i = split_held_slot(p);
+  if (i >= 0 && --g_split_held[i].depth == 0) {
+    g_split_held[i].key = nullptr;
+    g_split_held[i].valid = false;
   }
 }
 
@@ -558,22 +569,24 @@ int split_gemm(const DMat& A, const DMat& B, DMat C, double alpha, double beta, 
   }
   const size_t plane = 2 * (size_t)ld * ld;  // bytes of one BF16 plane
   const bool same = (A.p == B.p);
-  const bool held_a = g_split_held.depth > 0 && A.p == g_split_held.key;
-  const bool held_b = g_split_held.depth > 0 && B.p == g_split_held.key && !same;
+  const int ha = split_held_slot(A.p), hb = same ? -1 : split_held_slot(B.p);
   int st = OK;
-  char* pa = (char*)workspace(held_a ? "splitg_planes_held" : "splitg_planes_a", 2 * plane, &st);
+  char* pa = (char*)workspace(ha >= 0 ? kSplitHeldPlanes[ha] : "splitg_planes_a", 2 * plane, &st);
   char* pb = same ? pa
-                  : (char*)workspace(held_b ? "splitg_planes_held" : "splitg_planes_b",
-                                     2 * plane, &st);
+                  : (char*)workspace(hb >= 0 ? kSplitHeldPlanes[hb] : "splitg_planes_b", 2 * plane,
+                                     &st);
   if (st) return st;
-  if ((held_a || held_b) && g_split_held.ld != ld) g_split_held.valid = false;
-  if (!(held_a && g_split_held.valid) && (st = split_f16(A, pa, pa + plane, true))) return st;
-  if (!same && !(held_b && g_split_held.valid) && (st = split_f16(B, pb, pb + plane, true)))
-    return st;
-  if (held_a || held_b) {
-    g_split_held.valid = true;
-    g_split_held.ld = ld;
-  }
+  auto form = [&](const DMat& X, char* planes, int h) -> int {
+    if (h >= 0 && g_split_held[h].valid && g_split_held[h].ld == ld) return OK;
+    const int e = split_f16(X, planes, planes + plane, true);
+    if (!e && h >= 0) {
+      g_split_held[h].valid = true;
+      g_split_held[h].ld = ld;
+    }
+    return e;
+  };
+  if ((st = form(A, pa, ha))) return st;
+  if (!same && (st = form(B, pb, hb))) return st;
   SplitGemmArgs g;
   g.ahi = pa;
   g.alo = pa + plane;

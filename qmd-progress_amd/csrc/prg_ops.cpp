@@ -10,6 +10,7 @@
 namespace prg {
 
 int transpose_kernel_launch(const DMat& A, DMat out);
+int symmetrize_pair_launch(const DMat& W, const DMat& F, DMat U, DMat S);
 int scale_cols_kernel_launch(const DMat& A, const double* d_f, DMat out);
 int scale_rows_kernel_launch(const DMat& A, const double* d_f, DMat out);
 int inv_diag_kernel_launch(const DMat& A, double* d_out);
@@ -185,6 +186,9 @@ int sums_of(const DMat& A, Sums* s) {
   return lin(A, 1.0, nullptr, 0.0, 0.0, T, s);
 }
 int transpose(const DMat& A, DMat out) { return transpose_kernel_launch(A, out); }
+int symmetrize_pair(const DMat& W, const DMat& F, DMat U, DMat S) {
+  return symmetrize_pair_launch(W, F, U, S);
+}
 int scale_cols(const DMat& A, const double* d_f, DMat out) {
   return scale_cols_kernel_launch(A, d_f, out);
 }

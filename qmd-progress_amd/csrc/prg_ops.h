@@ -25,8 +25,9 @@ void gemm_counters(double* products, double* alg_flops, double* exec_flops, bool
 int product_precision();
 int set_product_precision(int mode);
 
-// Scope during which A is not modified: int8 CRT products reuse its residue
-// planes (no effect on FP64 products).
+// Scope during which A is not modified: int8 CRT (BF16 split) products form its
+// residue (hi/lo) planes once and reuse them (no effect on FP64 products).  Up
+// to two operands at a time; a third is simply not held.
 struct HoldOperand {
   explicit HoldOperand(const DMat& A);
   ~HoldOperand();
@@ -55,6 +56,8 @@ int identity(DMat dst, double diag = 1.0);
 int sums_of(const DMat& A, Sums* s);
 // out = A^T (out must not alias A)
 int transpose(const DMat& A, DMat out);
+// U = sym(W - 2 F), S = F + F^T (neither may alias W or F)
+int symmetrize_pair(const DMat& W, const DMat& F, DMat U, DMat S);
 // out[:, j] = A[:, j] * f[j]  (f: device vector of length n)
 int scale_cols(const DMat& A, const double* d_f, DMat out);
 // out[i, :] = f[i] * A[i, :]  (f: device vector of length n)
