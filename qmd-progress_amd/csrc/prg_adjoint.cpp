@@ -16,6 +16,7 @@
 // self-adjoint, dL/dH for L = Tr(D A) equals that response with H1 = A.
 #include <cmath>
 #include <string>
+#include <utility>
 #include <vector>
 
 #include "prg_ops.h"
@@ -43,17 +44,21 @@ int sp2_adjoint(const DMat& H, const DMat& Gout, DMat grad, const int* pp, int i
   if ((st = ops::temp("adj_x", n, &X)) || (st = ops::temp("adj_y", n, &Y)) ||
       (st = ops::temp("adj_g", n, &G)) || (st = ops::temp("adj_s", n, &S)))
     return st;
-  // forward with checkpoints
+  // The updates are the products' epilogues: X_{k+1} = X^2 or 2 X - X^2, and
+  // G_k = S or 2 G - S, with S = X G + G X, each written to the next buffer.
+  auto step = [&](const DMat& x, DMat next, int sq) -> int {
+    return sq ? ops::mm(x, x, next, true) : ops::mm(x, x, next, true, -1.0, 2.0, &x);
+  };
+  // forward with checkpoints: step k is written straight to checkpoint
+  // (k + 1) / ckpt where one is due
   const double inv = 1.0 / (hi - lo);
-  if ((st = ops::lin(H, -inv, nullptr, 0.0, hi * inv, X))) return st;
-  for (int k = 0; k < iters; ++k) {
-    if (k % ckpt == 0 && (st = ops::copy(X, ckm(k / ckpt)))) return st;
-    if ((st = ops::mm(X, X, Y, true))) return st;
-    if (pp[k]) {
-      if ((st = ops::copy(Y, X))) return st;
-    } else {
-      if ((st = ops::lin(X, 2.0, &Y, -1.0, 0.0, X))) return st;
-    }
+  DMat cur = ckm(0);
+  if ((st = ops::lin(H, -inv, nullptr, 0.0, hi * inv, cur))) return st;
+  // (the last checkpoint's segment is recomputed below: X_iters is not needed)
+  for (int k = 0; k < (nck - 1) * ckpt; ++k) {
+    const DMat next = ((k + 1) % ckpt == 0) ? ckm((k + 1) / ckpt) : (cur.p == X.p ? Y : X);
+    if ((st = step(cur, next, pp[k]))) return st;
+    cur = next;
   }
   // backward
   if ((st = ops::lin(Gout, 2.0, nullptr, 0.0, 0.0, G))) return st;
@@ -66,27 +71,19 @@ int sp2_adjoint(const DMat& H, const DMat& Gout, DMat grad, const int* pp, int i
   for (int k = iters - 1; k >= 0; --k) {
     const int c = k / ckpt;
     if (c * ckpt != seg_start) {
-      // recompute X_{c*ckpt} .. X_{min(iters, (c+1)*ckpt) - 1} into the segment buffer
+      // recompute X_{c*ckpt + 1} .. X_{min(iters, (c+1)*ckpt) - 1} into the
+      // segment buffer
       seg_start = c * ckpt;
-      if ((st = ops::copy(ckm(c), segm(0)))) return st;
-      for (int j = 1; j < ckpt && seg_start + j < iters; ++j) {
-        const DMat prev = segm(j - 1);
-        if ((st = ops::mm(prev, prev, Y, true))) return st;
-        if (pp[seg_start + j - 1]) {
-          if ((st = ops::copy(Y, segm(j)))) return st;
-        } else {
-          if ((st = ops::lin(prev, 2.0, &Y, -1.0, 0.0, segm(j)))) return st;
-        }
-      }
+      for (int j = 1; j < ckpt && seg_start + j < iters; ++j)
+        if ((st = step(j == 1 ? ckm(c) : segm(j - 1), segm(j), pp[seg_start + j - 1]))) return st;
     }
-    const DMat Xk = segm(k - seg_start);
-    // S = X_k G + G X_k
-    if ((st = ops::mm2(Xk, G, G, Xk, S, sym))) return st;
-    if (pp[k]) {
-      if ((st = ops::copy(S, G))) return st;
-    } else {
-      if ((st = ops::lin(G, 2.0, &S, -1.0, 0.0, G))) return st;
-    }
+    const DMat Xk = (k == seg_start) ? ckm(c) : segm(k - seg_start);
+    if (pp[k])
+      st = ops::mm2(Xk, G, G, Xk, S, sym);
+    else
+      st = ops::mm2(Xk, G, G, Xk, S, sym, -1.0, 2.0, &G);
+    if (st) return st;
+    std::swap(G, S);
   }
   return ops::lin(G, -inv, nullptr, 0.0, 0.0, grad);
 }

@@ -63,14 +63,13 @@ struct GemmArgs {
 template <typename S, int FUSE, int PLACE>
 __device__ __forceinline__ void gemm_finish(const GemmArgs& g, d4 (&acc)[S::MB][S::NB],
                                             int ks, int r0, int c0, double* lds,
-                                            double (&sums)[4]) {
+                                            const f64tile::Entries<S>& cin, double (&sums)[4]) {
   const int ld = g.ld;
   f64tile::finish_tile<S>(acc, ks, lds, [&](auto grp, auto& y) {
     const int r = ks;
     constexpr int G = decltype(grp)::value, W = f64tile::kWidth<S, G>;
     const int col0 = f64tile::entry_col<S, G>(c0, r);
-    double cin[S::MB][W], e[S::MB][W];
-    if (FUSE & 1) f64tile::load_entries<S, G, W>(g.Cin, ld, r0, c0, r, cin);
+    double e[S::MB][W];
     if (FUSE & 2) f64tile::load_entries<S, G, W>(g.dotE, ld, r0, c0, r, e);
 #pragma unroll
     for (int w = 0; w < W; ++w) {
@@ -79,7 +78,7 @@ __device__ __forceinline__ void gemm_finish(const GemmArgs& g, d4 (&acc)[S::MB][
       for (int m = 0; m < S::MB; ++m) {
         const int row = f64tile::entry_row<S>(r0, m);
         double v = y[m][w] * g.alpha;
-        if (FUSE & 1) v += g.beta * cin[m][w];
+        if (FUSE & 1) v += g.beta * cin.v[G][m][w];
         const bool diag = PLACE != 1 && (row == col);
         if (PLACE != 1) v += (diag && row < g.n) ? g.gamma : 0.0;
         y[m][w] = v;
@@ -112,21 +111,24 @@ __global__ __launch_bounds__(S::NT, 2) void gemm_kernel(GemmArgs g) {
   const int t = xcd_remap(blockIdx.x, gridDim.x);
   int I, J;
   if (g.sym) sym_tile_banded<kBand>(t, g.nt, I, J); else full_tile(t, g.nt, I, J);
-  const int ks = f64tile::k_wave(), r0 = I * S::TM, c0 = J * S::TM;
+  const int ks = f64tile::k_wave(), r0 = I * S::TM, c0 = J * S::TM, ld = g.ld;
   int first, count;
   f64tile::k_share<S>(g.kdim / S::CK, ks, first, count);
   d4 acc[S::MB][S::NB];
   zero<S>(acc);
   f64tile::WaveProduct<S, BT> product;
   product.start(g.A[0], g.B[0], g.A[1], g.B[1], g.npair, g.ld, r0, c0, first * S::CK, count);
-  product.run(acc, [] {});
+  f64tile::Entries<S> cin;
+  product.run(acc, [&] {
+    if (FUSE & 1) cin.load(g.Cin, ld, r0, c0, ks);
+  });
   double sums[4] = {0.0, 0.0, 0.0, 0.0};
   if (!g.sym)
-    gemm_finish<S, FUSE, 0>(g, acc, ks, r0, c0, lds, sums);
+    gemm_finish<S, FUSE, 0>(g, acc, ks, r0, c0, lds, cin, sums);
   else if (I != J)
-    gemm_finish<S, FUSE, 1>(g, acc, ks, r0, c0, lds, sums);
+    gemm_finish<S, FUSE, 1>(g, acc, ks, r0, c0, lds, cin, sums);
   else
-    gemm_finish<S, FUSE, 2>(g, acc, ks, r0, c0, lds, sums);
+    gemm_finish<S, FUSE, 2>(g, acc, ks, r0, c0, lds, cin, sums);
   if (g.part) block_store4<S::NT>(sums, g.part + 4 * (size_t)t);
 }
 
