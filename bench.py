@@ -322,22 +322,26 @@ def main():
     print(json.dumps(out))
 
 
-def batched_executed_flops(m, panel):
+def batched_executed_flops(n, panel, rows=None):
     """MFMA flops one iteration of the batched SP2 kernel executes on a part
-    of padded size m: the upper-triangle tiles over panels of `panel` (the
-    last one 64 wide when panel does not divide m); a diagonal tile leaves
+    of n rows: the upper-triangle tiles (all, or those that start within the
+    first `rows` rows) over panels of `panel`.  48-wide panels cover n and
+    their K ends there; the staged tiles cover the size padded to 64 (the last
+    panel 64 wide when `panel` does not divide it), and a diagonal tile leaves
     its strictly lower quadrant to the mirror write (3/4 of its product)."""
-    widths = [min(panel, m - s) for s in range(0, m, panel)]
+    m = n if panel == 48 else max(64, ((n + 63) // 64) * 64)
+    widths = [panel if panel == 48 else min(panel, m - s) for s in range(0, m, panel)]
     f = 0.0
     for b, wb in enumerate(widths):
         for a in range(b + 1):
-            wa = widths[a]
-            f += 2.0 * wa * wb * m * (0.75 if a == b else 1.0)
+            if rows is None or a * panel < rows:
+                f += 2.0 * widths[a] * wb * m * (0.75 if a == b and panel != 48 else 1.0)
     return f
 
 
-def batched_tile_count(m, panel):
-    """Upper-triangle tiles of a part of padded size m over panels of `panel`."""
+def batched_tile_count(n, panel):
+    """Upper-triangle tiles of a part of n rows over panels of `panel`."""
+    m = n if panel == 48 else max(64, ((n + 63) // 64) * 64)
     k = len(range(0, m, panel))
     return k * (k + 1) // 2
 
@@ -419,8 +423,9 @@ def graph_bench(args, P, torch, np):
     dev_s = sum(times) / len(times)
     alg = sum(2.0 * float(m) ** 3 for m in ls) * it
     panel, depth, kslab, launch = P.subgraph_config()
-    mpad = [max(64, ((m + 63) // 64) * 64) for m in ls]
-    executed = sum(batched_executed_flops(m, panel) for m in mpad) * it
+    # the last iteration computes the tiles that hold core rows only
+    executed = sum(batched_executed_flops(m, panel) * (it - 1) +
+                   batched_executed_flops(m, panel, c) for m, c in zip(ls, core))
     if args.graph_precision != "fp64":
         executed *= 3.0  # hi.hi, hi.lo and lo.hi 16-bit products per tile
     loop_s = last[1] * 1e-3
@@ -465,7 +470,7 @@ def graph_bench(args, P, torch, np):
         "accuracy_vs_dense": {"fro": err, "rel_fro": rel, "trace_err": tr_err,
                               "band_energy_err": eb_err},
         "tiles": {"panel": panel, "prefetch_slabs": depth, "k_slab": kslab,
-                  "count": sum(batched_tile_count(m, panel) for m in mpad),
+                  "count": sum(batched_tile_count(m, panel) for m in ls),
                   "launch": {0: "eager", 1: "captured hipGraph", 2: "hipGraph replay"}[launch]},
         "roofline": {"bound": "mfma",
                      "kernel": (f"batched_sp2_kernel (FP64 MFMA, {panel}-wide panels)"

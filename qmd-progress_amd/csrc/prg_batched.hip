@@ -8,13 +8,14 @@
 // are packed one after another in HBM, each zero-padded to a multiple of 64.
 // The work list holds the upper-triangle tiles of every part, largest parts
 // first; consecutive workgroups (per XCD) walk consecutive tiles, so a part's
-// panels stay in one XCD's L2.  A part is cut into panels of 64 or of 128
-// (the last one 64 wide when the size is an odd multiple of 64), giving
-// 64 x 64, 128 x 64 and 128 x 128 tiles; the panel width is picked per batch
-// by timing both (prg_graph.cpp).  Each tile runs the FP64 MFMA product and
+// panels stay in one XCD's L2.  A part is cut into panels of 48, of 64 or
+// of 128 (the last one 64 wide when the size is an odd multiple of 64; 48-wide
+// ones may overhang), giving 48 x 48, 64 x 64, 128 x 64 and 128 x 128 tiles;
+// the panel width is picked per batch (prg_graph.cpp).  Each tile runs the FP64 MFMA product and
 // the fused update X <- X + (1 - 2 pp)(X - X^2) with the core-row sum of
 // (X - X^2)^2 for vv.
 #include "prg_graph.h"
+#include "prg_f64_tile.h"
 #include "prg_lds_dma.h"
 #include "prg_tile.h"
 
@@ -46,7 +47,16 @@ struct BatchArgs {
   const void* lo;
   void* hin;
   void* lon;
+  // the last iteration: only the core rows of X are read after it, so only
+  // the tiles that hold some of them are computed
+  int core_only;
 };
+
+__device__ __forceinline__ bool tile_wanted(const BatchArgs& g, int t, const int4& tl) {
+  if (!g.core_only || tl.y < g.parts[tl.x].core) return true;
+  if (threadIdx.x == 0) g.part_sums[t] = 0.0;
+  return false;
+}
 
 // One TM x TN tile of X^2 (rows r0.., columns c0..) of one part and its fused
 // SP2 update.  Four waves (2 x 2), each (TM/2) x (TN/2) = (TM/32) x (TN/32)
@@ -184,6 +194,7 @@ __global__ __launch_bounds__(NT, WIDE ? 2 : 4) void batched_sp2_kernel(BatchArgs
       if (k >= count) break;
       const int t = first + k;
       const int4 tl = g.tiles[t];
+      if (!tile_wanted(g, t, tl)) continue;
       if constexpr (WIDE) {
         if (tl.w == 3)
           sp2_tile<128, 128, PF, BK>(g, t, tl, smem);
@@ -194,6 +205,75 @@ __global__ __launch_bounds__(NT, WIDE ? 2 : 4) void batched_sp2_kernel(BatchArgs
       } else {
         sp2_tile<64, 64, PF, BK>(g, t, tl, smem);
       }
+    }
+  }
+}
+
+// The same queues over 48 x 48 tiles with operands straight to registers and K
+// split over the workgroup's four waves (prg_f64_tile.h): no staging and no
+// barrier in the main loop, two workgroups per CU, the next ticket fetched
+// under the product.  Bound by the matrix cores and the last tiles of a queue;
+// 16 parts of 1151-1712 rows take 1.31 ms per iteration, 1.42 with the staged
+// 64 x 64 tiles; a last iteration computes its core rows' tiles only.
+__global__ __launch_bounds__(NT, 2) void batched_sp2_direct_kernel(BatchArgs g) {
+  typedef f64tile::S48 S;
+  __shared__ double lds[S::kLdsDoubles];
+  __shared__ int s_ticket;
+  const int home = blockIdx.x & 7, ks = f64tile::k_wave();
+  const double ca = g.sigma ? 1.0 : -1.0, cb = g.sigma ? 0.0 : 2.0;
+  for (int q = 0; q < 8; ++q) {
+    const int qi = (home + q) & 7;
+    const int begin = g.queue_off[qi], size = g.queue_off[qi + 1] - begin;
+    int ticket = 0;
+    if (threadIdx.x == 0) ticket = atomicAdd(&g.tickets[qi], 1);
+    for (;;) {
+      __syncthreads();  // every thread has read the previous ticket and lds
+      if (threadIdx.x == 0) s_ticket = ticket;
+      __syncthreads();
+      const int k = __builtin_amdgcn_readfirstlane(s_ticket);
+      if (k >= size) break;
+      // the next ticket arrives under this tile's product
+      if (threadIdx.x == 0) ticket = atomicAdd(&g.tickets[qi], 1);
+      const int t = begin + k;
+      const int4 tl = g.tiles[t];
+      if (!tile_wanted(g, t, tl)) continue;
+      const PartDesc pd = g.parts[tl.x];
+      const int m = pd.m, core = pd.core, r0 = tl.y, c0 = tl.z;
+      const double* X = g.x + pd.offset;
+      double* Xn = g.xn + pd.offset;
+      // the rows and columns past n are zero: K ends at n's chunk
+      int first, count;
+      f64tile::k_share<S>((pd.n + S::CK - 1) / S::CK, ks, first, count);
+      f64tile::d4 acc[S::MB][S::NB];
+#pragma unroll
+      for (int a = 0; a < S::MB; ++a)
+#pragma unroll
+        for (int b = 0; b < S::NB; ++b) acc[a][b] = f64tile::d4{0.0, 0.0, 0.0, 0.0};
+      f64tile::WaveProduct<S, false> product;
+      product.start(X, X, X, X, 1, m, r0, c0, first * S::CK, count);
+      f64tile::Entries<S> xs;
+      product.run(acc, [&] { xs.load(X, m, r0, c0, ks); });
+      const bool mirror = (r0 != c0);
+      double sum[1] = {0.0};
+      f64tile::finish_tile<S>(acc, ks, lds, [&](auto grp, auto& y) {
+        constexpr int G = decltype(grp)::value, W = f64tile::kWidth<S, G>;
+        const int col0 = f64tile::entry_col<S, G>(c0, ks);
+#pragma unroll
+        for (int w = 0; w < W; ++w)
+#pragma unroll
+          for (int a = 0; a < S::MB; ++a) {
+            const int row = f64tile::entry_row<S>(r0, a), col = col0 + w;
+            const double x = xs.v[G][a][w];
+            // rows and columns past the block repeat its last ones
+            const double yv = (row < m && col < m) ? y[a][w] : 0.0;
+            const double d = x - yv;
+            sum[0] += ((row < core ? 1.0 : 0.0) + (mirror && col < core ? 1.0 : 0.0)) * d * d;
+            y[a][w] = fma(cb, x, ca * yv);
+          }
+        f64tile::store_entries<S, G, W>(Xn, m, r0, c0, ks, y);
+        if (mirror) f64tile::store_mirrored<S, G, W>(Xn, m, r0, c0, ks, y);
+      });
+      block_store_partials<1>(sum, g.part_sums + t);
     }
   }
 }
@@ -504,6 +584,7 @@ __global__ __launch_bounds__(NT, 2) void batched_split_wide_kernel(BatchArgs g) 
       if (k >= count) break;
       const int t = first + k;
       const int4 tl = g.tiles[t];
+      if (!tile_wanted(g, t, tl)) continue;
       if (tl.w == 3)
         split_tile_wide<T, 128, 128>(g, t, tl, smem);
       else if (tl.w == 1)
@@ -732,6 +813,7 @@ __global__ __launch_bounds__(RNT, 1) void batched_split_ring_kernel(BatchArgs g)
       if (k >= count) break;
       const int t = first + k;
       const int4 tl = g.tiles[t];
+      if (!tile_wanted(g, t, tl)) continue;
       if (tl.w == 3)
         split_tile_ring<T, 128, 128>(g, t, tl, ring, stage);
       else if (tl.w == 1)
@@ -759,7 +841,9 @@ __global__ __launch_bounds__(NT, 4) void batched_split_kernel(BatchArgs g) {
       const int k = s_ticket;
       if (k >= count) break;
       const int t = first + k;
-      split_tile<T>(g, t, g.tiles[t], smem);
+      const int4 tl = g.tiles[t];
+      if (!tile_wanted(g, t, tl)) continue;
+      split_tile<T>(g, t, tl, smem);
     }
   }
 }
@@ -798,6 +882,7 @@ BatchKernel batch_kernel(const BatchPlan& p) {
                           : batched_split_ring_kernel<_Float16>;
     return nullptr;
   }
+  if (p.direct) return batched_sp2_direct_kernel;
   if (p.wide) return (p.depth == 1 && p.kslab == 16) ? batched_sp2_kernel<true, 1, 16> : nullptr;
   if (p.kslab == 32) return p.depth == 1 ? batched_sp2_kernel<false, 1, 32> : nullptr;
   if (p.kslab == 16)
@@ -974,8 +1059,9 @@ int batched_gather(const DMat& H, const BatchPlan& plan, double* x, double minev
 }
 
 int batched_step(const BatchPlan& plan, const double* x, double* xn, int sigma, double* d_part,
-                 int* d_tickets, int parity) {
+                 int* d_tickets, int parity, bool last) {
   BatchArgs g;
+  g.core_only = last ? 1 : 0;
   g.x = x;
   g.xn = xn;
   g.hi = plan.planes[2 * parity];

@@ -123,9 +123,9 @@ int make_plan(const prg_graph_partitioning_t* gp, HostPlan* hp, BatchPlan* plan)
 }
 
 // Upper-triangle tiles (part, first row, first column, shape) of every part
-// over panels of width `panel` (64 or 128); the last panel of a part is 64
+// over panels of width `panel` (48, 64 or 128); the last panel of a part is 64
 // wide when 128 does not divide its size, so the shapes are 128 x 128
-// (code 3), 128 x 64 (1) and 64 x 64 (0).  The parts are dealt to 8 queues,
+// (code 3), 128 x 64 (1) and 64 x 64 (0); 48-wide panels may overhang it.  The parts are dealt to 8 queues,
 // one per XCD, largest work first to the least loaded queue (work of a tile:
 // rows x columns x m); a queue lists its parts' tiles part by part, column
 // by column.  off[q] is the first tile of queue q, off[8] the total.
@@ -140,18 +140,25 @@ TileQueues make_tiles(const HostPlan& hp, int panel) {
   std::vector<double> work(np, 0.0);
   std::vector<int> start, width;
   for (int q = 0; q < np; ++q) {
-    const int m = hp.parts[q].m;
+    // 48-wide panels cover the n rows that are not padding (their kernel
+    // reads no others), the staged tiles all m
+    const int m = panel == 48 ? hp.parts[q].n : hp.parts[q].m;
     start.clear();
     width.clear();
     for (int s = 0; s < m; s += panel) {
       start.push_back(s);
       width.push_back(std::min(panel, m - s));
     }
-    for (size_t b = 0; b < start.size(); ++b)
-      for (size_t a = 0; a <= b; ++a) {
-        per[q].push_back(int4{q, start[a], start[b], (width[a] == 128 ? 1 : 0) | (width[b] == 128 ? 2 : 0)});
-        work[q] += (double)width[a] * width[b] * m;
-      }
+    // 48-wide panels: in bands of 8 columns, row by row, so that the tiles an
+    // XCD runs at a time form blocks that share panels both ways
+    const size_t band = panel == 48 ? 8 : 1;
+    for (size_t b0 = 0; b0 < start.size(); b0 += band)
+      for (size_t a = 0; a < std::min(b0 + band, start.size()); ++a)
+        for (size_t b = std::max(a, b0); b < std::min(b0 + band, start.size()); ++b) {
+          per[q].push_back(
+              int4{q, start[a], start[b], (width[a] == 128 ? 1 : 0) | (width[b] == 128 ? 2 : 0)});
+          work[q] += (double)width[a] * width[b] * m;
+        }
   }
   std::vector<int> order(np);
   for (int q = 0; q < np; ++q) order[q] = q;
@@ -175,11 +182,12 @@ TileQueues make_tiles(const HostPlan& hp, int panel) {
 int upload_tiles(const TileQueues& tq, int panel, BatchPlan* plan) {
   int st = OK;
   plan->wide = panel == 128 ? 1 : 0;
+  plan->direct = panel == 48 ? 1 : 0;
   plan->ntiles = (int)tq.tiles.size();
-  plan->d_tiles = (int4*)workspace(panel == 128 ? "gp_tiles128" : "gp_tiles64",
+  const std::string suffix = std::to_string(panel);
+  plan->d_tiles = (int4*)workspace(("gp_tiles" + suffix).c_str(),
                                    sizeof(int4) * std::max<size_t>(1, tq.tiles.size()), &st);
-  plan->d_queue_off =
-      (int*)workspace(panel == 128 ? "gp_qoff128" : "gp_qoff64", sizeof(int) * 9, &st);
+  plan->d_queue_off = (int*)workspace(("gp_qoff" + suffix).c_str(), sizeof(int) * 9, &st);
   if (st) return st;
   PRG_HIP_CHECK(hipMemcpyAsync(plan->d_tiles, tq.tiles.data(), sizeof(int4) * tq.tiles.size(),
                                hipMemcpyHostToDevice, stream()));
@@ -188,21 +196,44 @@ int upload_tiles(const TileQueues& tq, int panel, BatchPlan* plan) {
   return OK;
 }
 
-// Kernel configuration per batch: the tile panel width (64 or 128), the
+// Kernel configuration per batch: the tile panel width (48, 64 or 128), the
 // number of K slabs prefetched ahead (1 or 2) and the slab depth (16 or 32);
-// the compiled combinations are the candidates below.  PRG_BATCH_TILE,
-// PRG_BATCH_DEPTH and PRG_BATCH_KSLAB restrict them; the remaining ones are
-// timed on the batch itself (one untimed and three timed iterations each on
-// the gathered first iterate, results discarded) and the fastest is kept for
-// every later call with the same padded part sizes and restrictions.
+// the compiled combinations are the candidates below.  FP64 products take
+// 48/1/16 or 64/1/16 by rule (staged_is_faster): timing four candidates on
+// every new set of part sizes cost 16 iterations, as much as the loop itself.
+// PRG_BATCH_TILE, PRG_BATCH_DEPTH and PRG_BATCH_KSLAB restrict the candidates
+// instead, and what they leave (as the split-precision ones) is timed on the
+// batch itself (one untimed and three timed iterations each on the gathered
+// first iterate, results discarded) and the fastest is kept for every later
+// call with the same padded part sizes and restrictions.
 struct BatchConfig {
   int panel = 0, depth = 0, kslab = 0;
 };
-constexpr BatchConfig kCandidates[] = {{64, 1, 16}, {64, 2, 16}, {64, 1, 32}, {128, 1, 16}};
+constexpr BatchConfig kCandidates[] = {
+    {48, 1, 16}, {64, 1, 16}, {64, 2, 16}, {64, 1, 32}, {128, 1, 16}};
 // split-precision products: 64 x 64 tiles (64-deep slabs), 128-wide panels
 // (32-deep slabs through registers), or 128-wide panels with the slabs copied
 // into a 4-slot LDS ring (depth 4)
 constexpr BatchConfig kSplitCandidates[] = {{64, 1, 64}, {128, 1, 32}, {128, 4, 32}};
+
+// Whether a batch's FP64 products take less time on staged 64-wide tiles than
+// on 48-wide ones.  A 48-wide tile's multiply-add takes 0.97 of the other's
+// time once both fill the chip (twenty iterations: 124 parts of 640 rows 13.4
+// against 13.1 ms, 21 of 1000 8.2 / 9.1, 12 of 1500 14.8 / 15.6), so there
+// the padding decides: 2304 parts of 128 rows (3 panels against 2) take 6.1
+// against 5.4 ms.  Where the 64-wide tiles are fewer than two rounds of their
+// 4 workgroups per CU, the 48-wide ones win whatever the padding: 216 parts of
+// 128 rows 1.5 / 2.1 ms, 481 of 64 1.4 / 2.1, 70 of 320 2.1 / 2.8.
+bool staged_is_faster(const HostPlan& hp, size_t tiles64) {
+  if (tiles64 < 2 * 4 * 256) return false;
+  double direct = 0.0, staged = 0.0;
+  for (const PartDesc& d : hp.parts) {
+    const double t48 = (d.n + 47) / 48, t64 = d.m / 64;
+    direct += t48 * (t48 + 1) * 48 * 48 * d.n;
+    staged += t64 * (t64 + 1) * 64 * 64 * d.m;
+  }
+  return staged < 0.97 * direct;
+}
 
 std::map<std::pair<uint64_t, int>, BatchConfig>& config_cache() {
   static std::map<std::pair<uint64_t, int>, BatchConfig> c;
@@ -272,7 +303,7 @@ int enqueue_loop(const BatchPlan& plan, double* x0, double* x1, const int* pp, i
   double* nxt = x1;
   for (int it = 0; it < iters && !st; ++it) {
     st = batched_step(plan, cur, nxt, pp[it] != 0, d_part + (size_t)it * plan.ntiles,
-                      d_tickets + 8 * it, it & 1);
+                      d_tickets + 8 * it, it & 1, it == iters - 1);
     const double* t = cur;
     cur = nxt;
     nxt = const_cast<double*>(t);
@@ -292,7 +323,7 @@ int run_loop(const BatchPlan& plan, double* x0, double* x1, const int* pp, int i
                                (uint64_t)(uintptr_t)d_part,       (uint64_t)(uintptr_t)d_vv,
                                (uint64_t)(uintptr_t)d_tickets,    (uint64_t)(uintptr_t)plan.d_parts,
                                (uint64_t)(uintptr_t)plan.d_tiles, (uint64_t)(uintptr_t)plan.d_queue_off,
-                               (uint64_t)plan.ntiles,             (uint64_t)plan.wide,
+                               (uint64_t)plan.ntiles,             (uint64_t)(plan.wide + 2 * plan.direct),
                                (uint64_t)plan.depth,              (uint64_t)plan.grid,
                                (uint64_t)plan.kslab,
                                (uint64_t)plan.split,
@@ -352,7 +383,8 @@ int subgraph_sp2_loop(const DMat& H, DMat rho, prg_graph_partitioning_t* gp) {
   const size_t off = plan.total;
   const int iters = gp->maxIter;
   const TileQueues tiles64 = make_tiles(hp, 64);
-  const size_t maxtiles = tiles64.tiles.size();  // the 64-wide tiling has the most tiles
+  const TileQueues tiles48 = make_tiles(hp, 48);
+  const size_t maxtiles = std::max(tiles48.tiles.size(), tiles64.tiles.size());
   double* x0 = (double*)workspace("gp_x0", sizeof(double) * off, &st);
   double* x1 = (double*)workspace("gp_x1", sizeof(double) * off, &st);
   // iters x ntiles loop partials and iters x 8 queue tickets, + one slice each
@@ -427,10 +459,17 @@ int subgraph_sp2_loop(const DMat& H, DMat rho, prg_graph_partitioning_t* gp) {
   if (const char* e = std::getenv("PRG_BATCH_DEPTH")) force.depth = std::atoi(e);
   if (const char* e = std::getenv("PRG_BATCH_KSLAB")) force.kslab = std::atoi(e);
   std::vector<BatchConfig> cand;
-  for (const BatchConfig& c : kCandidates)
-    if ((!force.panel || c.panel == force.panel) && (!force.depth || c.depth == force.depth) &&
-        (!force.kslab || c.kslab == force.kslab))
-      cand.push_back(c);
+  if (force.panel || force.depth || force.kslab) {
+    for (const BatchConfig& c : kCandidates)
+      if ((!force.panel || c.panel == force.panel) && (!force.depth || c.depth == force.depth) &&
+          (!force.kslab || c.kslab == force.kslab))
+        cand.push_back(c);
+  } else {
+    cand.push_back(staged_is_faster(hp, tiles64.tiles.size()) ? kCandidates[1] : kCandidates[0]);
+  }
+  auto tiles_of = [&](int panel) -> TileQueues {
+    return panel == 128 ? make_tiles(hp, 128) : panel == 48 ? tiles48 : tiles64;
+  };
   if (cand.empty()) {
     set_error(ERR_ARG, "PRG_BATCH_TILE / PRG_BATCH_DEPTH / PRG_BATCH_KSLAB: no compiled batched "
                        "SP2 kernel has this configuration");
@@ -439,16 +478,17 @@ int subgraph_sp2_loop(const DMat& H, DMat rho, prg_graph_partitioning_t* gp) {
   const auto key =
       std::make_pair(size_signature(hp), (force.panel * 4 + force.depth) * 64 + force.kslab);
   BatchConfig cfg = cand[0];
-  auto hit = config_cache().find(key);
+  auto hit = config_cache().end();
+  if (cand.size() > 1) hit = config_cache().find(key);
   if (hit != config_cache().end()) {
     cfg = hit->second;
   } else if (cand.size() > 1) {
     if ((st = batched_gather(H, plan, x0, gp->mineval, gp->maxeval))) return st;
-    const TileQueues tiles128 = make_tiles(hp, 128);
     float best = 0.f;
     for (size_t k = 0; k < cand.size(); ++k) {
       const BatchConfig& c = cand[k];
-      if ((st = upload_tiles(c.panel == 128 ? tiles128 : tiles64, c.panel, &plan))) return st;
+      const TileQueues tq = tiles_of(c.panel);
+      if ((st = upload_tiles(tq, c.panel, &plan))) return st;
       plan.depth = c.depth;
       plan.kslab = c.kslab;
       float ms = 0.f;
@@ -461,10 +501,10 @@ int subgraph_sp2_loop(const DMat& H, DMat rho, prg_graph_partitioning_t* gp) {
         cfg = c;
       }
     }
+    config_cache()[key] = cfg;
   }
-  config_cache()[key] = cfg;
-  if ((st = upload_tiles(cfg.panel == 128 ? make_tiles(hp, 128) : tiles64, cfg.panel, &plan)))
-    return st;
+  const TileQueues tq = tiles_of(cfg.panel);
+  if ((st = upload_tiles(tq, cfg.panel, &plan))) return st;
   plan.depth = cfg.depth;
   plan.kslab = cfg.kslab;
   if ((st = batched_slots(&plan))) return st;

@@ -19,6 +19,7 @@ struct BatchPlan {
   int nparts = 0;
   int ntiles = 0;
   int wide = 0;              // 1: tiles of 128-wide panels (see batched_sp2_kernel)
+  int direct = 0;            // 1: 48 x 48 tiles, operands to registers (batched_sp2_direct_kernel)
   int depth = 1;             // K slabs prefetched ahead (1 or 2)
   int kslab = 16;            // K slab depth (16 or 32)
   int grid = 0;              // workgroups of the persistent batched SP2 launch
@@ -43,9 +44,10 @@ int batched_gather(const DMat& H, const BatchPlan& plan, double* x, double minev
 // One SP2 iteration of every part: xn from x, per-tile vv partials in
 // d_part; d_tickets: 8 queue counters, zero before the launch.  Split plans:
 // parity selects the planes of x (planes[2 parity], [2 parity + 1]); those of
-// xn are the others.
+// xn are the others.  last: nothing but the core rows of xn is read
+// afterwards (and nothing else is computed).
 int batched_step(const BatchPlan& plan, const double* x, double* xn, int sigma, double* d_part,
-                 int* d_tickets, int parity = 0);
+                 int* d_tickets, int parity = 0, bool last = false);
 // hi / lo planes 0 and 1 of a split plan from the packed FP64 x
 int batched_split_prepare(const BatchPlan& plan, const double* x);
 // whether a kernel is compiled for plan's wide / depth / kslab
