@@ -54,9 +54,7 @@ struct Split<__bf16> {
 
 constexpr int BM = 128, NT = 256;
 constexpr int KB = 32;                 // halves of K per slab and per plane block
-constexpr int kPanel = BM * KB * 2;    // bytes of one operand plane's slab
-constexpr int kSlab = 4 * kPanel;      // A hi, A lo, B hi, B lo
-constexpr int kRing = 2 * kSlab;       // two slabs: 64 KB, two workgroups per CU
+constexpr int kRing = 64 * 1024;       // the slabs in LDS: two workgroups per CU
 
 // Planes are stored in blocks of 32 columns, element (r, k) at
 // (k / 32) 32 ld + 32 r + k % 32: the 128 rows of a slab are 8 KB in one piece.
@@ -64,10 +62,11 @@ __device__ __forceinline__ size_t plane_at(int r, int k, int ld) {
   return (size_t)(k >> 5) * KB * ld + (size_t)r * KB + (k & 31);
 }
 
-// One 128 x 128 tile of A B (both symmetric, by their planes) over the whole
-// K: four waves in a 2 x 2 grid of 64 x 64.  The slabs are copied global ->
-// LDS directly (dma16), the next one while this one is multiplied; a slab is
-// 32 chunks of 16 rows x 64 bytes, wave w copies chunks w + 4 q.  Within a
+// One tile of A B (both symmetric, by their planes) over the whole K, 128 x 128
+// (H = 4) or 64 x 64 (H = 2): four waves in a 2 x 2 grid, each H x H blocks of
+// 16 x 16.  The slabs are copied global -> LDS directly (dma16), the ring's
+// other slabs (1 or 3) while this one is multiplied; a panel of a slab is 2 H
+// chunks of 16 rows x 64 bytes, wave w copies chunks w + 4 q.  Within a
 // row the 16-byte chunk g sits in slot g ^ ((row >> 1) & 3), which keeps the
 // fragment reads of 8 consecutive rows on distinct banks.  Two workgroups
 // share a CU: one multiplies while the other waits for its slab and reads its
@@ -76,84 +75,115 @@ __device__ __forceinline__ size_t plane_at(int r, int k, int ld) {
 // Bound: the operand stream from L2, 32 KB per slab of 3 x 128 x 128 x 32
 // products (42 B/clk per CU at the 16-bit peak).  Registers: 128 for the two
 // accumulator sets, 64 for a slab's fragments.
-template <typename T>
+template <typename T, int H>
 __device__ __forceinline__ void split_tile(const T* ahi, const T* alo, const T* bhi, const T* blo,
-                                           int ld, int I, int J, int8_t* ring, f4 (&hh)[4][4],
-                                           f4 (&xx)[4][4]) {
+                                           int ld, int I, int J, int8_t* ring, f4 (&hh)[H][H],
+                                           f4 (&xx)[H][H]) {
+  constexpr int E = 32 * H;            // tile edge
+  constexpr int kPanel = E * KB * 2;   // bytes of one operand plane's slab
+  constexpr int kSlab = 4 * kPanel;    // A hi, A lo, B hi, B lo
+  constexpr int D = kRing / kSlab;     // slabs in the ring
+  constexpr int CPP = H / 2;           // chunks of a panel per wave
   typedef typename Split<T>::v8 h8;
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6), wm = w & 1, wn = w >> 1;
   const int lrow = lane >> 2;
   const uint32_t voff = (uint32_t)(lrow * 64 + 16 * ((lane & 3) ^ ((lrow >> 1) & 3)));
   const uint32_t ring0 = __builtin_amdgcn_readfirstlane(lds_dma::lds_addr(ring));
-  // chunk w + 4 q (q < 8) is rows 16 ((w + 4 q) % 8) of panel q / 2
   const size_t kblock = (size_t)KB * ld * sizeof(T);
   const uint64_t panel[4] = {
-      lds_dma::uniform64((uint64_t)(uintptr_t)(ahi + (size_t)I * BM * KB)),
-      lds_dma::uniform64((uint64_t)(uintptr_t)(alo + (size_t)I * BM * KB)),
-      lds_dma::uniform64((uint64_t)(uintptr_t)(bhi + (size_t)J * BM * KB)),
-      lds_dma::uniform64((uint64_t)(uintptr_t)(blo + (size_t)J * BM * KB))};
+      lds_dma::uniform64((uint64_t)(uintptr_t)(ahi + (size_t)I * E * KB)),
+      lds_dma::uniform64((uint64_t)(uintptr_t)(alo + (size_t)I * E * KB)),
+      lds_dma::uniform64((uint64_t)(uintptr_t)(bhi + (size_t)J * E * KB)),
+      lds_dma::uniform64((uint64_t)(uintptr_t)(blo + (size_t)J * E * KB))};
   auto issue = [&](int s) {
     const size_t off = (size_t)s * kblock;
-    const uint32_t slot = ring0 + kSlab * (s & 1);
+    const uint32_t slot = ring0 + kSlab * (s % D);
 #pragma unroll
-    for (int q = 0; q < 8; ++q) {
-      const int c = w + 4 * (q & 1);  // chunk of its panel
-      lds_dma::dma16(panel[q >> 1] + off + 1024 * c, voff,
-                     __builtin_amdgcn_readfirstlane(slot + kPanel * (q >> 1) + 1024 * c));
+    for (int q = 0; q < 4 * CPP; ++q) {
+      const int c = w + 4 * (q % CPP);  // chunk of its panel
+      lds_dma::dma16(panel[q / CPP] + off + 1024 * c, voff,
+                     __builtin_amdgcn_readfirstlane(slot + kPanel * (q / CPP) + 1024 * c));
     }
   };
   const int fo = (lane & 15) * 64 + 16 * ((lane >> 4) ^ (((lane & 15) >> 1) & 3));
-  const int8_t* fa = ring + wm * 64 * 64 + fo;
-  const int8_t* fb = ring + 2 * kPanel + wn * 64 * 64 + fo;
+  const int8_t* fa = ring + wm * (E / 2) * 64 + fo;
+  const int8_t* fb = ring + 2 * kPanel + wn * (E / 2) * 64 + fo;
 #pragma unroll
-  for (int m = 0; m < 4; ++m)
+  for (int m = 0; m < H; ++m)
 #pragma unroll
-    for (int n = 0; n < 4; ++n) {
+    for (int n = 0; n < H; ++n) {
       hh[m][n] = f4{0.f, 0.f, 0.f, 0.f};
       xx[m][n] = f4{0.f, 0.f, 0.f, 0.f};
     }
   const int slabs = ld / KB;
-  issue(0);
+#pragma unroll
+  for (int s = 0; s < D - 1; ++s)
+    if (s < slabs) issue(s);
   for (int s = 0; s < slabs; ++s) {
-    // slab s has landed in every wave, and every wave has read slab s - 1
-    lds_dma::wait_vm_barrier<0>();
-    if (s + 1 < slabs) issue(s + 1);
-    const int o = kSlab * (s & 1);
-    h8 ah[4], al[4], bh[4], bl[4];
+    // slab s has landed in every wave (the D - 2 after it may be in flight),
+    // and every wave has read slab s - 1
+    if (s + D - 2 < slabs)
+      lds_dma::wait_vm_barrier<(D - 2) * 4 * CPP>();
+    else
+      lds_dma::wait_vm_barrier<0>();
+    if (s + D - 1 < slabs) issue(s + D - 1);
+    const int o = kSlab * (s % D);
+    h8 ah[H], al[H], bh[H], bl[H];
 #pragma unroll
-    for (int m = 0; m < 4; ++m) ah[m] = *(const h8*)(fa + o + 1024 * m);
+    for (int m = 0; m < H; ++m) ah[m] = *(const h8*)(fa + o + 1024 * m);
 #pragma unroll
-    for (int n = 0; n < 4; ++n) bh[n] = *(const h8*)(fb + o + 1024 * n);
+    for (int n = 0; n < H; ++n) bh[n] = *(const h8*)(fb + o + 1024 * n);
 #pragma unroll
-    for (int n = 0; n < 4; ++n) bl[n] = *(const h8*)(fb + o + kPanel + 1024 * n);
+    for (int n = 0; n < H; ++n) bl[n] = *(const h8*)(fb + o + kPanel + 1024 * n);
 #pragma unroll
-    for (int m = 0; m < 4; ++m) al[m] = *(const h8*)(fa + o + kPanel + 1024 * m);
+    for (int m = 0; m < H; ++m) al[m] = *(const h8*)(fa + o + kPanel + 1024 * m);
 #pragma unroll
-    for (int m = 0; m < 4; ++m)
+    for (int m = 0; m < H; ++m)
 #pragma unroll
-      for (int n = 0; n < 4; ++n) hh[m][n] = Split<T>::mfma(bh[n], ah[m], hh[m][n]);
+      for (int n = 0; n < H; ++n) hh[m][n] = Split<T>::mfma(bh[n], ah[m], hh[m][n]);
 #pragma unroll
-    for (int m = 0; m < 4; ++m)
+    for (int m = 0; m < H; ++m)
 #pragma unroll
-      for (int n = 0; n < 4; ++n) xx[m][n] = Split<T>::mfma(bl[n], ah[m], xx[m][n]);
+      for (int n = 0; n < H; ++n) xx[m][n] = Split<T>::mfma(bl[n], ah[m], xx[m][n]);
 #pragma unroll
-    for (int m = 0; m < 4; ++m)
+    for (int m = 0; m < H; ++m)
 #pragma unroll
-      for (int n = 0; n < 4; ++n) xx[m][n] = Split<T>::mfma(bh[n], al[m], xx[m][n]);
+      for (int n = 0; n < H; ++n) xx[m][n] = Split<T>::mfma(bh[n], al[m], xx[m][n]);
   }
 }
 
 // Operands were swapped, so a lane holds (A B)[row][col] with
 // row = lane % 16 and col = 4 (lane / 16) + r inside each 16 x 16 block.
+template <int H>
 struct SplitAt {
   int lane, row0, col0;  // the lane's first row and column
   int w;
   __device__ SplitAt(int I, int J) {
     lane = threadIdx.x & 63;
     w = threadIdx.x >> 6;
-    row0 = I * BM + (w & 1) * 64 + (lane & 15);
-    col0 = J * BM + (w >> 1) * 64 + 4 * (lane >> 4);
+    row0 = 32 * H * I + (w & 1) * 16 * H + (lane & 15);
+    col0 = 32 * H * J + (w >> 1) * 16 * H + 4 * (lane >> 4);
+  }
+};
+
+constexpr int kBand = 8;  // tile columns of a band: an XCD's 64 workgroups cover 8 x 8 tiles
+
+// The tiles of a launch: the first `full` upper-triangle 128 x 128 ones (in
+// banded order), and the rest as four 64 x 64 ones each.
+struct SplitTile {
+  int I, J;
+  bool quarter;
+  // false: a quarter below the diagonal, left to its mirror
+  __device__ bool find(int nt, int full) {
+    quarter = (int)blockIdx.x >= full;
+    const int q = (int)blockIdx.x - full;
+    sym_tile_banded<kBand>(quarter ? full + q / 4 : xcd_remap(blockIdx.x, full), nt, I, J);
+    if (quarter) {
+      I = 2 * I + (q & 1);
+      J = 2 * J + ((q >> 1) & 1);
+    }
+    return I <= J;
   }
 };
 
@@ -161,57 +191,50 @@ struct F16Args {
   const double* buf[2];         // FP64 master ping-pong (lower triangle)
   const void* hi[2];            // hi planes ping-pong (T)
   const void* lo[2];            // lo planes ping-pong (T)
-  int ld, nt;
+  int ld, nt, full;
   Sp2State* st;
   double* part;
 };
 
-constexpr int kBand = 8;  // tile columns of a band: an XCD's 64 workgroups cover 8 x 8 tiles
-constexpr int kPitch = 64 + 4;  // halves per row of a wave's 64 x 64 block in LDS
 
 // The upper-triangle tile (I, J) of X^2 and the SP2 update.  The FP64 master
-// lives in the lower triangle (and the whole of each diagonal 128 x 128
-// block), where a lane's four columns are 32 contiguous bytes; the loop's end
-// restores the upper one.  Both positions of the planes are written: (row,
+// lives in the lower triangle (and the whole of each diagonal tile), where a
+// lane's four columns are 32 contiguous bytes; the loop's end restores the
+// upper one.  Both positions of the planes are written: (row,
 // col) by the lane's four columns at a time, (col, row) after a transposition
 // of each wave's block through LDS, 8 bytes per lane each.
-template <typename T>
-__global__ __launch_bounds__(NT, 2) void sp2_f16split_kernel(F16Args g) {
+template <typename T, int H>
+__device__ __forceinline__ void sp2_split_tile(const F16Args& g, const volatile Sp2State* stv,
+                                               int I, int J, int8_t* ring, double (&sums)[4]) {
   constexpr double kScale = Split<T>::kScale;
-  __shared__ __attribute__((aligned(1024))) int8_t ring[kRing];
-  const volatile Sp2State* stv = g.st;
-  if (!stv->planned) return;
+  constexpr int kPitch = 16 * H + 4;  // halves per row of a wave's block in LDS
   const int apply = stv->apply, sigma = stv->sigma, cur = stv->cur;
   // prg_sp2_submatrix: the idempotency sum runs over the first `core` rows
   // (and, by symmetry, the mirrored columns) only
   const int core_lim = (stv->variant == V_SUBMATRIX) ? stv->core : 0x7fffffff;
   const int ld = g.ld;
-  const int t = xcd_remap(blockIdx.x, gridDim.x);
-  int I, J;
-  sym_tile_banded<kBand>(t, g.nt, I, J);
-  f4 hh[4][4], xx[4][4];
-  split_tile<T>((const T*)g.hi[cur], (const T*)g.lo[cur], (const T*)g.hi[cur], (const T*)g.lo[cur],
-                ld, I, J, ring, hh, xx);
+  f4 hh[H][H], xx[H][H];
+  split_tile<T, H>((const T*)g.hi[cur], (const T*)g.lo[cur], (const T*)g.hi[cur], (const T*)g.lo[cur],
+                   ld, I, J, ring, hh, xx);
   const double* X = g.buf[cur];
   double* Xn = const_cast<double*>(g.buf[cur ^ 1]);
   T* hin = (T*)const_cast<void*>(g.hi[cur ^ 1]);
   T* lon = (T*)const_cast<void*>(g.lo[cur ^ 1]);
   const double ca = apply ? (sigma ? 1.0 : -1.0) : 0.0;
   const double cb = apply ? (sigma ? 0.0 : 2.0) : 1.0;
-  const SplitAt at(I, J);
-  double sums[4] = {0.0, 0.0, 0.0, 0.0};
+  const SplitAt<H> at(I, J);
   typedef T t4 __attribute__((ext_vector_type(4)));
   // every wave is done with the ring: its LDS takes the waves' blocks
   lds_dma::wait_vm_barrier<0>();
-  T* block = (T*)ring + (size_t)at.w * 64 * kPitch;
+  T* block = (T*)ring + (size_t)at.w * 16 * H * kPitch;
   if (I != J) {
 #pragma unroll
-    for (int m = 0; m < 4; ++m) {
+    for (int m = 0; m < H; ++m) {
       const int row = at.row0 + 16 * m;
       const double wrow = row < core_lim ? 1.0 : 0.0;
-      t4 lov[4];
+      t4 lov[H];
 #pragma unroll
-      for (int n = 0; n < 4; ++n) {
+      for (int n = 0; n < H; ++n) {
         const int col = at.col0 + 16 * n;
         const double2* xp = (const double2*)(X + col + (size_t)row * ld);
         const double2 u = xp[0], v = xp[1];
@@ -240,28 +263,30 @@ __global__ __launch_bounds__(NT, 2) void sp2_f16split_kernel(F16Args g) {
       }
       // the lo halves wait in the accumulators' place for the second pass
 #pragma unroll
-      for (int n = 0; n < 4; ++n) {
+      for (int n = 0; n < H; ++n) {
         const uint2 b = __builtin_bit_cast(uint2, lov[n]);
         hh[m][n][0] = __uint_as_float(b.x);
         hh[m][n][1] = __uint_as_float(b.y);
       }
     }
     // Transposed store of the wave's block: lane b handles the 4 x 4 blocks
-    // (row block b % 16, column blocks b / 16 + 4 q), 16 lanes covering the
-    // 64 rows, i.e. two runs of 64 bytes per column.
+    // (row block b % RB, column blocks b / RB + CB q), RB lanes covering the
+    // 4 RB rows, i.e. runs of 64 bytes per column.
     auto mirror = [&](T* plane) {
       __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
       __builtin_amdgcn_wave_barrier();
-      const int rb = 4 * (at.lane & 15), cb0 = 4 * (at.lane >> 4);
-      const int rowb = I * BM + (at.w & 1) * 64 + rb, colb = J * BM + (at.w >> 1) * 64 + cb0;
+      constexpr int RB = 4 * H, CB = 64 / RB;
+      const int rb = 4 * (at.lane % RB), cb0 = 4 * (at.lane / RB);
+      const int rowb = 32 * H * I + (at.w & 1) * 16 * H + rb;
+      const int colb = 32 * H * J + (at.w >> 1) * 16 * H + cb0;
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
+      for (int q = 0; q < RB / CB; ++q) {
         t4 e[4];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) e[i] = *(const t4*)(block + (rb + i) * kPitch + cb0 + 16 * q);
+        for (int i = 0; i < 4; ++i) e[i] = *(const t4*)(block + (rb + i) * kPitch + cb0 + 4 * CB * q);
 #pragma unroll
         for (int j = 0; j < 4; ++j)
-          *(t4*)(plane + plane_at(colb + 16 * q + j, rowb, ld)) =
+          *(t4*)(plane + plane_at(colb + 4 * CB * q + j, rowb, ld)) =
               t4{e[0][j], e[1][j], e[2][j], e[3][j]};
       }
       __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
@@ -269,9 +294,9 @@ __global__ __launch_bounds__(NT, 2) void sp2_f16split_kernel(F16Args g) {
     };
     mirror(hin);
 #pragma unroll
-    for (int m = 0; m < 4; ++m)
+    for (int m = 0; m < H; ++m)
 #pragma unroll
-      for (int n = 0; n < 4; ++n)
+      for (int n = 0; n < H; ++n)
         *(uint2*)(block + (16 * m + (at.lane & 15)) * kPitch + 16 * n + 4 * (at.lane >> 4)) =
             uint2{__float_as_uint(hh[m][n][0]), __float_as_uint(hh[m][n][1])};
     mirror(lon);
@@ -280,10 +305,10 @@ __global__ __launch_bounds__(NT, 2) void sp2_f16split_kernel(F16Args g) {
     // hi.lo and lo.hi terms of (r, c) and (c, r) accumulate in different
     // orders), so X_next is exactly symmetric
 #pragma unroll
-    for (int m = 0; m < 4; ++m) {
+    for (int m = 0; m < H; ++m) {
       const int row = at.row0 + 16 * m;
 #pragma unroll
-      for (int n = 0; n < 4; ++n) {
+      for (int n = 0; n < H; ++n) {
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           const int col = at.col0 + 16 * n + r;
@@ -313,7 +338,22 @@ __global__ __launch_bounds__(NT, 2) void sp2_f16split_kernel(F16Args g) {
       }
     }
   }
-  block_store4<NT>(sums, g.part + 4 * (size_t)t);
+}
+
+template <typename T>
+__global__ __launch_bounds__(NT, 2) void sp2_f16split_kernel(F16Args g) {
+  __shared__ __attribute__((aligned(1024))) int8_t ring[kRing];
+  const volatile Sp2State* stv = g.st;
+  if (!stv->planned) return;
+  double sums[4] = {0.0, 0.0, 0.0, 0.0};
+  SplitTile tl;
+  if (tl.find(g.nt, g.full)) {
+    if (tl.quarter)
+      sp2_split_tile<T, 2>(g, stv, tl.I, tl.J, ring, sums);
+    else
+      sp2_split_tile<T, 4>(g, stv, tl.I, tl.J, ring, sums);
+  }
+  block_store4<NT>(sums, g.part + 4 * (size_t)blockIdx.x);
 }
 
 // X (current buffer) from its lower triangle: the upper 64 x 64 blocks are
@@ -339,34 +379,30 @@ struct SplitGemmArgs {
   double* C;
   double* part;       // per tile [Tr C, ||C||_F^2, <C, E>, 0], or null
   double alpha, beta, gamma;
-  int ld, n, nt;
+  int ld, n, nt, full;
 };
 
 // C = alpha A B + beta Cin + gamma I (gamma on the n x n diagonal) for
 // symmetric, commuting A and B from their hi/lo planes: one workgroup per
-// upper-triangle 128 x 128 tile, the tile mirrored; inside a diagonal tile
+// upper-triangle tile, the tile mirrored; inside a diagonal tile
 // the upper half is mirrored onto the lower one, so C is exactly symmetric.
 // FUSE bit 0: with Cin, bit 1: with <C, E>.
-template <typename T, int FUSE>
-__global__ __launch_bounds__(NT, 2) void split_gemm_kernel(SplitGemmArgs g) {
+template <typename T, int FUSE, int H>
+__device__ __forceinline__ void split_gemm_tile(const SplitGemmArgs& g, int I, int J, int8_t* ring,
+                                                double (&sums)[4]) {
   constexpr double kScale = Split<T>::kScale;
-  __shared__ __attribute__((aligned(1024))) int8_t ring[kRing];
   const int ld = g.ld;
-  const int t = xcd_remap(blockIdx.x, gridDim.x);
-  int I, J;
-  sym_tile_banded<kBand>(t, g.nt, I, J);
-  f4 hh[4][4], xx[4][4];
-  split_tile<T>((const T*)g.ahi, (const T*)g.alo, (const T*)g.bhi, (const T*)g.blo, ld, I, J, ring,
-                hh, xx);
-  const SplitAt at(I, J);
-  double sums[4] = {0.0, 0.0, 0.0, 0.0};
+  f4 hh[H][H], xx[H][H];
+  split_tile<T, H>((const T*)g.ahi, (const T*)g.alo, (const T*)g.bhi, (const T*)g.blo, ld, I, J,
+                   ring, hh, xx);
+  const SplitAt<H> at(I, J);
   if (I != J) {
     // the (col, row) position is 32 contiguous bytes per lane
 #pragma unroll
-    for (int m = 0; m < 4; ++m) {
+    for (int m = 0; m < H; ++m) {
       const int row = at.row0 + 16 * m;
 #pragma unroll
-      for (int n = 0; n < 4; ++n) {
+      for (int n = 0; n < H; ++n) {
         const int col = at.col0 + 16 * n;
         const size_t tdx = col + (size_t)row * ld;
         double v[4];
@@ -398,10 +434,10 @@ __global__ __launch_bounds__(NT, 2) void split_gemm_kernel(SplitGemmArgs g) {
     }
   } else {
 #pragma unroll
-    for (int m = 0; m < 4; ++m) {
+    for (int m = 0; m < H; ++m) {
       const int row = at.row0 + 16 * m;
 #pragma unroll
-      for (int n = 0; n < 4; ++n) {
+      for (int n = 0; n < H; ++n) {
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           const int col = at.col0 + 16 * n + r;
@@ -422,7 +458,20 @@ __global__ __launch_bounds__(NT, 2) void split_gemm_kernel(SplitGemmArgs g) {
       }
     }
   }
-  if (g.part) block_store4<NT>(sums, g.part + 4 * (size_t)t);
+}
+
+template <typename T, int FUSE>
+__global__ __launch_bounds__(NT, 2) void split_gemm_kernel(SplitGemmArgs g) {
+  __shared__ __attribute__((aligned(1024))) int8_t ring[kRing];
+  double sums[4] = {0.0, 0.0, 0.0, 0.0};
+  SplitTile tl;
+  if (tl.find(g.nt, g.full)) {
+    if (tl.quarter)
+      split_gemm_tile<T, FUSE, 2>(g, tl.I, tl.J, ring, sums);
+    else
+      split_gemm_tile<T, FUSE, 4>(g, tl.I, tl.J, ring, sums);
+  }
+  if (g.part) block_store4<NT>(sums, g.part + 4 * (size_t)blockIdx.x);
 }
 
 // hi/lo planes of a symmetric FP64 matrix (whole ld x ld buffer, padding stays
@@ -452,7 +501,27 @@ __global__ void split_f16_kernel(const double* __restrict__ x, T* __restrict__ h
   }
 }
 
+// How many of the upper triangle's 128 x 128 tiles a launch keeps whole: all
+// but those of the last round over the chip's two workgroups per CU, if that
+// round holds few.  Whole, a lone tile takes as long as a round (its operand
+// stream has the CU to itself but nothing to hide behind); its quarters, with
+// three slabs in flight, about half of that.  BF16 products with their split
+// pass, last rounds whole / quartered: 1024 (36 tiles) 52 / 36 us, 1920 (120)
+// 75 / 55, 2176 (153) 83 / 78, 2432 (190) 90 / 86, 2560 (210) 95 / 98; behind
+// full rounds 4096 (16) 301 / 253, 4352 (83) 322 / 307, 4608 (154) 344 / 343,
+// 4736 (191) 362 / 362, 5888 (57) 665 / 606.
+constexpr int kSlots = 2 * 256, kQuarterMax = 160;
+int split_full_tiles(int nt) {
+  const int tiles = nt * (nt + 1) / 2, rest = tiles % kSlots;
+  return rest <= kQuarterMax ? tiles - rest : tiles;
+}
+
 }  // namespace
+
+int split_step_tiles(int ld) {
+  const int nt = ld / BM, full = split_full_tiles(nt);
+  return full + 4 * (nt * (nt + 1) / 2 - full);
+}
 
 int split_f16(const DMat& x, void* hi, void* lo, bool bf16) {
   if (bf16)
@@ -489,7 +558,8 @@ int sp2_step_mixed(const DMat& x0, const DMat& x1, Sp2State* d_state, double* d_
   g.nt = ld / BM;
   g.st = d_state;
   g.part = d_part;
-  const int nb = g.nt * (g.nt + 1) / 2;
+  g.full = split_full_tiles(g.nt);
+  const int nb = split_step_tiles(ld);
   if (ntiles) *ntiles = nb;
   if (bf16)
     hipLaunchKernelGGL(sp2_f16split_kernel<__bf16>, dim3(nb), dim3(NT), 0, stream(), g);
@@ -602,7 +672,8 @@ int split_gemm(const DMat& A, const DMat& B, DMat C, double alpha, double beta, 
   g.ld = ld;
   g.n = C.n;
   g.nt = ld / BM;
-  const int nb = g.nt * (g.nt + 1) / 2;
+  g.full = split_full_tiles(g.nt);
+  const int nb = split_step_tiles(ld);
   if (nparts) *nparts = nb;
   const int fuse = (g.Cin ? 1 : 0) | (g.E ? 2 : 0);
   void (*k)(SplitGemmArgs) = fuse == 0   ? split_gemm_kernel<__bf16, 0>

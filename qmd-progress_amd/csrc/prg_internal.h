@@ -173,6 +173,8 @@ struct Sp2Link;
 int sp2_step(const DMat& x0, const DMat& x1, const DMat* d0, const DMat* d1, const Sp2Link& link,
              double* d_part, int* ntiles, bool thresholded, int cur);
 int sp2_step_tiles(int ld);
+// Records of partial sums of an FP16 / BF16 split step or product.
+int split_step_tiles(int ld);
 // Device-side SP2 bookkeeping kernels.
 int sp2_init_state(Sp2State* d_state, const double* d_part, int nblocks);
 int sp2_absorb_plan(Sp2State* d_state, const double* d_part, int ntiles);

@@ -100,7 +100,8 @@ int fetch(const double* d_part, int nb, int nq, double* host) {
 static double* part_buf(int ld, int* st) {
   const size_t nb = ld / 64;
   const size_t records =
-      std::max({nb * nb, (size_t)gemm_tiles(ld, 0), (size_t)gemm_tiles(ld, 1)}) + 2048;
+      std::max({nb * nb, (size_t)gemm_tiles(ld, 0), (size_t)gemm_tiles(ld, 1),
+                (size_t)split_step_tiles(ld)}) + 2048;
   return (double*)workspace("ops_part", sizeof(double) * 4 * records, st);
 }
 

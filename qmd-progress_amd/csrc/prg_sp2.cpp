@@ -118,8 +118,8 @@ namespace {
 // alternates between two sets: a step's workgroups read the last step's while
 // others already write theirs.
 size_t part_doubles(int ld) {
-  const int nt = ld / kTile;
-  const int nslots = std::max({nt * (nt + 1) / 2, sp2_step_tiles(ld), crt_update_blocks(ld)});
+  const int nslots =
+      std::max({split_step_tiles(ld), sp2_step_tiles(ld), crt_update_blocks(ld)});
   return 4 * (size_t)(nslots + 2048);
 }
 }  // namespace
