@@ -258,10 +258,7 @@ def main():
     kern = hr.get("product_kernel_mfma_tops")
     roofline = {
         "bound": "mfma",
-        "kernel": {"fp64": ("sp2_step_kernel (FP64 MFMA, fused SP2 update)"
-                            if P.sp2_split_slices(n) == 1 else
-                            f"sp2_split_product_kernel + sp2_split_epilogue_kernel (FP64 MFMA, "
-                            f"K in {P.sp2_split_slices(n)} slices; the pair's time)"),
+        "kernel": {"fp64": "sp2_step_kernel (FP64 MFMA, fused SP2 update)",
                    "f16split": "sp2_f16split_kernel (FP16 MFMA, 3 products)",
                    "bf16split": "sp2_f16split_kernel<bf16> (BF16 MFMA, 3 products)",
                    "int8crt": f"{crt_kernel_name(hr.get('int8_config'))} (int8 MFMA, {hmod} "
@@ -780,13 +777,24 @@ def fermi_adjoint_bench(args, P, torch, np):
            "cpu_baseline": None, "roofline": None})
 
 
+def fp64_tile_edge(ld):
+    """Tile edge of the FP64 step kernel at a leading dimension: the library's
+    cost rule (prg_f64_tile.h, best_edge)."""
+    def cost(e):
+        nb = -(-ld // e)
+        return -(-(nb * (nb + 1) // 2) // 256) * e * e * {48: 1.0, 32: 1.1, 16: 2.0}[e]
+    return min((48, 32, 16), key=cost)
+
+
 def executed_ops(ld, mode, moduli):
     """MFMA operations of one symmetric SP2 product launch: upper-triangle
-    128x128 tiles (fp64, f16split, bf16split) or 256x256 tiles over the residue planes'
-    leading dimension rounded up to 256 (int8crt)."""
-    tm = 256 if mode == "int8crt" else 128
+    tiles of the FP64 kernel's edge (fp64), 128x128 tiles (f16split, bf16split;
+    the few whose last round is cut into quarters counted whole) or 256x256
+    tiles over the residue planes' leading dimension rounded up to 256
+    (int8crt)."""
+    tm = {"int8crt": 256, "fp64": fp64_tile_edge(ld)}.get(mode, 128)
     kd = ((ld + 255) // 256) * 256 if mode == "int8crt" else ld
-    nt = kd // tm
+    nt = -(-kd // tm)
     per_pass = nt * (nt + 1) // 2 * 2.0 * tm * tm * kd
     return per_pass * {"fp64": 1, "f16split": 3, "bf16split": 3, "int8crt": moduli}[mode]
 
