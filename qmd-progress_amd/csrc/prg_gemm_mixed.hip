@@ -25,6 +25,7 @@ namespace prg {
 namespace {
 
 using tile::block_store4;
+using tile::sym_tile;
 using tile::sym_tile_banded;
 using tile::xcd_remap;
 
@@ -475,18 +476,25 @@ __global__ __launch_bounds__(NT, 2) void split_gemm_kernel(SplitGemmArgs g) {
 }
 
 // hi/lo planes of a symmetric FP64 matrix (whole ld x ld buffer, padding stays
-// zero) in the blocked layout: a thread converts 4 consecutive k's of a row r,
-// read as (k, r), 32 contiguous bytes.
+// zero) in the blocked layout.  One workgroup per 64 x 64 block (I, J) of the
+// upper triangle: its entries are read once, as (k, r) with a thread's four
+// k's in 32 contiguous bytes, and both planes get the block and, through LDS,
+// its transpose.  Bound: HBM, 4 bytes read and 4 written per entry; N = 4096:
+// 27.2 us (134 MB, 4.9 TB/s; 40.1 us when the whole matrix was read).
 template <typename T>
-__global__ void split_f16_kernel(const double* __restrict__ x, T* __restrict__ hi,
-                                 T* __restrict__ lo, int ld) {
+__global__ __launch_bounds__(NT) void split_f16_kernel(const double* __restrict__ x,
+                                                       T* __restrict__ hi, T* __restrict__ lo,
+                                                       int ld) {
   typedef T t4 __attribute__((ext_vector_type(4)));
-  const size_t count = (size_t)ld * ld / 4;
-  for (size_t i = (size_t)blockIdx.x * NT + threadIdx.x; i < count; i += (size_t)gridDim.x * NT) {
-    // i-th group of 4 in plane order: 8 groups per row of a 32-column block
-    const int kq = (int)(i & 7);
-    const size_t q = i >> 3;
-    const int r = (int)(q % ld), k = (int)(q / ld) * KB + 4 * kq;
+  constexpr int B = 64, kPitch = B + 4;
+  __shared__ __attribute__((aligned(16))) T th[B * kPitch], tl[B * kPitch];
+  int I, J;
+  sym_tile(blockIdx.x, I, J);
+  const int g = threadIdx.x & 15, y = threadIdx.x >> 4;
+  const bool mirror = I != J;
+#pragma unroll
+  for (int p = 0; p < 4; ++p) {
+    const int rl = 16 * p + y, r = B * I + rl, k = B * J + 4 * g;
     const double2* xp = (const double2*)(x + k + (size_t)r * ld);
     const double2 a = xp[0], b = xp[1];
     const double z[4] = {a.x, a.y, b.x, b.y};
@@ -496,9 +504,28 @@ __global__ void split_f16_kernel(const double* __restrict__ x, T* __restrict__ h
       h[j] = (T)z[j];
       l[j] = (T)((z[j] - (double)h[j]) * Split<T>::kScale);
     }
-    *(t4*)(hi + 4 * i) = h;
-    *(t4*)(lo + 4 * i) = l;
+    const size_t at = plane_at(r, k, ld);
+    *(t4*)(hi + at) = h;
+    *(t4*)(lo + at) = l;
+    if (mirror) {
+      *(t4*)(th + rl * kPitch + 4 * g) = h;
+      *(t4*)(tl + rl * kPitch + 4 * g) = l;
+    }
   }
+  if (!mirror) return;
+  __syncthreads();
+  // the 4 x 4 block of rows 4 g .. and k's 4 y .., transposed
+  auto transposed = [&](const T* t, T* plane) {
+    t4 e[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) e[i] = *(const t4*)(t + (4 * g + i) * kPitch + 4 * y);
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      *(t4*)(plane + plane_at(B * J + 4 * y + j, B * I + 4 * g, ld)) =
+          t4{e[0][j], e[1][j], e[2][j], e[3][j]};
+  };
+  transposed(th, hi);
+  transposed(tl, lo);
 }
 
 // How many of the upper triangle's 128 x 128 tiles a launch keeps whole: all
@@ -524,11 +551,13 @@ int split_step_tiles(int ld) {
 }
 
 int split_f16(const DMat& x, void* hi, void* lo, bool bf16) {
+  const int nb = x.ld / 64;
+  const dim3 grid(nb * (nb + 1) / 2);
   if (bf16)
-    hipLaunchKernelGGL(split_f16_kernel<__bf16>, dim3(2048), dim3(NT), 0, stream(), x.p,
-                       (__bf16*)hi, (__bf16*)lo, x.ld);
+    hipLaunchKernelGGL(split_f16_kernel<__bf16>, grid, dim3(NT), 0, stream(), x.p, (__bf16*)hi,
+                       (__bf16*)lo, x.ld);
   else
-    hipLaunchKernelGGL(split_f16_kernel<_Float16>, dim3(2048), dim3(NT), 0, stream(), x.p,
+    hipLaunchKernelGGL(split_f16_kernel<_Float16>, grid, dim3(NT), 0, stream(), x.p,
                        (_Float16*)hi, (_Float16*)lo, x.ld);
   PRG_HIP_CHECK(hipGetLastError());
   return OK;
