@@ -13,6 +13,7 @@ struct bml_matrix_t {
   int ld = 0;
   bool host_valid = true;
   bool dev_valid = false;
+  bool host_written = false;  // its pages exist (calloc leaves them to the first write)
 };
 
 namespace prg {

@@ -227,10 +227,15 @@ class Matrix:
         n = self.n
         p = lib().bml_export_to_dense(self.h, _col_major)
         _check()
-        # the exported buffer becomes the array's memory, freed with its last view
         buf = (C.c_double * (n * n)).from_address(p)
-        weakref.finalize(buf, _free, p).atexit = False
-        return np.frombuffer(buf, dtype=np.float64).reshape((n, n), order="F")
+        out = np.frombuffer(buf, dtype=np.float64)
+        if n <= 128:  # a copy costs less than the finalizer below
+            out = out.copy()
+            _free(p)
+        else:
+            # the exported buffer becomes the array's memory, freed with its last view
+            weakref.finalize(buf, _free, p).atexit = False
+        return out.reshape((n, n), order="F")
 
     def close(self):
         if self.h:
