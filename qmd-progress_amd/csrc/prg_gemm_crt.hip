@@ -814,6 +814,14 @@ __global__ void crt_scale_kernel(const double* __restrict__ part, int nb, double
 // even modulus, has an exact quotient whose tie is the byte 0x80 either way.
 // N = 4096, 12 moduli: 45.4 us (268 MB, 5.9 TB/s; 84.5 us when the whole matrix
 // was read and every residue corrected).
+//
+// With 13 and 14 moduli the corrected residues of a small matrix's few blocks
+// are a serial chain, so up to 7 workgroups share a block's moduli, about 1200
+// in all.  A product of two matrices, 14 moduli: N = 50 70 -> 60 us, 512
+// 78 -> 62, 1024 90 -> 79, 1500 136 -> 124.  (The short chains of 12 and fewer
+// moduli lose by it: N = 50 55 -> 60 us.)
+template <int NP>
+constexpr bool kSliced = NP > 12;
 template <int NP>
 __global__ __launch_bounds__(NT) void crt_split_scaled_kernel(const double* __restrict__ x,
                                                               int8_t* __restrict__ p0, int ld,
@@ -825,8 +833,7 @@ __global__ __launch_bounds__(NT) void crt_split_scaled_kernel(const double* __re
   tile::sym_tile(blockIdx.x, I, J);
   const int tid = threadIdx.x, lane = tid & 63, b = tid >> 6;
   const int rl = 16 * b + (lane & 15), row = SB * I + rl, cl0 = 4 * (lane >> 4);
-  // v: the integers; with NP <= 12 also v + kMagic
-  double v[16];
+  double v[16];  // the integers
 #pragma unroll
   for (int n = 0; n < 4; ++n) {
     const int col0 = SB * J + 16 * n + cl0;
@@ -847,8 +854,12 @@ __global__ __launch_bounds__(NT) void crt_split_scaled_kernel(const double* __re
   const int qr = 4 * (tid & 15), qc = 4 * (tid >> 4);
   int8_t* pd = p0 + (size_t)J * pld * SB + (size_t)(SB * I + dr) * SB + dc;
   int8_t* pt = p0 + (size_t)I * pld * SB + (size_t)(SB * J + qc) * SB + qr;
+  // this workgroup's moduli
+  const int kbeg = kSliced<NP> ? NP * blockIdx.y / gridDim.y : 0;
+  const int kend = kSliced<NP> ? NP * (blockIdx.y + 1) / gridDim.y : NP;
 #pragma unroll
   for (int k = 0; k < NP; ++k) {
+    if (k < kbeg || k >= kend) continue;
     const double p = c.p[k], inv = c.inv[k];
     int8_t (*buf)[kPitch] = rb[k & 1];
 #pragma unroll
@@ -1200,9 +1211,10 @@ void launch_update(const UpdateArgs& g, int nblocks) {
 template <int NP>
 void launch_split_scaled(const double* x, int8_t* p, int ld, int pld, const CrtConst& c,
                          const double* sc) {
-  const int nb = pld / SB;
-  hipLaunchKernelGGL(crt_split_scaled_kernel<NP>, dim3(nb * (nb + 1) / 2), dim3(NT), 0, stream(),
-                     x, p, ld, pld, c, sc);
+  const int nb = pld / SB, blocks = nb * (nb + 1) / 2;
+  const int slices = kSliced<NP> ? std::min(7, std::max(1, 1200 / blocks)) : 1;
+  hipLaunchKernelGGL(crt_split_scaled_kernel<NP>, dim3(blocks, slices), dim3(NT), 0, stream(), x,
+                     p, ld, pld, c, sc);
 }
 
 template <int NP>

@@ -47,3 +47,37 @@ def test_product_equals_the_oracle(P, n, moduli):
     assert np.max(np.abs(c[:n, :n] - ref)) <= tol
     assert np.array_equal(c, c.T)
     assert not c[n:].any() and not c[:, n:].any()
+
+
+@pytest.mark.parametrize("moduli", [13, 14])
+@pytest.mark.parametrize("n", [1025, 1500, 1900, 2200])
+def test_shared_blocks_of_larger_matrices(P, n, moduli):
+    """The moduli of a block over 5, 4, 2 and 1 workgroups, against float64
+    (n eps of the norms): the fraction sum's rounding as above, and the
+    operands' of 2^-(a + 1) of a scale of at most twice their norm."""
+    import torch
+    print(f"[crt planes] n={n} moduli={moduli}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(n)
+    x = torch.randn((n, n), dtype=torch.float64, device="cuda", generator=g) / n ** 0.5
+    a = 0.5 * (x + x.T)
+    b = a @ a - 0.7 * a
+    b = 0.5 * (b + b.T)
+    ld = P.padded_ld(n)
+    pad = torch.zeros((3, ld, ld), dtype=torch.float64, device="cuda")
+    pad[0, :n, :n], pad[1, :n, :n], pad[2] = a, b, 7.0
+    torch.cuda.synchronize()
+    P.set_product_precision(P.PREC_INT8CRT)
+    P.set_int8_moduli(moduli)
+    try:
+        P.symmetric_product_device(pad[0], pad[1], pad[2], n)
+    finally:
+        P.set_int8_moduli(11)
+        P.set_product_precision(P.PREC_FP64)
+    c = pad[2]
+    scale_bits = O.crt_constants(moduli, square=False)[2]
+    eps = np.finfo(float).eps
+    rounding = n * eps + 4 * moduli * eps * 72 * 16 + 4 * n ** 0.5 * 2.0 ** -scale_bits
+    bound = rounding * float(a.norm(dim=0).max() * b.norm(dim=0).max())
+    assert float((c[:n, :n] - a @ b).abs().max()) <= bound
+    assert torch.equal(c, c.T)
+    assert not bool(c[n:].any()) and not bool(c[:, n:].any())
