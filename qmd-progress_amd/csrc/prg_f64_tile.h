@@ -393,18 +393,15 @@ typedef Shape<3> S48;
 // 67.5 / 84.5; 2048 - / 158 / 148; 2600 - / 313 / 321; 4096 - / 1148 / 1067.
 // (64-, 96- and 128-wide tiles of 2 x 2 waves: 187, 152 and 262 us at 2048,
 // 1309, 1101 and 1443 us at 4096.)
+inline double edge_cost(int tiles, int e) {
+  const double rounds = (tiles + 255) / 256;
+  return rounds * e * e * (e == 48 ? 1.0 : e == 32 ? 1.1 : 2.0);
+}
 template <typename F>
 inline int best_edge(F&& tiles) {
   int best = 48;
-  double best_cost = 1e300;
-  for (int e : {48, 32, 16}) {
-    const double rounds = (tiles(e) + 255) / 256;
-    const double cost = rounds * e * e * (e == 48 ? 1.0 : e == 32 ? 1.1 : 2.0);
-    if (cost < best_cost) {
-      best_cost = cost;
-      best = e;
-    }
-  }
+  for (int e : {32, 16})
+    if (edge_cost(tiles(e), e) < edge_cost(tiles(best), best)) best = e;
   return best;
 }
 
@@ -416,6 +413,21 @@ inline int tile_count(int ld, int edge, bool sym) {
 }
 inline int tile_edge(int ld, bool sym) {
   return best_edge([&](int e) { return tile_count(ld, e, sym); });
+}
+
+// Whether a full product of operands that are not symmetric takes less time on
+// the staged 128-wide tiles (gemm_staged_kernel), two workgroups per CU: a
+// round of 512 of them takes as long as 12.95 rounds of 48-wide ones (243 us
+// against 18.7 us at K = 1000), a single round of at most 256, one per CU, 0.58
+// of that.  Z^T A Z and Z A Z^T (two products each), ms, 48-wide / staged:
+// ld 1920 0.58, 0.54 / 0.65, 0.61; 2048 0.73, 0.65 / 0.69, 0.65; 2560 1.35,
+// 1.23 / 1.41, 1.34; 2816 1.77, 1.54 / 1.60, 1.53; 3072 2.16, 1.90 / 3.17,
+// 3.02; 4096 4.62, 4.34 / 4.45, 4.05; 5632 11.5, 11.4 / 11.0, 11.1; 6144 13.7,
+// 13.5 / 15.0, 15.0; 6400 16.5, 16.7 / 15.7, 15.7; 8192 34.2, 34.2 / 32.0, 32.0.
+inline bool full_is_staged(int ld) {
+  const int nt = ld / 128, tiles = nt * nt, edge = tile_edge(ld, false);
+  const double rounds = tiles <= 256 ? 0.58 : (tiles + 511) / 512;
+  return 12.95 * rounds * 48 * 48 < edge_cost(tile_count(ld, edge, false), edge);
 }
 
 #define PRG_F64_SHAPE_DISPATCH(EDGE, CALL) \

@@ -132,6 +132,97 @@ __global__ __launch_bounds__(S::NT, 2) void gemm_kernel(GemmArgs g) {
   if (g.part) block_store4<S::NT>(sums, g.part + 4 * (size_t)t);
 }
 
+// ----------------------------------------------- full products, staged tiles
+// The same C for operands that are not symmetric, one 128 x 128 tile per
+// workgroup: 16-deep slabs of both panels go through LDS with the next slab
+// in registers, four waves in a 2 x 2 grid of 4 x 4 MFMA blocks.  B is read
+// along its columns, 64 bytes per thread, where a 48-wide tile's fragments
+// take 64 bytes of each of 16 columns; with two workgroups per CU 67 TFLOP/s,
+// whatever the leading dimension.  What it costs is the tiles' size (see
+// full_is_staged).
+namespace staged {
+constexpr int BM = 128, BK = 16, NT = 256;
+constexpr int LROW = BM + 4;  // padded LDS row length in doubles
+}  // namespace staged
+
+__global__ __launch_bounds__(staged::NT, 2) void gemm_staged_kernel(GemmArgs g) {
+  using namespace staged;
+  typedef f64tile::d2 d2;
+  __shared__ double As[BK][LROW], Bs[BK][LROW];
+  const int t = xcd_remap(blockIdx.x, gridDim.x), ld = g.ld;
+  int I, J;
+  full_tile(t, g.nt, I, J);
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, wm = w & 1, wn = w >> 1;
+  const int ar = (tid & 63) * 2, ak = tid >> 6;  // A: rows ar, ar + 1; k = ak + 4 q
+  const int bj = tid >> 1, bk = (tid & 1) * 8;   // B: column bj; k = bk .. bk + 7
+  const int slabs = g.kdim / BK, total = slabs * g.npair;
+  d2 ra[4], rb[4];
+  auto load = [&](int s) {
+    const int p = s >= slabs, k0 = (s - p * slabs) * BK;
+    const double* Ap = g.A[p] + (size_t)I * BM + ar;
+    const double* Bp = g.B[p] + (size_t)(J * BM + bj) * ld + k0 + bk;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      ra[q] = *(const d2*)(Ap + (size_t)(k0 + ak + 4 * q) * ld);
+      rb[q] = *(const d2*)(Bp + 2 * q);
+    }
+  };
+  d4 acc[4][4];
+#pragma unroll
+  for (int m = 0; m < 4; ++m)
+#pragma unroll
+    for (int n = 0; n < 4; ++n) acc[m][n] = d4{0.0, 0.0, 0.0, 0.0};
+  load(0);
+  for (int s = 0; s < total; ++s) {
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      As[ak + 4 * q][ar] = ra[q].x;
+      As[ak + 4 * q][ar + 1] = ra[q].y;
+      Bs[bk + 2 * q][bj] = rb[q].x;
+      Bs[bk + 2 * q + 1][bj] = rb[q].y;
+    }
+    __syncthreads();
+    if (s + 1 < total) load(s + 1);
+#pragma unroll
+    for (int kk = 0; kk < BK / 4; ++kk) {
+      const int kr = kk * 4 + (lane >> 4);
+      double a[4], b[4];
+#pragma unroll
+      for (int m = 0; m < 4; ++m) a[m] = As[kr][wm * 64 + m * 16 + (lane & 15)];
+#pragma unroll
+      for (int n = 0; n < 4; ++n) b[n] = Bs[kr][wn * 64 + n * 16 + (lane & 15)];
+#pragma unroll
+      for (int m = 0; m < 4; ++m)
+#pragma unroll
+        for (int n = 0; n < 4; ++n)
+          acc[m][n] = __builtin_amdgcn_mfma_f64_16x16x4f64(b[n], a[m], acc[m][n], 0, 0, 0);
+    }
+  }
+  double sums[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+  for (int m = 0; m < 4; ++m) {
+    const int row = I * BM + wm * 64 + m * 16 + (lane & 15);
+#pragma unroll
+    for (int n = 0; n < 4; ++n) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int col = J * BM + wn * 64 + n * 16 + (lane >> 4) + 4 * r;
+        const size_t idx = row + (size_t)col * ld;
+        double v = acc[m][n][r] * g.alpha;
+        if (g.beta != 0.0) v += g.beta * g.Cin[idx];
+        const bool diag = (row == col);
+        v += (diag && row < g.n) ? g.gamma : 0.0;
+        sums[0] += diag ? v : 0.0;
+        sums[1] += v * v;
+        if (g.dotE) sums[2] += v * g.dotE[idx];
+        g.C[idx] = v;
+      }
+    }
+  }
+  if (g.part) block_store4<NT>(sums, g.part + 4 * (size_t)t);
+}
+
 // ------------------------------------------------------------- SP2 step
 struct Sp2Args {
   const double* buf[2];  // ping-pong X buffers
@@ -340,7 +431,8 @@ int gemm(int npair, const DMat* A, const DMat* B, double alpha, double beta, con
     g.A[p] = A[p < npair ? p : 0].p;
     g.B[p] = B[p < npair ? p : 0].p;
   }
-  const int edge = f64tile::tile_edge(ld, sym != 0);
+  const bool on_staged = !sym && !b_symmetric && f64tile::full_is_staged(ld);
+  const int edge = on_staged ? staged::BM : f64tile::tile_edge(ld, sym != 0);
   g.npair = npair;
   g.ld = ld;
   // the padding of the operands is zero, so K ends at n's chunk
@@ -357,6 +449,11 @@ int gemm(int npair, const DMat* A, const DMat* B, double alpha, double beta, con
   g.part = d_part;
   const int nb = f64tile::tile_count(ld, edge, sym != 0);
   if (ntiles) *ntiles = nb;
+  if (on_staged) {
+    hipLaunchKernelGGL(gemm_staged_kernel, dim3(nb), dim3(staged::NT), 0, stream(), g);
+    PRG_HIP_CHECK(hipGetLastError());
+    return OK;
+  }
   const int fuse = (beta != 0.0 ? 1 : 0) | (dotE ? 2 : 0);
 #define PRG_CALL(S) launch_gemm<S>(g, nb, !b_symmetric, fuse)
   PRG_F64_SHAPE_DISPATCH(edge, PRG_CALL)
