@@ -40,7 +40,7 @@ struct BatchArgs {
   int sigma;            // 1: X^2 ; 0: 2X - X^2
   double* part_sums;    // per tile: core-row sum of (X - X^2)^2
   const int* queue_off; // queue q holds tiles [queue_off[q], queue_off[q + 1]), q < 8
-  int* tickets;         // 8 ticket counters, zero at launch
+  int* tickets;         // 8 ticket counters, kTicketStride apart, zero at launch
   // split-precision kernels: 16-bit hi / lo planes of the current and the
   // next X, packed like x (same element offsets)
   const void* hi;
@@ -188,7 +188,7 @@ __global__ __launch_bounds__(NT, WIDE ? 2 : 4) void batched_sp2_kernel(BatchArgs
     const int first = g.queue_off[qi], count = g.queue_off[qi + 1] - first;
     for (;;) {
       __syncthreads();  // every thread has read the previous ticket
-      if (threadIdx.x == 0) s_ticket = atomicAdd(&g.tickets[qi], 1);
+      if (threadIdx.x == 0) s_ticket = atomicAdd(&g.tickets[kTicketStride * qi], 1);
       __syncthreads();
       const int k = s_ticket;
       if (k >= count) break;
@@ -225,7 +225,7 @@ __global__ __launch_bounds__(NT, 2) void batched_sp2_direct_kernel(BatchArgs g) 
     const int qi = (home + q) & 7;
     const int begin = g.queue_off[qi], size = g.queue_off[qi + 1] - begin;
     int ticket = 0;
-    if (threadIdx.x == 0) ticket = atomicAdd(&g.tickets[qi], 1);
+    if (threadIdx.x == 0) ticket = atomicAdd(&g.tickets[kTicketStride * qi], 1);
     for (;;) {
       __syncthreads();  // every thread has read the previous ticket and lds
       if (threadIdx.x == 0) s_ticket = ticket;
@@ -233,7 +233,7 @@ __global__ __launch_bounds__(NT, 2) void batched_sp2_direct_kernel(BatchArgs g) 
       const int k = __builtin_amdgcn_readfirstlane(s_ticket);
       if (k >= size) break;
       // the next ticket arrives under this tile's product
-      if (threadIdx.x == 0) ticket = atomicAdd(&g.tickets[qi], 1);
+      if (threadIdx.x == 0) ticket = atomicAdd(&g.tickets[kTicketStride * qi], 1);
       const int t = begin + k;
       const int4 tl = g.tiles[t];
       if (!tile_wanted(g, t, tl)) continue;
@@ -578,7 +578,7 @@ __global__ __launch_bounds__(NT, 2) void batched_split_wide_kernel(BatchArgs g) 
     const int first = g.queue_off[qi], count = g.queue_off[qi + 1] - first;
     for (;;) {
       __syncthreads();  // every thread has read the previous ticket
-      if (threadIdx.x == 0) s_ticket = atomicAdd(&g.tickets[qi], 1);
+      if (threadIdx.x == 0) s_ticket = atomicAdd(&g.tickets[kTicketStride * qi], 1);
       __syncthreads();
       const int k = s_ticket;
       if (k >= count) break;
@@ -807,7 +807,7 @@ __global__ __launch_bounds__(RNT, 1) void batched_split_ring_kernel(BatchArgs g)
     const int first = g.queue_off[qi], count = g.queue_off[qi + 1] - first;
     for (;;) {
       __syncthreads();  // every thread has read the previous ticket
-      if (threadIdx.x == 0) s_ticket = atomicAdd(&g.tickets[qi], 1);
+      if (threadIdx.x == 0) s_ticket = atomicAdd(&g.tickets[kTicketStride * qi], 1);
       __syncthreads();
       const int k = s_ticket;
       if (k >= count) break;
@@ -836,7 +836,7 @@ __global__ __launch_bounds__(NT, 4) void batched_split_kernel(BatchArgs g) {
     const int first = g.queue_off[qi], count = g.queue_off[qi + 1] - first;
     for (;;) {
       __syncthreads();  // every thread has read the previous ticket
-      if (threadIdx.x == 0) s_ticket = atomicAdd(&g.tickets[qi], 1);
+      if (threadIdx.x == 0) s_ticket = atomicAdd(&g.tickets[kTicketStride * qi], 1);
       __syncthreads();
       const int k = s_ticket;
       if (k >= count) break;

@@ -125,10 +125,10 @@ int make_plan(const prg_graph_partitioning_t* gp, HostPlan* hp, BatchPlan* plan)
 // Upper-triangle tiles (part, first row, first column, shape) of every part
 // over panels of width `panel` (48, 64 or 128); the last panel of a part is 64
 // wide when 128 does not divide its size, so the shapes are 128 x 128
-// (code 3), 128 x 64 (1) and 64 x 64 (0); 48-wide panels may overhang it.  The parts are dealt to 8 queues,
-// one per XCD, largest work first to the least loaded queue (work of a tile:
-// rows x columns x m); a queue lists its parts' tiles part by part, column
-// by column.  off[q] is the first tile of queue q, off[8] the total.
+// (code 3), 128 x 64 (1) and 64 x 64 (0); 48-wide panels may overhang it.  The
+// parts are dealt to 8 queues, one per XCD, largest work first to the least
+// loaded queue (work of a tile: rows x columns x m); a queue lists its parts'
+// tiles part by part, column by column (48-wide ones in bands).  off[q] is the first tile of queue q, off[8] the total.
 struct TileQueues {
   std::vector<int4> tiles;
   std::vector<int> off;
@@ -216,23 +216,48 @@ constexpr BatchConfig kCandidates[] = {
 // into a 4-slot LDS ring (depth 4)
 constexpr BatchConfig kSplitCandidates[] = {{64, 1, 64}, {128, 1, 32}, {128, 4, 32}};
 
-// Whether a batch's FP64 products take less time on staged 64-wide tiles than
-// on 48-wide ones.  A 48-wide tile's multiply-add takes 0.97 of the other's
-// time once both fill the chip (twenty iterations: 124 parts of 640 rows 13.4
-// against 13.1 ms, 21 of 1000 8.2 / 9.1, 12 of 1500 14.8 / 15.6), so there
-// the padding decides: 2304 parts of 128 rows (3 panels against 2) take 6.1
-// against 5.4 ms.  Where the 64-wide tiles are fewer than two rounds of their
-// 4 workgroups per CU, the 48-wide ones win whatever the padding: 216 parts of
-// 128 rows 1.5 / 2.1 ms, 481 of 64 1.4 / 2.1, 70 of 320 2.1 / 2.8.
-bool staged_is_faster(const HostPlan& hp, size_t tiles64) {
-  if (tiles64 < 2 * 4 * 256) return false;
-  double direct = 0.0, staged = 0.0;
+// Upper-triangle tiles of a part over panels of 48 (its n rows) or 64 (all m).
+size_t part_tiles(const PartDesc& d, int panel) {
+  const size_t t = panel == 48 ? (d.n + 47) / 48 : d.m / 64;
+  return t * (t + 1) / 2;
+}
+
+// Time of one FP64 iteration over square tiles, us: what a launch takes, and
+// per resident workgroup (`slots` on the chip) what a tile and its
+// multiply-adds take, no less than one tile's.
+double iteration_time(const HostPlan& hp, int panel, int slots, double launch, double per_tile,
+                      double per_mac) {
+  double tiles = 0.0, macs = 0.0, largest = 0.0;
   for (const PartDesc& d : hp.parts) {
-    const double t48 = (d.n + 47) / 48, t64 = d.m / 64;
-    direct += t48 * (t48 + 1) * 48 * 48 * d.n;
-    staged += t64 * (t64 + 1) * 64 * 64 * d.m;
+    const double t = part_tiles(d, panel);
+    const double tile = (double)panel * panel * (panel == 48 ? d.n : d.m);
+    tiles += t;
+    macs += t * tile;
+    largest = std::max(largest, tile);
   }
-  return staged < 0.97 * direct;
+  return launch + per_tile * std::max(tiles / slots, 1.0) +
+         per_mac * std::max(macs / slots, largest);
+}
+
+// Whether a batch's FP64 products take less time on staged 64-wide tiles (four
+// workgroups per CU) than on 48-wide ones (two).  The constants fit both
+// kernels' times over 54 to 3072 parts of 32 to 384 rows to 20 % (the staged
+// one's below 60 us to 30 %); where they pick the slower one it is by at most
+// 15 %, and below 0.5 ms.  What decides is mostly the padding; ms for
+// 17 iterations, 48-wide / staged: 528 parts of 64 rows 0.53 / 0.43, 3072 of
+// 64 1.95 / 1.03; 532 of 80 0.64 / 0.91; 264 of 128 0.71 / 0.64, 3072 of 128
+// 5.9 / 4.5; 1008 of 144 2.5 / 3.6; 1026 of 160 3.98 / 3.69; 512 of 192
+// 2.29 / 2.00; 585 of 224 4.06 / 4.47; 516 of 256 5.0 / 4.2; 512 of 384 11.1 /
+// 11.1.  Large parts fill the chip with either and take 0.95 of the staged
+// tiles' time per multiply-add on 48-wide ones (32 parts of 2048 rows 72.0 /
+// 75.4).  (Two slabs of prefetch are
+// within 3 % of one everywhere, except 384 rows: 4 to 8 % better.  32-deep
+// slabs are slower than 16-deep ones, and 128-wide panels than 64-wide ones
+// but for a few 0.01 ms below 300 parts of 64 rows.  They are compiled for
+// the restrictions above.)
+bool staged_is_faster(const HostPlan& hp) {
+  return iteration_time(hp, 64, 4 * 256, 4.2, 10.2, 33.6e-6) <
+         iteration_time(hp, 48, 2 * 256, 10.0, 4.7, 16e-6);
 }
 
 std::map<std::pair<uint64_t, int>, BatchConfig>& config_cache() {
@@ -257,7 +282,7 @@ int time_step(const BatchPlan& plan, const double* x, double* xn, double* part, 
   PRG_HIP_CHECK(hipEventCreate(&b));
   int st = OK;
   for (int r = 0; r < 4 && !st; ++r) {
-    if ((st = batched_zero_tickets(tickets, 8))) break;
+    if ((st = batched_zero_tickets(tickets, kTickets))) break;
     PRG_HIP_CHECK(hipEventRecord(a, stream()));
     if ((st = batched_step(plan, x, xn, 1, part, tickets))) break;
     PRG_HIP_CHECK(hipEventRecord(b, stream()));
@@ -298,12 +323,12 @@ int g_cfg[4] = {0, 0, 0, 0};
 // idempotency sums.  d_part holds iters x ntiles partials.
 int enqueue_loop(const BatchPlan& plan, double* x0, double* x1, const int* pp, int iters,
                  double* d_part, int* d_tickets, double* d_vv) {
-  int st = batched_zero_tickets(d_tickets, 8 * iters);
+  int st = batched_zero_tickets(d_tickets, kTickets * iters);
   const double* cur = x0;
   double* nxt = x1;
   for (int it = 0; it < iters && !st; ++it) {
     st = batched_step(plan, cur, nxt, pp[it] != 0, d_part + (size_t)it * plan.ntiles,
-                      d_tickets + 8 * it, it & 1, it == iters - 1);
+                      d_tickets + kTickets * it, it & 1, it == iters - 1);
     const double* t = cur;
     cur = nxt;
     nxt = const_cast<double*>(t);
@@ -382,15 +407,18 @@ int subgraph_sp2_loop(const DMat& H, DMat rho, prg_graph_partitioning_t* gp) {
   if ((st = make_plan(gp, &hp, &plan))) return st;
   const size_t off = plan.total;
   const int iters = gp->maxIter;
-  const TileQueues tiles64 = make_tiles(hp, 64);
-  const TileQueues tiles48 = make_tiles(hp, 48);
-  const size_t maxtiles = std::max(tiles48.tiles.size(), tiles64.tiles.size());
+  size_t count48 = 0, count64 = 0;  // 128-wide panels have fewer
+  for (const PartDesc& d : hp.parts) {
+    count48 += part_tiles(d, 48);
+    count64 += part_tiles(d, 64);
+  }
+  const size_t maxtiles = std::max(count48, count64);
   double* x0 = (double*)workspace("gp_x0", sizeof(double) * off, &st);
   double* x1 = (double*)workspace("gp_x1", sizeof(double) * off, &st);
-  // iters x ntiles loop partials and iters x 8 queue tickets, + one slice each
+  // iters x ntiles loop partials and iters x kTickets queue tickets, + one slice each
   // for the configuration timing
   double* d_part = (double*)workspace("gp_part", sizeof(double) * maxtiles * (iters + 1), &st);
-  int* d_tickets = (int*)workspace("gp_tickets", sizeof(int) * 8 * (iters + 1), &st);
+  int* d_tickets = (int*)workspace("gp_tickets", sizeof(int) * kTickets * (iters + 1), &st);
   double* d_vv = (double*)workspace("gp_vv", sizeof(double) * 100, &st);
   if (st) return st;
   // split-precision products (prg_set_precision FP16 / BF16 split): the
@@ -427,17 +455,17 @@ int subgraph_sp2_loop(const DMat& H, DMat rho, prg_graph_partitioning_t* gp) {
       if ((st = batched_gather(H, plan, x0, gp->mineval, gp->maxeval)) ||
           (st = batched_split_prepare(plan, x0)))
         return st;
-      const TileQueues tiles128 = make_tiles(hp, 128);
       float best = 0.f;
       for (size_t k = 0; k < scand.size(); ++k) {
         const BatchConfig& c = scand[k];
-        if ((st = upload_tiles(c.panel == 128 ? tiles128 : tiles64, c.panel, &plan))) return st;
+        const TileQueues tq = make_tiles(hp, c.panel);
+        if ((st = upload_tiles(tq, c.panel, &plan))) return st;
         plan.depth = c.depth;
         plan.kslab = c.kslab;
         float ms = 0.f;
         if ((st = batched_slots(&plan)) ||
             (st = time_step(plan, x0, x1, d_part + (size_t)iters * maxtiles,
-                            d_tickets + 8 * iters, &ms)))
+                            d_tickets + kTickets * iters, &ms)))
           return st;
         if (k == 0 || ms < best) {
           best = ms;
@@ -446,8 +474,8 @@ int subgraph_sp2_loop(const DMat& H, DMat rho, prg_graph_partitioning_t* gp) {
       }
     }
     config_cache()[skey] = cfg;
-    if ((st = upload_tiles(cfg.panel == 128 ? make_tiles(hp, 128) : tiles64, cfg.panel, &plan)))
-      return st;
+    const TileQueues tq = make_tiles(hp, cfg.panel);
+    if ((st = upload_tiles(tq, cfg.panel, &plan))) return st;
     plan.depth = cfg.depth;
     plan.kslab = cfg.kslab;
     if ((st = batched_slots(&plan))) return st;
@@ -465,11 +493,8 @@ int subgraph_sp2_loop(const DMat& H, DMat rho, prg_graph_partitioning_t* gp) {
           (!force.kslab || c.kslab == force.kslab))
         cand.push_back(c);
   } else {
-    cand.push_back(staged_is_faster(hp, tiles64.tiles.size()) ? kCandidates[1] : kCandidates[0]);
+    cand.push_back(staged_is_faster(hp) ? kCandidates[1] : kCandidates[0]);
   }
-  auto tiles_of = [&](int panel) -> TileQueues {
-    return panel == 128 ? make_tiles(hp, 128) : panel == 48 ? tiles48 : tiles64;
-  };
   if (cand.empty()) {
     set_error(ERR_ARG, "PRG_BATCH_TILE / PRG_BATCH_DEPTH / PRG_BATCH_KSLAB: no compiled batched "
                        "SP2 kernel has this configuration");
@@ -487,13 +512,13 @@ int subgraph_sp2_loop(const DMat& H, DMat rho, prg_graph_partitioning_t* gp) {
     float best = 0.f;
     for (size_t k = 0; k < cand.size(); ++k) {
       const BatchConfig& c = cand[k];
-      const TileQueues tq = tiles_of(c.panel);
+      const TileQueues tq = make_tiles(hp, c.panel);
       if ((st = upload_tiles(tq, c.panel, &plan))) return st;
       plan.depth = c.depth;
       plan.kslab = c.kslab;
       float ms = 0.f;
       if ((st = batched_slots(&plan)) ||
-          (st = time_step(plan, x0, x1, d_part + (size_t)iters * maxtiles, d_tickets + 8 * iters,
+          (st = time_step(plan, x0, x1, d_part + (size_t)iters * maxtiles, d_tickets + kTickets * iters,
                           &ms)))
         return st;
       if (k == 0 || ms < best) {
@@ -503,7 +528,7 @@ int subgraph_sp2_loop(const DMat& H, DMat rho, prg_graph_partitioning_t* gp) {
     }
     config_cache()[key] = cfg;
   }
-  const TileQueues tq = tiles_of(cfg.panel);
+  const TileQueues tq = make_tiles(hp, cfg.panel);
   if ((st = upload_tiles(tq, cfg.panel, &plan))) return st;
   plan.depth = cfg.depth;
   plan.kslab = cfg.kslab;

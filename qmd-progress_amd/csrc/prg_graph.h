@@ -15,6 +15,13 @@ struct PartDesc {
   int idx_offset;  // first entry of the part's index list in the packed index array
 };
 
+// Ticket counters of one batched launch: 8, each in a line of its own.  Every
+// workgroup polls all 8 before it ends; side by side in one line these atomics
+// took 52 us of a launch of 512 workgroups and 100 us of 1024 (17 iterations
+// over 192 parts of 32 rows: 48-wide tiles 0.90 -> 0.24 ms, 64-wide 1.70 -> 0.37).
+constexpr int kTicketStride = 32;  // ints
+constexpr int kTickets = 8 * kTicketStride;
+
 struct BatchPlan {
   int nparts = 0;
   int ntiles = 0;

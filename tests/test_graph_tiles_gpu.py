@@ -73,3 +73,28 @@ def test_padded_panels_take_staged_tiles(P, monkeypatch):
     tol = 2.0 ** (imax + 2) * k * EPS * np.sqrt(k * blocks)
     assert np.linalg.norm(rho - ref) < tol
     assert np.allclose(vv, vv_ref, rtol=0, atol=tol * np.sqrt(k * blocks))
+
+
+@pytest.mark.parametrize("k,parts,panel", [(64, 640, 64), (80, 560, 48), (128, 512, 64),
+                                           (144, 432, 48), (256, 512, 64)])
+def test_tiles_of_uniform_parts(P, k, parts, panel):
+    """The rule's choice where the padding decides (64, 128 and 256 rows waste
+    nothing on 64-wide panels, 80 and 144 a quarter or more), and the result."""
+    blocks, imax = -(-parts // k), 3
+    n = k * blocks
+    print(f"[subgraph rule] parts={parts} of {k} rows", flush=True)
+    rng = np.random.default_rng(k)
+    h = np.zeros((n, n))
+    for b in range(blocks):
+        a = rng.standard_normal((k, k))
+        h[b * k:(b + 1) * k, b * k:(b + 1) * k] = (a + a.T) / 2
+    g = np.where(h != 0.0, 1.0, 0.0)
+    lo, hi = O.gershgorin(h)
+    cores = [[i] for i in range(parts)]
+    rho, vv = P.subgraph_sp2_loop(h, g, P.set_partition(cores, n), [1, 0, 1], imax, lo, hi)
+    assert P.subgraph_config()[:3] == (panel, 1, 16)
+    x = (hi * np.eye(n) - h) / (hi - lo)
+    for s in (1, 0, 1):
+        x = x @ x if s else 2 * x - x @ x
+    tol = 2.0 ** (imax + 2) * k * EPS * np.sqrt(n)
+    assert np.linalg.norm((rho - 2 * x)[:parts]) < tol
