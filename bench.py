@@ -470,7 +470,9 @@ def graph_bench(args, P, torch, np):
                   "count": sum(batched_tile_count(m, panel) for m in ls),
                   "launch": {0: "eager", 1: "captured hipGraph", 2: "hipGraph replay"}[launch]},
         "roofline": {"bound": "mfma",
-                     "kernel": (f"batched_sp2_kernel (FP64 MFMA, {panel}-wide panels)"
+                     "kernel": ((f"batched_sp2_kernel (FP64 MFMA, {panel}-wide panels)"
+                                 if panel != 48 else
+                                 "batched_sp2_direct_kernel (FP64 MFMA, 48 x 48 tiles)")
                                 if args.graph_precision == "fp64" else
                                 f"batched split-product kernel ({args.graph_precision}, 3 "
                                 f"16-bit products per tile)"),
@@ -481,7 +483,7 @@ def graph_bench(args, P, torch, np):
                      "frac": achieved / PEAK["fp64_tflops" if args.graph_precision == "fp64"
                                              else "fp16_tflops"],
                      "traffic": traffic_bytes("graph", n, None, args.water)
-                     if (panel, depth, kslab, args.graph_precision) == (64, 2, 16, "fp64")
+                     if (panel, depth, kslab, args.graph_precision) == (48, 1, 16, "fp64")
                      else None,
                      "algorithmic_tflops": alg / loop_s / 1e12,
                      "note": "executed MFMA work of the padded upper-triangle tiles per "

@@ -2,6 +2,7 @@
 --gpus is a JSON error line and a non-zero exit, not a silent fallback), and
 the helpers that turn the committed counter summaries into roofline traffic."""
 import json
+import re
 import subprocess
 import sys
 from pathlib import Path
@@ -34,6 +35,15 @@ def test_traffic_entries_resolve_for_the_headline_and_graph_kernels():
     assert bench.traffic_bytes("int8crt", 8192, 11, 803) is None
     assert bench.crt_kernel_name(944) == "crt_product_persistent_kernel"
     assert bench.crt_kernel_name(804) == "crt_product_kernel"
+
+
+def test_traffic_entries_name_kernels_of_the_library():
+    """A summary of a kernel that is gone says nothing about the present one."""
+    entries = json.loads((ROOT / "profiles" / "traffic.json").read_text())["kernels"]
+    source = "".join(f.read_text() for f in (ROOT / "qmd-progress_amd" / "csrc").glob("*.hip"))
+    assert entries
+    for e in entries:
+        assert re.search(rf"\bvoid {e['kernel'].split('<')[0]}\(", source), e["kernel"]
 
 
 @pytest.mark.parametrize("flag", ["--water", "--graph-precision"])
