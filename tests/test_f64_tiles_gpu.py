@@ -8,8 +8,6 @@ order, so it may differ by n eps sum_k |a_ik b_kj| (twice that is allowed)."""
 import numpy as np
 import pytest
 
-import progress_oracle as O
-
 pytestmark = pytest.mark.gpu
 
 SIZES = [1, 2, 15, 17, 33, 47, 100, 129, 352, 385, 500, 640, 701, 1000, 1153, 1500, 2305]
@@ -104,3 +102,71 @@ def test_response_steps(P, n):
     assert np.linalg.norm(rho - 2 * c @ c.T) < 1e-9
     assert np.linalg.norm(rsp - ref) < 1e-7 * np.linalg.norm(ref)
     assert np.array_equal(rsp, rsp.T)
+
+
+def test_response_steps_with_their_own_bookkeeping_launch(P, n=2320):
+    """Above 1280 tiles (leading dimension 2432 on) the response's step launch
+    neither absorbs nor plans.  H = Q diag(e) Q with the reflection
+    Q = I - 2 v v^T: density and response are known without an eigensolver."""
+    print(f"[response] n={n}", flush=True)
+    rng = np.random.default_rng(n)
+    v = rng.standard_normal(n)
+    v /= np.linalg.norm(v)
+    e = np.concatenate([rng.uniform(-3, -1, n // 2), rng.uniform(1, 3, n - n // 2)])
+
+    def conjugate(m):
+        """Q m Q."""
+        m = m - 2 * np.outer(v, v @ m)
+        return m - 2 * np.outer(m @ v, v)
+
+    h = conjugate(np.diag(e))
+    h = 0.5 * (h + h.T)
+    h1 = rng.standard_normal((n, n)) / np.sqrt(n)
+    h1 = 0.5 * (h1 + h1.T)
+    rho, rsp = P.compute_response_sp2(h, h1, (n // 2) / n, 1, 100, "Abs", 1e-10)
+    f = (np.arange(n) < n // 2).astype(float)
+    de = e[:, None] - e[None, :]
+    quotient = np.where(f[:, None] != f[None, :], (f[:, None] - f[None, :]) / np.where(de, de, 1.0), 0.0)
+    ref = 2 * conjugate(conjugate(h1) * quotient)
+    assert np.linalg.norm(rho - 2 * conjugate(np.diag(f))) < 1e-9
+    assert np.linalg.norm(rsp - ref) < 1e-7 * np.linalg.norm(ref)
+    assert np.array_equal(rsp, rsp.T)
+
+
+@pytest.mark.parametrize("n", [700, 2320])
+def test_thresholded_steps(P, n, thr=1e-6):
+    """The sparse formats' thresholding, with the bookkeeping in the step's
+    launch (700) and in its own (2320), against the elementwise rule."""
+    import torch
+    print(f"[thresholded steps] n={n}", flush=True)
+    i = np.arange(n)
+    d = np.abs(i[:, None] - i[None, :])
+    rng = np.random.default_rng(n)
+    h = -np.exp(-d / 8.0) * (1.0 + 0.1 * rng.standard_normal((n, n)))
+    h[d > 64] = 0.0
+    h = 0.5 * (h + h.T)
+    pp = [1, 0, 1, 1, 0]
+    ppa, vv, ic = P._ivec(len(pp), pp), P._dvec(len(pp)), P._ivec(1, [len(pp)])
+    rho = P._h_rho(P.lib().prg_sp2_alg2_seq, h, thr, P._ip(ppa), P._ip(ic), P._dp(vv), 0,
+                   matrix_type=P.ELLPACK)
+    r = np.abs(h).sum(0) - np.abs(np.diag(h))
+    lo, hi = (np.diag(h) - r).min(), (np.diag(h) + r).max()
+
+    def drop(a):
+        return torch.where(a.abs() > thr, a, torch.zeros_like(a))
+
+    x = torch.from_numpy((hi * np.eye(n) - h) / (hi - lo)).cuda()
+    idem = []
+    for s in pp:
+        y = drop(x @ x)
+        idem.append(float((x - y).norm()))
+        x = drop(y if s else 2 * x - y)
+    got = torch.from_numpy(rho.copy(order="C")).cuda()
+    diff = (got - 2 * x).abs()
+    zeros = int((x == 0).sum())
+    assert n < zeros < n * n  # the threshold decides, and not everywhere
+    # an entry whose sums end on both sides of the threshold may be dropped in
+    # one of them only, which moves what it enters by as much
+    assert int((diff > 1e-12).sum()) <= n and float(diff.max()) <= 8 * thr
+    assert np.allclose(np.asarray(vv[:len(pp)]), idem, rtol=0, atol=1e-9)
+    assert bool((got == got.T).all())
