@@ -223,7 +223,8 @@ def main():
             r["product_kernel_ms"] = kms
             r["product_kernel_launches"] = pcnt if nmod else cnt
             r["product_kernel_fp64_equiv_tflops"] = 2.0 * float(n) ** 3 / (kms * 1e-3) / 1e12
-            ops = executed_ops(ld, "int8crt" if nmod else name, nmod)
+            ops = (P.sp2_step_flops(n) if name == "fp64" else
+                   executed_ops(ld, "int8crt" if nmod else name, nmod))
             r["product_kernel_mfma_ops"] = ops
             r["product_kernel_mfma_tops"] = ops / (kms * 1e-3) / 1e12
             if nmod:
@@ -779,26 +780,17 @@ def fermi_adjoint_bench(args, P, torch, np):
            "cpu_baseline": None, "roofline": None})
 
 
-def fp64_tile_edge(ld):
-    """Tile edge of the FP64 step kernel at a leading dimension: the library's
-    cost rule (prg_f64_tile.h, best_edge)."""
-    def cost(e):
-        nb = -(-ld // e)
-        return -(-(nb * (nb + 1) // 2) // 256) * e * e * {48: 1.0, 32: 1.1, 16: 2.0}[e]
-    return min((48, 32, 16), key=cost)
-
-
 def executed_ops(ld, mode, moduli):
-    """MFMA operations of one symmetric SP2 product launch: upper-triangle
-    tiles of the FP64 kernel's edge (fp64), 128x128 tiles (f16split, bf16split;
+    """MFMA operations of one symmetric SP2 product launch of the
+    mixed-precision modes: upper-triangle 128x128 tiles (f16split, bf16split;
     the few whose last round is cut into quarters counted whole) or 256x256
     tiles over the residue planes' leading dimension rounded up to 256
-    (int8crt)."""
-    tm = {"int8crt": 256, "fp64": fp64_tile_edge(ld)}.get(mode, 128)
+    (int8crt).  The FP64 step's come from the library (sp2_step_flops)."""
+    tm = 256 if mode == "int8crt" else 128
     kd = ((ld + 255) // 256) * 256 if mode == "int8crt" else ld
     nt = -(-kd // tm)
     per_pass = nt * (nt + 1) // 2 * 2.0 * tm * tm * kd
-    return per_pass * {"fp64": 1, "f16split": 3, "bf16split": 3, "int8crt": moduli}[mode]
+    return per_pass * {"f16split": 3, "bf16split": 3, "int8crt": moduli}[mode]
 
 
 def crt_kernel_name(config):

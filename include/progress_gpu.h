@@ -425,10 +425,14 @@ int prg_get_int8_moduli(void);
  * forced with the environment variable PRG_CRT_CONFIG.  0 before any int8
  * product.  Measurement support; no reference counterpart. */
 int prg_gpu_int8_waves(void);
-/* K slices of the FP64 SP2 step at size N: 1, the step is one kernel
- * (sp2_step_kernel) at every size.  Measurement support; no reference
- * counterpart. */
+/* K slices of the FP64 SP2 step at size N: 1, as the product and its update
+ * are one kernel (sp2_step_kernel) at every size; kept for existing callers.
+ * Measurement support; no reference counterpart. */
 int prg_gpu_sp2_split_slices(int N);
+/* FP64 MFMA flops that one SP2 step executes at size N (the upper-triangle
+ * tiles of the edge it takes there, K up to N's multiple of 32).  Measurement
+ * support; no reference counterpart. */
+double prg_gpu_sp2_step_flops(int N);
 /* Forces the int8 CRT product kernel configuration (one of the codes above;
  * 0 returns to timing them per size).  Returns a status (1 for an unknown
  * code).  Test and measurement support; no reference counterpart. */

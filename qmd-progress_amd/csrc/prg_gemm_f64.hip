@@ -402,6 +402,18 @@ void launch_gemm(const GemmArgs& g, int nb, bool b_as_stored, int fuse) {
     launch_gemm_fused<S, false>(g, nb, fuse);
 }
 
+// The tiles of a product.
+struct GemmShape {
+  int edge, tiles, kdim;
+  double flops() const { return (double)tiles * 2.0 * edge * edge * kdim; }
+};
+GemmShape gemm_shape(int n, int ld, bool sym, bool b_symmetric) {
+  const bool on_staged = !sym && !b_symmetric && f64tile::full_is_staged(ld);
+  const int edge = on_staged ? staged::BM : f64tile::tile_edge(ld, sym);
+  // the padding of the operands is zero, so K ends at n's chunk
+  return GemmShape{edge, f64tile::tile_count(ld, edge, sym), (n + 31) / 32 * 32};
+}
+
 }  // namespace
 
 int gemm(int npair, const DMat* A, const DMat* B, double alpha, double beta, const DMat* Cin,
@@ -431,13 +443,11 @@ int gemm(int npair, const DMat* A, const DMat* B, double alpha, double beta, con
     g.A[p] = A[p < npair ? p : 0].p;
     g.B[p] = B[p < npair ? p : 0].p;
   }
-  const bool on_staged = !sym && !b_symmetric && f64tile::full_is_staged(ld);
-  const int edge = on_staged ? staged::BM : f64tile::tile_edge(ld, sym != 0);
+  const GemmShape shape = gemm_shape(C.n, ld, sym != 0, b_symmetric);
   g.npair = npair;
   g.ld = ld;
-  // the padding of the operands is zero, so K ends at n's chunk
-  g.kdim = (C.n + 31) / 32 * 32;
-  g.nt = (ld + edge - 1) / edge;
+  g.kdim = shape.kdim;
+  g.nt = (ld + shape.edge - 1) / shape.edge;
   g.n = C.n;
   g.sym = sym;
   g.alpha = alpha;
@@ -447,20 +457,26 @@ int gemm(int npair, const DMat* A, const DMat* B, double alpha, double beta, con
   g.C = C.p;
   g.dotE = dotE ? dotE->p : nullptr;
   g.part = d_part;
-  const int nb = f64tile::tile_count(ld, edge, sym != 0);
+  const int nb = shape.tiles;
   if (ntiles) *ntiles = nb;
-  if (on_staged) {
+  if (shape.edge == staged::BM) {
     hipLaunchKernelGGL(gemm_staged_kernel, dim3(nb), dim3(staged::NT), 0, stream(), g);
     PRG_HIP_CHECK(hipGetLastError());
     return OK;
   }
   const int fuse = (beta != 0.0 ? 1 : 0) | (dotE ? 2 : 0);
 #define PRG_CALL(S) launch_gemm<S>(g, nb, !b_symmetric, fuse)
-  PRG_F64_SHAPE_DISPATCH(edge, PRG_CALL)
+  PRG_F64_SHAPE_DISPATCH(shape.edge, PRG_CALL)
 #undef PRG_CALL
   PRG_HIP_CHECK(hipGetLastError());
   return OK;
 }
+
+double gemm_flops(int n, int ld, bool sym, bool b_symmetric) {
+  return gemm_shape(n, ld, sym, b_symmetric).flops();
+}
+
+double sp2_step_flops(int n, int ld) { return gemm_shape(n, ld, true, true).flops(); }
 
 int gemm_tiles(int ld, int sym) {
   return f64tile::tile_count(ld, f64tile::tile_edge(ld, sym != 0), sym != 0);
@@ -477,10 +493,11 @@ int sp2_step(const DMat& x0, const DMat& x1, const DMat* d0, const DMat* d1, con
   g.dbuf[0] = d0 ? d0->p : nullptr;
   g.dbuf[1] = d1 ? d1->p : nullptr;
   g.ld = x0.ld;
-  g.kdim = (x0.n + 31) / 32 * 32;
-  const int edge = f64tile::tile_edge(x0.ld, true);
+  const GemmShape shape = gemm_shape(x0.n, x0.ld, true, true);
+  const int edge = shape.edge;
+  g.kdim = shape.kdim;
   g.nt = (x0.ld + edge - 1) / edge;
-  g.ntiles = f64tile::tile_count(x0.ld, edge, true);
+  g.ntiles = shape.tiles;
   g.lazy = link.part != nullptr;
   g.link = link;
   g.part = d_part;

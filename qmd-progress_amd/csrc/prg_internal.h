@@ -160,7 +160,10 @@ int reduce_partials(const double* d_part, int nblocks, int nq, double* d_out);
 int gemm(int npair, const DMat* A, const DMat* B, double alpha, double beta, const DMat* Cin,
          double gamma, DMat C, int sym, double* d_part, int* ntiles, const DMat* dotE,
          bool b_symmetric);
-int gemm_tiles(int ld, int sym);  // records of partial sums it writes
+int gemm_tiles(int ld, int sym);  // records of partial sums it writes (at most)
+// MFMA flops that one product and one SP2 step execute.
+double gemm_flops(int n, int ld, bool sym, bool b_symmetric);
+double sp2_step_flops(int n, int ld);
 
 // Fused SP2 step in one launch: the previous step's sums are absorbed and the
 // next step planned (link; see prg_plan.h), Y = X*X, then per the planned

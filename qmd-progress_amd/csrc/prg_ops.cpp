@@ -19,19 +19,19 @@ int trace_mult_kernel_launch(const DMat& X, const DMat& Y, double* d_part, int* 
 namespace ops {
 
 // Products issued through mm / mm2 since the last reset: count, algorithmic
-// flops (2 n^3 each), FP64 MFMA flops executed (symmetric products compute
-// the upper-triangle 128 x 128 tiles only) and int8 MFMA operations executed
+// flops (2 n^3 each), FP64 MFMA flops executed (the tiles that the product is
+// cut into, the upper triangle's of a symmetric one) and int8 MFMA operations executed
 // (int8 CRT products: upper-triangle 256 x 256 tiles of the padded size, once
 // per modulus).  BF16 split products count in the first two only.
 namespace {
 double g_products = 0.0, g_alg_flops = 0.0, g_exec_flops = 0.0, g_int8_ops = 0.0;
 int g_product_precision = PRG_PREC_FP64;
 
-void count_products(int nprod, const DMat& C, bool sym) {
-  const double n = C.n, ld = C.ld, nt = C.ld / kTile;
+void count_products(int nprod, const DMat& C, bool sym, bool b_symmetric) {
+  const double n = C.n;
   g_products += nprod;
   g_alg_flops += nprod * 2.0 * n * n * n;
-  g_exec_flops += nprod * (sym ? nt * (nt + 1) / 2 * 2.0 * kTile * kTile * ld : 2.0 * ld * ld * ld);
+  g_exec_flops += nprod * gemm_flops(C.n, C.ld, sym, b_symmetric);
 }
 
 void count_crt_product(const DMat& C, int np) {
@@ -122,7 +122,7 @@ int mm(const DMat& A, const DMat& B, DMat C, bool sym, double alpha, double beta
   } else {
     if ((st = gemm(1, &A, &B, alpha, beta, Cin, gamma, C, sym ? 1 : 0, part, &nt, dotE, sym)))
       return st;
-    count_products(1, C, sym);
+    count_products(1, C, sym, sym);
   }
   if (sums) {
     double h[4];
@@ -137,7 +137,7 @@ int mm(const DMat& A, const DMat& B, DMat C, bool sym, double alpha, double beta
 int mm_symmetric_result(const DMat& A, const DMat& B, DMat C) {
   int nt = 0;
   const int st = gemm(1, &A, &B, 1.0, 0.0, nullptr, 0.0, C, 1, nullptr, &nt, nullptr, false);
-  if (!st) count_products(1, C, true);
+  if (!st) count_products(1, C, true, false);
   return st;
 }
 
@@ -150,7 +150,7 @@ int mm2(const DMat& A0, const DMat& B0, const DMat& A1, const DMat& B1, DMat C, 
   int nt = 0;
   if ((st = gemm(2, A, B, alpha, beta, Cin, gamma, C, sym ? 1 : 0, part, &nt, nullptr, sym)))
     return st;
-  count_products(2, C, sym);
+  count_products(2, C, sym, sym);
   if (sums) {
     double h[4];
     if ((st = fetch(part, nt, 4, h))) return st;

@@ -98,6 +98,7 @@ def lib():
         "prg_gpu_sp2_alg2_device": (i, [i, vp, vp, d, i, i, cp, d, i, ip, ip]),
         "prg_gpu_padded_ld": (i, [i]),
         "prg_gpu_sp2_split_slices": (i, [i]),
+        "prg_gpu_sp2_step_flops": (d, [i]),
         "prg_gpu_timing": (None, [i]),
         "prg_equalPartition": (None, [vp, i, i]),
         "prg_filePartition": (None, [vp, cp]),
@@ -277,8 +278,13 @@ def set_int8_config(config: int):
 
 
 def sp2_split_slices(n: int) -> int:
-    """K slices of the FP64 SP2 step at size n (1: the fused one-kernel step)."""
+    """K slices of the FP64 SP2 step at size n (1 at every size)."""
     return int(lib().prg_gpu_sp2_split_slices(n))
+
+
+def sp2_step_flops(n: int) -> float:
+    """FP64 MFMA flops that one SP2 step executes at size n."""
+    return float(lib().prg_gpu_sp2_step_flops(n))
 
 
 def int8_waves() -> int:

@@ -170,3 +170,34 @@ def test_thresholded_steps(P, n, thr=1e-6):
     assert int((diff > 1e-12).sum()) <= n and float(diff.max()) <= 8 * thr
     assert np.allclose(np.asarray(vv[:len(pp)]), idem, rtol=0, atol=1e-9)
     assert bool((got == got.T).all())
+
+
+# (n, tiles of the upper triangle, edge): the edges of prg_f64_tile.h over the
+# leading dimensions 256, 768, 1024 and 3072
+@pytest.mark.parametrize("n,tiles,edge", [(129, 136, 16), (700, 300, 32), (1000, 253, 48),
+                                          (2999, 2080, 48)])
+def test_counted_flops_of_symmetric_products(P, n, tiles, edge):
+    """The executed flops are those of the launched tiles, K up to n's multiple
+    of 32."""
+    import torch
+    ld = P.padded_ld(n)
+    a = torch.zeros((ld, ld), dtype=torch.float64, device="cuda")
+    a[:n, :n] = torch.eye(n, dtype=torch.float64, device="cuda")
+    expected = tiles * 2.0 * edge * edge * (-(-n // 32) * 32)
+    P.gemm_counters(reset=True)
+    P.symmetric_product_device(a, a, torch.empty_like(a), n)
+    assert P.gemm_counters(reset=True) == (1.0, 2.0 * n ** 3, expected)
+    assert P.sp2_step_flops(n) == expected
+
+
+# full products: 32-wide tiles over ld 1024, staged 128-wide ones over 4096
+@pytest.mark.parametrize("n,tiles,edge", [(1000, 1024, 32), (4060, 1024, 128)])
+def test_counted_flops_of_full_products(P, n, tiles, edge):
+    m, out = P.Matrix.from_numpy(np.eye(n)), P.Matrix.zeros(n)
+    P.gemm_counters(reset=True)
+    P.lib().prg_orthogonalize(m.h, m.h, out.h, 0.0, b"dense", 0)
+    products, alg, executed = P.gemm_counters(reset=True)
+    assert products == 2.0 and alg == 4.0 * n ** 3
+    assert executed == 2 * tiles * 2.0 * edge * edge * (-(-n // 32) * 32)
+    m.close()
+    out.close()
