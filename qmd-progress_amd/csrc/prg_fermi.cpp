@@ -185,8 +185,18 @@ double g_last_mu = 0.0;
 double g_resp_mu0 = 0.0, g_resp_mu[3] = {0.0, 0.0, 0.0};
 
 // P0 = (0.5 + cnst mu) I - cnst H   (prg_normalize_implicit_fermi)
+// (BF16 products take P by one triangle: a value of the other one that is not
+// finite, which FP64 products pass on to the first residual, is looked for.)
 int normalize_if(const DMat& H, double cnst, double mu, DMat P) {
-  return ops::lin(H, -cnst, nullptr, 0.0, 0.5 + cnst * mu, P);
+  const bool check = ops::product_precision() == PRG_PREC_BF16SPLIT;
+  Sums s;
+  const int st = ops::lin(H, -cnst, nullptr, 0.0, 0.5 + cnst * mu, P, check ? &s : nullptr);
+  if (st) return st;
+  if (check && !std::isfinite(s.fro2)) {
+    set_error(ERR_NUMERIC, "implicit Fermi: non-finite Hamiltonian");
+    return ERR_NUMERIC;
+  }
+  return OK;
 }
 
 }  // namespace
