@@ -14,7 +14,10 @@
  *     one character by value, so through its C path "Rel" never matches;
  *   - arrays (pp, vv) are plain pointers with the lengths stated per call;
  *   - out-parameters the reference loses through `value` (mu, occiter,
- *     totns) are pointers.
+ *     totns) are pointers;
+ *   - Hamiltonians, perturbations and overlaps are symmetric, and products of
+ *     them may read either triangle.  (FP64 SP2 of up to 128 rows squares any
+ *     matrix.)
  *
  * The matrix handle: BML (lanl/bml) is not linked, so the
  * library carries its own bml_matrix_t holding a dense double-precision

@@ -8,7 +8,11 @@ order, so it may differ by n eps sum_k |a_ik b_kj| (twice that is allowed)."""
 import numpy as np
 import pytest
 
+import progress_oracle as O
+
 pytestmark = pytest.mark.gpu
+
+EPS = np.finfo(float).eps
 
 SIZES = [1, 2, 15, 17, 33, 47, 100, 129, 352, 385, 500, 640, 701, 1000, 1153, 1500, 2305]
 
@@ -102,6 +106,32 @@ def test_response_steps(P, n):
     assert np.linalg.norm(rho - 2 * c @ c.T) < 1e-9
     assert np.linalg.norm(rsp - ref) < 1e-7 * np.linalg.norm(ref)
     assert np.array_equal(rsp, rsp.T)
+
+
+@pytest.mark.parametrize("thr,kind", [(0.0, None), (1e-3, "ELLPACK")])
+@pytest.mark.parametrize("n", [2, 15, 16, 17, 33, 100, 127, 128])
+def test_replayed_steps_of_a_matrix_without_symmetry(P, n, thr, kind):
+    """Up to 128 rows a matrix need not be symmetric: its steps are those of the
+    dense product (each at most doubles the error and adds 2 n eps of
+    || |X|^2 ||), thresholded in the sparse formats."""
+    rng = np.random.default_rng(n)
+    h = rng.standard_normal((n, n)) / np.sqrt(n)
+    pp = [1, 0, 0, 1]
+    ppa, vv, ic = P._ivec(len(pp), pp), P._dvec(len(pp)), P._ivec(1, [len(pp)])
+    got = P._h_rho(P.lib().prg_sp2_alg2_seq, h, thr, P._ip(ppa), P._ip(ic), P._dp(vv), 0,
+                   matrix_type=getattr(P, kind) if kind else None)
+    lo, hi = O.gershgorin(h)
+    x = (hi * np.eye(n) - h) / (hi - lo)
+    drop = lambda a: np.where(np.abs(a) > thr, a, 0.0)
+    bound, idem = 0.0, []
+    for s in pp:
+        bound = 3 * bound * max(1.0, np.linalg.norm(x)) + 2 * n * EPS * np.linalg.norm(
+            np.abs(x) @ np.abs(x))
+        y = drop(x @ x)
+        idem.append(np.linalg.norm(x - y))
+        x = drop(y if s else 2 * x - y)
+    assert np.linalg.norm(got - 2 * x) <= 2 * bound
+    assert np.allclose(np.asarray(vv[:len(pp)]), idem, rtol=0, atol=2 * bound + 1e-14)
 
 
 def test_response_steps_with_their_own_bookkeeping_launch(P, n=2320):
