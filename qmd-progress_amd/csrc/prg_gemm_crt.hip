@@ -1488,7 +1488,9 @@ struct HeldOperand {
   int np = 0, ld = 0;
 };
 HeldOperand g_held[2];
-const char* const kHeldPlanes[2] = {"crtg_planes_held", "crtg_planes_held2"};
+// The second one's planes take the set that a product of two operands that are
+// not held needs, which ends its validity; one such operand takes the other.
+const char* const kHeldPlanes[2] = {"crtg_planes_held", "crtg_planes_a"};
 
 int held_slot(const double* p) {
   for (int i = 0; i < 2; ++i)
@@ -1537,7 +1539,10 @@ int crt_gemm(const DMat& A, const DMat& B, DMat C, double alpha, double beta, co
   const bool same = (A.p == B.p);
   const int ha = held_slot(A.p), hb = same ? -1 : held_slot(B.p);
   int st = OK;
-  int8_t* pa_planes = (int8_t*)workspace(ha >= 0 ? kHeldPlanes[ha] : "crtg_planes_a",
+  const bool both = ha < 0 && hb < 0 && !same;
+  if (both) g_held[1].valid = false;
+  const char* scratch_a = both ? "crtg_planes_a" : "crtg_planes_b";
+  int8_t* pa_planes = (int8_t*)workspace(ha >= 0 ? kHeldPlanes[ha] : scratch_a,
                                          (size_t)np * plane, &st);
   int8_t* pb_planes = same ? nullptr
                            : (int8_t*)workspace(hb >= 0 ? kHeldPlanes[hb] : "crtg_planes_b",

@@ -629,7 +629,8 @@ struct SplitHeld {
   int ld = 0;
 };
 SplitHeld g_split_held[2];
-const char* const kSplitHeldPlanes[2] = {"splitg_planes_held", "splitg_planes_held2"};
+// (the second one's planes: as in the int8 products)
+const char* const kSplitHeldPlanes[2] = {"splitg_planes_held", "splitg_planes_a"};
 
 int split_held_slot(const double* p) {
   for (int i = 0; i < 2; ++i)
@@ -670,7 +671,10 @@ int split_gemm(const DMat& A, const DMat& B, DMat C, double alpha, double beta, 
   const bool same = (A.p == B.p);
   const int ha = split_held_slot(A.p), hb = same ? -1 : split_held_slot(B.p);
   int st = OK;
-  char* pa = (char*)workspace(ha >= 0 ? kSplitHeldPlanes[ha] : "splitg_planes_a", 2 * plane, &st);
+  const bool both = ha < 0 && hb < 0 && !same;
+  if (both) g_split_held[1].valid = false;
+  const char* scratch_a = both ? "splitg_planes_a" : "splitg_planes_b";
+  char* pa = (char*)workspace(ha >= 0 ? kSplitHeldPlanes[ha] : scratch_a, 2 * plane, &st);
   char* pb = same ? pa
                   : (char*)workspace(hb >= 0 ? kSplitHeldPlanes[hb] : "splitg_planes_b", 2 * plane,
                                      &st);
