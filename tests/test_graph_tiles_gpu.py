@@ -98,3 +98,31 @@ def test_tiles_of_uniform_parts(P, k, parts, panel):
         x = x @ x if s else 2 * x - x @ x
     tol = 2.0 ** (imax + 2) * k * EPS * np.sqrt(n)
     assert np.linalg.norm((rho - 2 * x)[:parts]) < tol
+
+
+def test_direct_tiles_round_no_worse_than_staged_ones(P, monkeypatch, n=300, imax=6):
+    """Against the same steps in extended precision (64-bit mantissas): the sums
+    over four waves' quarters of K leave an error within that of the staged
+    tiles' sequential ones, plus a quarter for the input's luck."""
+    if np.finfo(np.longdouble).nmant < 63:
+        pytest.skip("no extended precision here")
+    rng = np.random.default_rng(n)
+    a = rng.standard_normal((n, n))
+    h = (a + a.T) / 2
+    lo, hi = O.gershgorin(h)
+    seq = [1, 0, 0, 1, 0, 1]
+    x = (np.longdouble(hi) * np.eye(n, dtype=np.longdouble) - h) / (np.longdouble(hi) - lo)
+    for s in seq:
+        x = x.dot(x) if s else 2 * x - x.dot(x)
+    err = {}
+    for panel in ("48", "64"):
+        monkeypatch.setenv("PRG_BATCH_TILE", panel)
+        monkeypatch.setenv("PRG_BATCH_DEPTH", "1")
+        monkeypatch.setenv("PRG_BATCH_KSLAB", "16")
+        gp = P.set_partition([list(range(n))], n)
+        rho, _ = P.subgraph_sp2_loop(h, np.ones((n, n)), gp, seq, imax, lo, hi)
+        assert P.subgraph_config()[0] == int(panel)
+        err[panel] = float(np.sqrt(((rho - 2 * x) ** 2).sum()) / np.sqrt((4 * x ** 2).sum()))
+    print(f"[subgraph rounding] error of 48-wide tiles {err['48']:.2e}, staged {err['64']:.2e}",
+          flush=True)
+    assert err["48"] <= 1.25 * err["64"]
