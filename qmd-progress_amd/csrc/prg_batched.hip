@@ -213,7 +213,7 @@ __global__ __launch_bounds__(NT, WIDE ? 2 : 4) void batched_sp2_kernel(BatchArgs
 // split over the workgroup's four waves (prg_f64_tile.h): no staging and no
 // barrier in the main loop, two workgroups per CU, the next ticket fetched
 // under the product.  Bound by the matrix cores and the last tiles of a queue;
-// 16 parts of 1151-1712 rows take 1.31 ms per iteration, 1.42 with the staged
+// 24 parts of 1151-1712 rows take 1.27 ms per iteration, 1.42 with the staged
 // 64 x 64 tiles; a last iteration computes its core rows' tiles only.
 __global__ __launch_bounds__(NT, 2) void batched_sp2_direct_kernel(BatchArgs g) {
   typedef f64tile::S48 S;

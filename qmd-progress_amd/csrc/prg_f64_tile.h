@@ -392,7 +392,9 @@ typedef Shape<3> S48;
 // 700 23.6 / 19.1 / 21.3; 1024 - / 31.2 / 25.8; 1300 - / 49.4 / 51.2; 1500 - /
 // 67.5 / 84.5; 2048 - / 158 / 148; 2600 - / 313 / 321; 4096 - / 1148 / 1067.
 // (64-, 96- and 128-wide tiles of 2 x 2 waves: 187, 152 and 262 us at 2048,
-// 1309, 1101 and 1443 us at 4096.)
+// 1309, 1101 and 1443 us at 4096.)  The response's step launches twice the
+// tiles, half of them over two products, at the edge chosen for the plain one:
+// N = 700 2 x 300 tiles of 32, 32.5 us.
 inline double edge_cost(int tiles, int e) {
   const double rounds = (tiles + 255) / 256;
   return rounds * e * e * (e == 48 ? 1.0 : e == 32 ? 1.1 : 2.0);

@@ -13,9 +13,6 @@
 // sums ||X - X^2||_F^2 (genseq) or its core-row restriction (submatrix).
 #include "prg_internal.h"
 
-#include <algorithm>
-#include <cmath>
-#include <cstdlib>
 #include "prg_f64_tile.h"
 #include "prg_plan.h"
 #include "prg_tile.h"
@@ -328,8 +325,8 @@ __device__ __forceinline__ void response_finish(const Sp2Args& g, const Sp2State
   });
 }
 
-// One SP2 step in one launch: absorb the previous step's sums and plan
-// (sp2_link, wave 0), product, update.  The current X is known before the
+// One SP2 step: absorb the previous step's sums and plan (sp2_link, wave 0; a
+// launch of its own does both above 1280 tiles), product, update.  The current X is known before the
 // plan: every step before the last toggles the buffers (g.cur), and the last
 // plans nothing after it.  So the product's first operands are on their way
 // while wave 0 plans, and (g.lazy) the other waves multiply meanwhile: the

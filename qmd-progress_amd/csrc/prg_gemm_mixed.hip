@@ -30,7 +30,6 @@ using tile::sym_tile_banded;
 using tile::xcd_remap;
 
 typedef float f4 __attribute__((ext_vector_type(4)));
-typedef int i4 __attribute__((ext_vector_type(4)));
 
 // The two 16-bit split formats: element type, lo scale (2^(mantissa bits)),
 // and the 16x16x32 MFMA with FP32 accumulation.
@@ -536,7 +535,9 @@ __global__ __launch_bounds__(NT) void split_f16_kernel(const double* __restrict_
 // pass, last rounds whole / quartered: 1024 (36 tiles) 52 / 36 us, 1920 (120)
 // 75 / 55, 2176 (153) 83 / 78, 2432 (190) 90 / 86, 2560 (210) 95 / 98; behind
 // full rounds 4096 (16) 301 / 253, 4352 (83) 322 / 307, 4608 (154) 344 / 343,
-// 4736 (191) 362 / 362, 5888 (57) 665 / 606.
+// 4736 (191) 362 / 362, 5888 (57) 665 / 606.  Quarters gain up to about 200
+// tiles of an only round and 160 behind full ones; the smaller number serves
+// both, which leaves 4 % at 171 and 190 tiles of an only round.
 constexpr int kSlots = 2 * 256, kQuarterMax = 160;
 int split_full_tiles(int nt) {
   const int tiles = nt * (nt + 1) / 2, rest = tiles % kSlots;

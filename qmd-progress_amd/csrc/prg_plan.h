@@ -1,9 +1,10 @@
 // Device-side FP64 bookkeeping of the SP2 loop: the branch decision for the
 // next step and the absorption of a step's partial sums.  The mixed-precision
-// loops run them in a one-block kernel after each step.  The FP64 loop runs
-// them at the start of the next step's launch, in every workgroup, on an LDS
-// copy of the state header: the launch and its gap (4.5 + 1 us per step) give
-// way to about 2 us of reads that a workgroup needs anyway.  (A last-workgroup
+// loops, and the FP64 loop above 1280 tiles (leading dimension 2432 on), run
+// them in a one-block kernel after each step.  The FP64 loop of smaller
+// matrices runs them at the start of the next step's launch, in every
+// workgroup, on an LDS copy of the state header: the launch and its gap (4.5 +
+// 1 us per step) give way to about 2 us of reads that a workgroup needs anyway.  (A last-workgroup
 // absorb at the end of the step was slower than a launch of its own: the
 // device-scope fences it needs write back and invalidate the per-XCD L2s.)
 #pragma once

@@ -1,9 +1,9 @@
 // SP2 purification drivers (src/prg_sp2_mod.F90) on one GPU.
 //
 // The whole iteration runs on the device: in FP64 one launch per step (the
-// bookkeeping of the step before, the product and the update), in the
-// mixed-precision modes a product, an update and a single-workgroup
-// bookkeeping launch, enqueued in chunks.  The host reads the state
+// bookkeeping of the step before, the product and the update) up to 1280
+// tiles, above that and in the mixed-precision modes the products and updates
+// with a single-workgroup bookkeeping launch after each, enqueued in chunks.  The host reads the state
 // header of a chunk (an asynchronous copy into pinned memory) only after the
 // next chunk is enqueued, so no scalar crosses PCIe per iteration and the
 // device does not wait for the host.  Once the loop has stopped, the
