@@ -417,19 +417,24 @@ inline int tile_edge(int ld, bool sym) {
   return best_edge([&](int e) { return tile_count(ld, e, sym); });
 }
 
-// Whether a full product of operands that are not symmetric takes less time on
-// the staged 128-wide tiles (gemm_staged_kernel), two workgroups per CU: a
-// round of 512 of them takes as long as 12.95 rounds of 48-wide ones (243 us
-// against 18.7 us at K = 1000), a single round of at most 256, one per CU, 0.58
-// of that.  Z^T A Z and Z A Z^T (two products each), ms, 48-wide / staged:
+// Whether a product takes less time on the staged 128-wide tiles
+// (gemm_staged_kernel), two workgroups per CU: a round of 512 of them takes as
+// long as 12.95 rounds of 48-wide ones (243 us against 18.7 us at K = 1000) if
+// the operands are not symmetric, as 13.8 (17.6 us) if they are; a single
+// round of at most 256, one per CU, 0.58 of that.
+// Z^T A Z and Z A Z^T (two products each), ms, 48-wide / staged:
 // ld 1920 0.58, 0.54 / 0.65, 0.61; 2048 0.73, 0.65 / 0.69, 0.65; 2560 1.35,
 // 1.23 / 1.41, 1.34; 2816 1.77, 1.54 / 1.60, 1.53; 3072 2.16, 1.90 / 3.17,
 // 3.02; 4096 4.62, 4.34 / 4.45, 4.05; 5632 11.5, 11.4 / 11.0, 11.1; 6144 13.7,
 // 13.5 / 15.0, 15.0; 6400 16.5, 16.7 / 15.7, 15.7; 8192 34.2, 34.2 / 32.0, 32.0.
-inline bool full_is_staged(int ld) {
-  const int nt = ld / 128, tiles = nt * nt, edge = tile_edge(ld, false);
+// Symmetric products: 6912 4.92 / 5.07; 7936 7.6 / 7.7; 8064 8.09 / 7.85; 8192
+// 8.3 / 9.2; 9088 11.6 / 11.0; 10112 16.0 / 17.2; 11520 23.5 / 22.3; 12288 28.7
+// / 29.4.  Below 2048 staged tiles (1 to 3 rounds) the two are within 1 %.
+inline bool staged_is_faster(int ld, bool sym, bool b_symmetric) {
+  const int tiles = tile_count(ld, 128, sym), edge = tile_edge(ld, sym);
+  if (sym && (!b_symmetric || tiles < 2016)) return false;
   const double rounds = tiles <= 256 ? 0.58 : (tiles + 511) / 512;
-  return 12.95 * rounds * 48 * 48 < edge_cost(tile_count(ld, edge, false), edge);
+  return (sym ? 13.8 : 12.95) * rounds * 48 * 48 < edge_cost(tile_count(ld, edge, sym), edge);
 }
 
 #define PRG_F64_SHAPE_DISPATCH(EDGE, CALL) \

@@ -1,6 +1,6 @@
 // FP64 MFMA GEMM family for gfx950 (v_mfma_f64_16x16x4_f64) on the tiles of
 // prg_f64_tile.h: operands straight to registers, the tile edge chosen by how
-// its tiles fill the CUs.  For symmetric products (X*X, X*D + D*X, products
+// its tiles fill the CUs, or staged 128-wide tiles where those fill them better.  For symmetric products (X*X, X*D + D*X, products
 // of commuting symmetric matrices) only the upper-triangle tiles are computed;
 // the epilogue writes each tile and its transpose, so the result is exactly
 // symmetric and the executed flops are half of the algorithmic 2 N^3.
@@ -129,42 +129,40 @@ __global__ __launch_bounds__(S::NT, 2) void gemm_kernel(GemmArgs g) {
   if (g.part) block_store4<S::NT>(sums, g.part + 4 * (size_t)t);
 }
 
-// ----------------------------------------------- full products, staged tiles
-// The same C for operands that are not symmetric, one 128 x 128 tile per
-// workgroup: 16-deep slabs of both panels go through LDS with the next slab
-// in registers, four waves in a 2 x 2 grid of 4 x 4 MFMA blocks.  B is read
-// along its columns, 64 bytes per thread, where a 48-wide tile's fragments
-// take 64 bytes of each of 16 columns; with two workgroups per CU 67 TFLOP/s,
-// whatever the leading dimension.  What it costs is the tiles' size (see
-// full_is_staged).
+// --------------------------------------------------------- staged tiles
+// The same products on 128 x 128 tiles, one per workgroup: 16-deep slabs of
+// both panels go through LDS with the next slab in registers, four waves in a
+// 2 x 2 grid of 4 x 4 MFMA blocks.  B is read along its columns, 64 bytes per
+// thread, where a 48-wide tile's fragments of an operand that is not symmetric
+// take 64 bytes of each of 16 columns; with two workgroups per CU 67 to 69
+// TFLOP/s, whatever the leading dimension.  What it costs is the tiles' size
+// (see staged_is_faster).
 namespace staged {
 constexpr int BM = 128, BK = 16, NT = 256;
-constexpr int LROW = BM + 4;  // padded LDS row length in doubles
-}  // namespace staged
+struct Slabs {
+  double A[BK][BM + 4], B[BK][BM + 4];  // rows padded
+};
 
-__global__ __launch_bounds__(staged::NT, 2) void gemm_staged_kernel(GemmArgs g) {
-  using namespace staged;
+// acc = the tile (I, J) of A[0] B[0] (+ A[1] B[1]).
+__device__ __forceinline__ void product(const double* const (&A)[2], const double* const (&B)[2],
+                                        int npair, int ld, int kdim, int I, int J, Slabs& lds,
+                                        d4 (&acc)[4][4]) {
   typedef f64tile::d2 d2;
-  __shared__ double As[BK][LROW], Bs[BK][LROW];
-  const int t = xcd_remap(blockIdx.x, gridDim.x), ld = g.ld;
-  int I, J;
-  full_tile(t, g.nt, I, J);
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, wm = w & 1, wn = w >> 1;
   const int ar = (tid & 63) * 2, ak = tid >> 6;  // A: rows ar, ar + 1; k = ak + 4 q
   const int bj = tid >> 1, bk = (tid & 1) * 8;   // B: column bj; k = bk .. bk + 7
-  const int slabs = g.kdim / BK, total = slabs * g.npair;
+  const int slabs = kdim / BK, total = slabs * npair;
   d2 ra[4], rb[4];
   auto load = [&](int s) {
     const int p = s >= slabs, k0 = (s - p * slabs) * BK;
-    const double* Ap = g.A[p] + (size_t)I * BM + ar;
-    const double* Bp = g.B[p] + (size_t)(J * BM + bj) * ld + k0 + bk;
+    const double* Ap = (p ? A[1] : A[0]) + (size_t)I * BM + ar;
+    const double* Bp = (p ? B[1] : B[0]) + (size_t)(J * BM + bj) * ld + k0 + bk;
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
       ra[q] = *(const d2*)(Ap + (size_t)(k0 + ak + 4 * q) * ld);
       rb[q] = *(const d2*)(Bp + 2 * q);
     }
   };
-  d4 acc[4][4];
 #pragma unroll
   for (int m = 0; m < 4; ++m)
 #pragma unroll
@@ -174,10 +172,10 @@ __global__ __launch_bounds__(staged::NT, 2) void gemm_staged_kernel(GemmArgs g) 
     __syncthreads();
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
-      As[ak + 4 * q][ar] = ra[q].x;
-      As[ak + 4 * q][ar + 1] = ra[q].y;
-      Bs[bk + 2 * q][bj] = rb[q].x;
-      Bs[bk + 2 * q + 1][bj] = rb[q].y;
+      lds.A[ak + 4 * q][ar] = ra[q].x;
+      lds.A[ak + 4 * q][ar + 1] = ra[q].y;
+      lds.B[bk + 2 * q][bj] = rb[q].x;
+      lds.B[bk + 2 * q + 1][bj] = rb[q].y;
     }
     __syncthreads();
     if (s + 1 < total) load(s + 1);
@@ -186,9 +184,9 @@ __global__ __launch_bounds__(staged::NT, 2) void gemm_staged_kernel(GemmArgs g) 
       const int kr = kk * 4 + (lane >> 4);
       double a[4], b[4];
 #pragma unroll
-      for (int m = 0; m < 4; ++m) a[m] = As[kr][wm * 64 + m * 16 + (lane & 15)];
+      for (int m = 0; m < 4; ++m) a[m] = lds.A[kr][wm * 64 + m * 16 + (lane & 15)];
 #pragma unroll
-      for (int n = 0; n < 4; ++n) b[n] = Bs[kr][wn * 64 + n * 16 + (lane & 15)];
+      for (int n = 0; n < 4; ++n) b[n] = lds.B[kr][wn * 64 + n * 16 + (lane & 15)];
 #pragma unroll
       for (int m = 0; m < 4; ++m)
 #pragma unroll
@@ -196,28 +194,49 @@ __global__ __launch_bounds__(staged::NT, 2) void gemm_staged_kernel(GemmArgs g) 
           acc[m][n] = __builtin_amdgcn_mfma_f64_16x16x4f64(b[n], a[m], acc[m][n], 0, 0, 0);
     }
   }
-  double sums[4] = {0.0, 0.0, 0.0, 0.0};
+}
+
+// f(row, column, entry) for the lane's entries, one MFMA block at a time (the
+// loads of a block's entries are not hoisted over another's: registers).
+template <typename F>
+__device__ __forceinline__ void for_entries(const d4 (&acc)[4][4], int I, int J, F&& f) {
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int row0 = I * BM + (w & 1) * 64 + (lane & 15), col0 = J * BM + (w >> 1) * 64 + (lane >> 4);
 #pragma unroll
-  for (int m = 0; m < 4; ++m) {
-    const int row = I * BM + wm * 64 + m * 16 + (lane & 15);
+  for (int m = 0; m < 4; ++m)
 #pragma unroll
     for (int n = 0; n < 4; ++n) {
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int col = J * BM + wn * 64 + n * 16 + (lane >> 4) + 4 * r;
-        const size_t idx = row + (size_t)col * ld;
-        double v = acc[m][n][r] * g.alpha;
-        if (g.beta != 0.0) v += g.beta * g.Cin[idx];
-        const bool diag = (row == col);
-        v += (diag && row < g.n) ? g.gamma : 0.0;
-        sums[0] += diag ? v : 0.0;
-        sums[1] += v * v;
-        if (g.dotE) sums[2] += v * g.dotE[idx];
-        g.C[idx] = v;
-      }
+      for (int r = 0; r < 4; ++r) f(row0 + 16 * m, col0 + 16 * n + 4 * r, acc[m][n][r]);
+      __builtin_amdgcn_sched_barrier(0);
     }
-  }
-  if (g.part) block_store4<NT>(sums, g.part + 4 * (size_t)t);
+}
+}  // namespace staged
+
+template <bool SYM>
+__global__ __launch_bounds__(staged::NT, 2) void gemm_staged_kernel(GemmArgs g) {
+  __shared__ staged::Slabs lds;
+  const int t = xcd_remap(blockIdx.x, gridDim.x), ld = g.ld;
+  int I, J;
+  if (SYM) tile::sym_tile(t, I, J); else full_tile(t, g.nt, I, J);
+  d4 acc[4][4];
+  staged::product(g.A, g.B, g.npair, ld, g.kdim, I, J, lds, acc);
+  double sums[4] = {0.0, 0.0, 0.0, 0.0};
+  staged::for_entries(acc, I, J, [&](int row, int col, double y) {
+    if (SYM && row > col) return;  // the lower half of a diagonal tile
+    const bool diag = (row == col);
+    const double wgt = SYM && !diag ? 2.0 : 1.0;
+    const size_t idx = row + (size_t)col * ld;
+    double v = y * g.alpha;
+    if (g.beta != 0.0) v += g.beta * g.Cin[idx];
+    v += (diag && row < g.n) ? g.gamma : 0.0;
+    sums[0] += diag ? v : 0.0;
+    sums[1] += wgt * v * v;
+    if (g.dotE) sums[2] += wgt * v * g.dotE[idx];
+    g.C[idx] = v;
+    if (SYM && !diag) g.C[col + (size_t)row * ld] = v;
+  });
+  if (g.part) block_store4<staged::NT>(sums, g.part + 4 * (size_t)t);
 }
 
 // ------------------------------------------------------------- SP2 step
@@ -384,6 +403,53 @@ __global__ __launch_bounds__(S::NT, 2) void sp2_step_kernel(Sp2Args g) {
   block_store4<S::NT>(sums, g.part + 4 * (size_t)t);
 }
 
+// The step on staged tiles, planned by a launch of its own: the X update, or
+// (RESP) the response's.
+template <bool RESP>
+__global__ __launch_bounds__(staged::NT, 2) void sp2_staged_kernel(Sp2Args g) {
+  __shared__ staged::Slabs lds;
+  const Sp2State* st = g.link.in;
+  if (!st->planned || (RESP && !st->apply)) return;
+  const int ld = g.ld, apply = st->apply, sigma = st->sigma;
+  const double ca = apply ? (sigma ? 1.0 : -1.0) : 0.0, cb = apply ? (sigma ? 0.0 : 2.0) : 1.0;
+  const double* X = g.buf[g.cur];
+  const double* D = g.dbuf[g.cur];
+  const int t = xcd_remap(blockIdx.x, gridDim.x);
+  int I, J;
+  tile::sym_tile(t, I, J);
+  d4 acc[4][4];
+  if (RESP) {
+    double* Dn = const_cast<double*>(g.dbuf[g.cur ^ 1]);
+    staged::product({X, D}, {D, X}, 2, ld, g.kdim, I, J, lds, acc);
+    staged::for_entries(acc, I, J, [&](int row, int col, double y) {
+      if (row > col) return;  // X D + D X adds (r, c) and (c, r) in different orders
+      const double z = fma(cb, D[row + (size_t)col * ld], ca * y);
+      Dn[row + (size_t)col * ld] = z;
+      Dn[col + (size_t)row * ld] = z;
+    });
+    return;
+  }
+  double* Xn = const_cast<double*>(g.buf[g.cur ^ 1]);
+  const int core = st->variant == V_SUBMATRIX ? st->core : 0x7fffffff;
+  const bool mirror = (I != J);
+  const double wz = mirror ? 2.0 : 1.0;
+  double sums[4] = {0.0, 0.0, 0.0, 0.0};
+  staged::product({X, X}, {X, X}, 1, ld, g.kdim, I, J, lds, acc);
+  staged::for_entries(acc, I, J, [&](int row, int col, double y) {
+    const size_t idx = row + (size_t)col * ld;
+    const double x = X[idx], z = fma(cb, x, ca * y), d = x - y;
+    const bool diag = (row == col);
+    sums[0] += wz * z * z;
+    sums[1] += diag ? z : 0.0;
+    sums[2] += ((row < core ? 1.0 : 0.0) + (mirror && col < core ? 1.0 : 0.0)) * d * d;
+    sums[3] += diag ? y : 0.0;
+    Xn[idx] = z;
+    // on a diagonal tile the lane rewrites its own entry
+    Xn[mirror ? col + (size_t)row * ld : idx] = z;
+  });
+  block_store4<staged::NT>(sums, g.part + 4 * (size_t)t);
+}
+
 template <typename S, bool BT>
 void launch_gemm_fused(const GemmArgs& g, int nb, int fuse) {
   void (*k)(GemmArgs) = fuse == 0   ? gemm_kernel<S, BT, 0>
@@ -407,8 +473,8 @@ struct GemmShape {
   double flops() const { return (double)tiles * 2.0 * edge * edge * kdim; }
 };
 GemmShape gemm_shape(int n, int ld, bool sym, bool b_symmetric) {
-  const bool on_staged = !sym && !b_symmetric && f64tile::full_is_staged(ld);
-  const int edge = on_staged ? staged::BM : f64tile::tile_edge(ld, sym);
+  const int edge = f64tile::staged_is_faster(ld, sym, b_symmetric) ? staged::BM
+                                                                   : f64tile::tile_edge(ld, sym);
   // the padding of the operands is zero, so K ends at n's chunk
   return GemmShape{edge, f64tile::tile_count(ld, edge, sym), (n + 31) / 32 * 32};
 }
@@ -418,8 +484,12 @@ GemmShape gemm_shape(int n, int ld, bool sym, bool b_symmetric) {
 // taken as symmetric.  (N = 100: 6.8 us per step on 64 workgroups, 7.0 on the
 // 36 of one triangle.)
 bool step_is_full(int ld) { return ld == kTile; }
-GemmShape step_shape(int n, int ld) {
+GemmShape step_shape(int n, int ld, bool thresholded = false) {
   GemmShape s = gemm_shape(n, ld, true, true);
+  if (s.edge == staged::BM && thresholded) {
+    s.edge = f64tile::tile_edge(ld, true);
+    s.tiles = f64tile::tile_count(ld, s.edge, true);
+  }
   if (step_is_full(ld)) {
     s.edge = 16;
     s.tiles = f64tile::tile_count(ld, s.edge, false);
@@ -473,7 +543,8 @@ int gemm(int npair, const DMat* A, const DMat* B, double alpha, double beta, con
   const int nb = shape.tiles;
   if (ntiles) *ntiles = nb;
   if (shape.edge == staged::BM) {
-    hipLaunchKernelGGL(gemm_staged_kernel, dim3(nb), dim3(staged::NT), 0, stream(), g);
+    hipLaunchKernelGGL(sym ? gemm_staged_kernel<true> : gemm_staged_kernel<false>, dim3(nb),
+                       dim3(staged::NT), 0, stream(), g);
     PRG_HIP_CHECK(hipGetLastError());
     return OK;
   }
@@ -495,7 +566,8 @@ int gemm_tiles(int ld, int sym) {
   return f64tile::tile_count(ld, f64tile::tile_edge(ld, sym != 0), sym != 0);
 }
 
-int sp2_step_tiles(int ld) { return step_shape(ld, ld).tiles; }
+// (of the 48-wide tiles where the staged ones are fewer)
+int sp2_step_tiles(int ld) { return step_shape(ld, ld, true).tiles; }
 
 int sp2_step(const DMat& x0, const DMat& x1, const DMat* d0, const DMat* d1, const Sp2Link& link,
              double* d_part, int* ntiles, bool thresholded, int cur) {
@@ -506,7 +578,7 @@ int sp2_step(const DMat& x0, const DMat& x1, const DMat* d0, const DMat* d1, con
   g.dbuf[0] = d0 ? d0->p : nullptr;
   g.dbuf[1] = d1 ? d1->p : nullptr;
   g.ld = x0.ld;
-  const GemmShape shape = step_shape(x0.n, x0.ld);
+  const GemmShape shape = step_shape(x0.n, x0.ld, thresholded);
   const int edge = shape.edge;
   g.kdim = shape.kdim;
   g.nt = (x0.ld + edge - 1) / edge;
@@ -523,7 +595,11 @@ int sp2_step(const DMat& x0, const DMat& x1, const DMat* d0, const DMat* d1, con
                                        : sp2_step_kernel<S, false, false, F>;
     hipLaunchKernelGGL(k, dim3(d0 ? 2 * g.ntiles : g.ntiles), dim3(S::NT), 0, stream(), g);
   };
-  if (step_is_full(x0.ld)) {
+  if (edge == staged::BM) {
+    if (d0)
+      hipLaunchKernelGGL(sp2_staged_kernel<true>, dim3(g.ntiles), dim3(staged::NT), 0, stream(), g);
+    hipLaunchKernelGGL(sp2_staged_kernel<false>, dim3(g.ntiles), dim3(staged::NT), 0, stream(), g);
+  } else if (step_is_full(x0.ld)) {
     launch(f64tile::S16{}, std::true_type{});
   } else {
 #define PRG_CALL(S) launch(S{}, std::false_type{})

@@ -1,7 +1,7 @@
-"""Full FP64 products (operands that are not symmetric) at sizes that take the
-staged 128-wide tiles (leading dimensions 2048, 2816 and 3968) and at their
-neighbours that do not: products, two-product sums with an input term, the
-partial sums and <C, E>.
+"""FP64 products at sizes that take the staged 128-wide tiles and at neighbours
+that do not.  Operands that are not symmetric (leading dimensions 2048, 2816 and
+3968): products, two-product sums with an input term, the partial sums and
+<C, E>; symmetric ones (8064): products, SP2 steps and the response.
 
 Each entry of a product is a sum of n terms in another order: it may differ by
 n eps (|A| |B|) from another correct one (twice that is allowed)."""
@@ -102,3 +102,79 @@ def test_sums_and_elementwise_product(P, n=2700):
     P.implicit_fermi_adjoint_device(_padded(P, h), _padded(P, a - kappa * eye), g2, n, levels, 0.1,
                                     beta, 1e-10)
     assert float((g1 - g2).norm()) <= 1e-10 * float(g2.norm())
+
+
+def test_symmetric_products_and_steps(P, n=8010):
+    """A B + beta C + gamma I for commuting A, B through an adjoint (the two-product
+    sum), the product itself, and replayed SP2 steps, whose results are
+    symmetric to the bit."""
+    print(f"[staged symmetric] n={n}", flush=True)
+    import torch
+    x = _random(n, n, 1.0 / n ** 0.5)
+    h = 0.5 * (x + x.T)
+    del x
+    a, c = _padded(P, h), _padded(P, torch.zeros_like(h))
+    c += 7.0
+    torch.cuda.synchronize()
+    P.gemm_counters(reset=True)
+    P.symmetric_product_device(a, a, c, n)
+    ld = P.padded_ld(n)
+    assert ld == 8064 and P.gemm_counters(reset=True)[2] == 63 * 64 / 2 * 2.0 * 128 * 128 * 8032
+    h2 = h @ h
+    habs = h.abs()
+    assert bool(((c[:n, :n] - h2).abs() <= 2 * n * EPS * (habs @ habs)).all())
+    assert torch.equal(c, c.T) and not bool(c[n:].any())
+    lo, hi, pp = -3.0, 3.0, [1, 0, 1]
+    P.sp2_seq_device(a, c, n, pp, lo, hi)
+    xs = [-h / (hi - lo)]
+    xs[0].diagonal().add_(hi / (hi - lo))
+    for s in pp:
+        xs.append(xs[-1] @ xs[-1] if s else 2 * xs[-1] - xs[-1] @ xs[-1])
+    # x <- x^2 or 2 x - x^2 keeps [0, 1]: a step adds at most n eps to an entry
+    # and at most doubles what the steps before left
+    assert float((c[:n, :n] - 2 * xs[-1]).abs().max()) <= 2 * 2 ** len(pp) * n * EPS
+    assert torch.equal(c, c.T)
+    gout = _random(n, n + 1)
+    gout = 0.5 * (gout + gout.T)
+    P.sp2_adjoint_device(a, _padded(P, gout), c, n, pp, lo, hi, 2)
+    g = 2 * gout
+    for k in (2, 1, 0):
+        s = xs[k] @ g
+        s = s + s.T
+        g = s if pp[k] else 2 * g - s
+    ref = -g / (hi - lo)
+    assert float((c[:n, :n] - ref).norm()) <= 2 * 3 * 2 * n * EPS * float(ref.norm() + 8 * gout.norm())
+    assert torch.equal(c, c.T)
+
+
+def test_density_and_response(P, n=8010):
+    """Both matrices of the response's steps, for H = Q diag(e) Q with the
+    reflection Q = I - 2 v v^T, whose density and response are known."""
+    print(f"[staged response] n={n}", flush=True)
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(n)
+    v = torch.randn(n, dtype=torch.float64, device="cuda", generator=g)
+    v /= v.norm()
+    u = torch.rand(n, dtype=torch.float64, device="cuda", generator=g)
+    occ = torch.arange(n, device="cuda") < n // 2
+    e = torch.where(occ, -3 + 2 * u, 1 + 2 * u)
+
+    def conjugate(m):
+        m = m - 2 * torch.outer(v, v @ m)
+        return m - 2 * torch.outer(m @ v, v)
+
+    h = conjugate(torch.diag(e))
+    h = 0.5 * (h + h.T)
+    h1 = _random(n, 5, 1.0 / n ** 0.5)
+    h1 = 0.5 * (h1 + h1.T)
+    rho, rsp = P.compute_response_sp2(h.cpu().numpy(), h1.cpu().numpy(), (n // 2) / n, 1, 100, "Abs",
+                                      1e-10)
+    f = occ.double()
+    df, de = f[:, None] - f[None, :], e[:, None] - e[None, :]
+    quotient = torch.where(df != 0, df / torch.where(de != 0, de, torch.ones_like(de)),
+                           torch.zeros_like(de))
+    ref = 2 * conjugate(conjugate(h1) * quotient)
+    rho, rsp = torch.from_numpy(rho).cuda(), torch.from_numpy(rsp).cuda()
+    assert float((rho - 2 * conjugate(torch.diag(f))).norm()) < 4e-9
+    assert float((rsp - ref).norm()) < 1e-7 * float(ref.norm())
+    assert torch.equal(rsp, rsp.T) and torch.equal(rho, rho.T)
